@@ -167,50 +167,84 @@ __global__ void classify_kernel(LNode* __restrict__ nodes, int32_t nn, Params P)
 
 // One wave per node with at most 64 references: every reference's minimum
 // and the float just past its maximum are candidate planes (host:
-// find_split, exact branch).
+// find_split, exact branch).  The node's 6 n candidates (axis, reference,
+// side) are dealt to the lanes; each lane counts the references below and
+// above its own plane by walking the n reference intervals of its axis in LDS
+// (the lanes of an axis read one address, a broadcast) and costs the plane
+// once, and the wave then reduces to the winner.  Bound by vector-instruction
+// issue.  The form before took the candidates one at a time with every lane
+// costing the same plane: 6 n rounds of two ballots, a cross-lane read and
+// the cost, where this one takes 6 n / 64 rounds of n short steps.
+struct SplitLds {
+  float2 iv[3][kExactMax + 1];  // per axis: {lo, hi} of each reference; the pad spreads the axes over the banks
+};
+
 __global__ void __launch_bounds__(256) exact_split_kernel(LNode* __restrict__ nodes, int32_t nn,
                                                           const Ref* __restrict__ refs, Params P) {
+  __shared__ SplitLds lds[4];
   const int lane = threadIdx.x & 63;
   const int w = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   if (w >= nn) return;
   LNode& nd = nodes[w];
   if (nd.mode != kModeExact) return;
+  SplitLds& S = lds[threadIdx.x >> 6];
   const int n = nd.n;
-  const bool have = lane < n;
-  Ref r{};
-  if (have) r = refs[nd.rbegin + lane];
-  const float sa = area_of(nd.hi[0] - nd.lo[0], nd.hi[1] - nd.lo[1], nd.hi[2] - nd.lo[2]);
+  if (lane < n) {
+    const Ref r = refs[nd.rbegin + lane];
+    for (int a = 0; a < 3; ++a) S.iv[a][lane] = make_float2(r.lo[a], r.hi[a]);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float nlo[3] = {nd.lo[0], nd.lo[1], nd.lo[2]}, nhi[3] = {nd.hi[0], nd.hi[1], nd.hi[2]};
+  const float sa = area_of(nhi[0] - nlo[0], nhi[1] - nlo[1], nhi[2] - nlo[2]);
   const float inv_sa = sa > 0.0f ? 1.0f / sa : 0.0f;
   float bc = kInf, bp = 0.0f;
-  int ba = -1;
-  int64_t bnl = 0, bnr = 0;
-  for (int a = 0; a < 3; ++a) {
-    const float lo = get3(nd.lo, a), hi = get3(nd.hi, a);
-    const float ext = hi - lo;
-    if (!(ext > 0.0f)) continue;
-    const float rl = get3(r.lo, a), rh = get3(r.hi, a);
-    const float c0 = rl, c1 = next_up(rh);
-    for (int j = 0; j < 2 * n; ++j) {
-      const float mine = (j & 1) ? c1 : c0;
-      const float pos = __shfl(mine, j >> 1);
-      if (!(pos > lo && pos < hi)) continue;
-      const int64_t nl = __popcll(__ballot(have && rl < pos));
-      const int64_t nr = __popcll(__ballot(have && rh >= pos));
-      const float c = split_cost(P, nd.lo, nd.hi, a, pos, nl, nr, inv_sa);
-      if (better(c, a, pos, bc, ba, bp)) {
-        bc = c;
-        ba = a;
-        bp = pos;
-        bnl = nl;
-        bnr = nr;
-      }
+  int ba = 3, bq = 0, bnl = 0, bnr = 0;  // axis 3: none
+  for (int e = lane; e < 6 * n; e += 64) {
+    const int a = e >= 4 * n ? 2 : (e >= 2 * n ? 1 : 0);
+    const int q = e - 2 * n * a;
+    const float2 own = S.iv[a][q >> 1];
+    const float pos = (q & 1) ? next_up(own.y) : own.x;
+    const float lo = get3(nlo, a), hi = get3(nhi, a);
+    if (!(hi - lo > 0.0f) || !(pos > lo && pos < hi)) continue;
+    int nl = 0, nr = 0;
+    for (int k = 0; k < n; ++k) {
+      const float2 r = S.iv[a][k];
+      nl += r.x < pos ? 1 : 0;
+      nr += r.y >= pos ? 1 : 0;
+    }
+    const float c = split_cost(P, nlo, nhi, a, pos, nl, nr, inv_sa);
+    if (better(c, a, pos, bc, ba, bp)) {
+      bc = c;
+      ba = a;
+      bp = pos;
+      bq = q;
+      bnl = nl;
+      bnr = nr;
+    }
+  }
+  // The winner over the lanes.  Planes at +0 and -0 compare equal (and have
+  // equal counts): the lower candidate index q of the axis is taken, as when
+  // the candidates are scanned in order.
+  for (int off = 32; off >= 1; off >>= 1) {
+    const float oc = __shfl_xor(bc, off), op = __shfl_xor(bp, off);
+    const int oa = __shfl_xor(ba, off), oq = __shfl_xor(bq, off), ol = __shfl_xor(bnl, off),
+              orr = __shfl_xor(bnr, off);
+    if (better(oc, oa, op, bc, ba, bp) || (oc < kInf && oc == bc && oa == ba && op == bp && oq < bq)) {
+      bc = oc;
+      ba = oa;
+      bp = op;
+      bq = oq;
+      bnl = ol;
+      bnr = orr;
     }
   }
   if (lane == 0) {
-    nd.axis = ba;
+    nd.axis = ba == 3 ? -1 : ba;
     nd.pos = bp;
-    nd.nl = (int32_t)bnl;
-    nd.nr = (int32_t)bnr;
+    nd.nl = bnl;
+    nd.nr = bnr;
   }
 }
 
@@ -334,88 +368,76 @@ __device__ __forceinline__ bool will_try(const LNode& nd) {
   return nd.mode != kModeLeaf && nd.axis >= 0 && !(nd.nl == nd.n && nd.nr == nd.n);
 }
 
-// Adds, per node, the below/above counts vl, vr (0 or 1) of the wave's
-// lanes; key is the lane's node (-1 for none).  The lanes of a wave usually
-// share one node (a node's references are contiguous), so one atomic per
-// wave replaces up to 64 on the same address.
-__device__ __forceinline__ void wave_count(LNode* __restrict__ nodes, int key, int vl, int vr) {
-  const int lane = threadIdx.x & 63;
-  const unsigned long long act = __ballot(1);
-  const int leader = __ffsll((unsigned long long)act) - 1;
-  const int lk = __shfl(key, leader);
-  const bool same = key == lk;
-  const unsigned long long ml = __ballot(same && vl), mr = __ballot(same && vr);
-  if (lane == leader && lk >= 0) {
-    if (ml) atomicAdd(&nodes[lk].cl, __popcll(ml));
-    if (mr) atomicAdd(&nodes[lk].cr, __popcll(mr));
-  }
-  if (!same && key >= 0) {
-    if (vl) atomicAdd(&nodes[key].cl, 1);
-    if (vr) atomicAdd(&nodes[key].cr, 1);
-  }
-}
+// Which side(s) each reference goes to (host: build, partition loop): the
+// flags word holds the below side in bit 0 and the above side in bit 32, so
+// that one scan ranks both.  References that straddle the plane while
+// clipping is on are listed for part_clip_kernel, which clips them with full
+// waves.  A block covers kFlagChunk references and takes its part of the list
+// with one atomic: with one per wave (and two more per wave on the node's
+// counts, which now come from the scan) the top levels, where every wave adds
+// to one address, took 289 us per launch on 2^20 triangles.
+constexpr int kFlagChunk = 1024;
+constexpr uint64_t kBelow = 1ull, kAbove = 1ull << 32;
 
-// Which side(s) each reference goes to (host: build, partition loop).
-// References that straddle the plane while clipping is on are listed for
-// part_clip_kernel, which clips them with full waves.
 __global__ void __launch_bounds__(256) part_flags_kernel(const Ref* __restrict__ refs,
                                                          const int32_t* __restrict__ ref_node, int64_t nref,
-                                                         LNode* __restrict__ nodes, Params P,
-                                                         int32_t* __restrict__ fl, int32_t* __restrict__ fr,
-                                                         Ref* __restrict__ box_l, Ref* __restrict__ box_r,
-                                                         int32_t* __restrict__ strad, int32_t* __restrict__ n_strad) {
+                                                         const LNode* __restrict__ nodes, Params P,
+                                                         uint64_t* __restrict__ flags, int32_t* __restrict__ strad,
+                                                         int32_t* __restrict__ n_strad) {
+  __shared__ int32_t list[kFlagChunk];
+  __shared__ int32_t n_list, base;
+  if (threadIdx.x == 0) n_list = 0;
+  __syncthreads();
   const int lane = threadIdx.x & 63;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool in = i < nref;
-  const int key = in ? ref_node[i] : -1;
-  int l = 0, rr = 0;
-  bool st = false;
-  if (in && will_try(nodes[key])) {
-    const LNode& nd = nodes[key];
-    const Ref r = refs[i];
-    const bool to_l = get3(r.lo, nd.axis) < nd.pos, to_r = get3(r.hi, nd.axis) >= nd.pos;
-    if (to_l && to_r && P.clip) {
-      st = true;
-    } else {
-      l = to_l ? 1 : 0;
-      rr = to_r ? 1 : 0;
-      box_l[i] = r;
-      box_r[i] = r;
+  const int64_t c0 = (int64_t)blockIdx.x * kFlagChunk;
+  for (int k = 0; k < kFlagChunk; k += 256) {
+    const int64_t i = c0 + k + threadIdx.x;
+    bool st = false;
+    if (i < nref) {
+      uint64_t f = 0;
+      const LNode& nd = nodes[ref_node[i]];
+      if (will_try(nd)) {
+        const bool to_l = refs[i].lo[nd.axis] < nd.pos, to_r = refs[i].hi[nd.axis] >= nd.pos;
+        st = to_l && to_r && P.clip;
+        if (!st) f = (to_l ? kBelow : 0) | (to_r ? kAbove : 0);
+      }
+      flags[i] = f;
+    }
+    const unsigned long long sm = __ballot(st);
+    if (sm) {
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&n_list, __popcll(sm));
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (st) list[at + __popcll(sm & ((1ull << lane) - 1ull))] = (int32_t)i;
     }
   }
-  if (in) {
-    fl[i] = l;
-    fr[i] = rr;
-  }
-  const unsigned long long sm = __ballot(st);
-  if (sm) {
-    const int leader = __ffsll(sm) - 1;
-    int base = 0;
-    if (lane == leader) base = atomicAdd(n_strad, __popcll(sm));
-    base = __shfl(base, leader);
-    if (st) strad[base + __popcll(sm & ((1ull << lane) - 1ull))] = (int32_t)i;
-  }
-  wave_count(nodes, key, l, rr);
+  __syncthreads();
+  const int m = n_list;
+  if (threadIdx.x == 0 && m > 0) base = atomicAdd(n_strad, m);
+  __syncthreads();
+  for (int k = threadIdx.x; k < m; k += 256) strad[base + k] = list[k];
 }
 
 // Thread 2s + side clips straddler s against the below (side 0) or above
-// (side 1) child box (host: Builder::clip_box on both children).
+// (side 1) child box (host: Builder::clip_box on both children).  The two
+// threads of a straddler are neighbouring lanes; the even one writes its
+// flags.
 __global__ void __launch_bounds__(256) part_clip_kernel(const float* __restrict__ tv, const Ref* __restrict__ refs,
-                                                        const int32_t* __restrict__ ref_node, LNode* __restrict__ nodes,
+                                                        const int32_t* __restrict__ ref_node,
+                                                        const LNode* __restrict__ nodes,
                                                         const int32_t* __restrict__ strad,
-                                                        const int32_t* __restrict__ n_strad, int32_t* __restrict__ fl,
-                                                        int32_t* __restrict__ fr, Ref* __restrict__ box_l,
+                                                        const int32_t* __restrict__ n_strad,
+                                                        uint64_t* __restrict__ flags, Ref* __restrict__ box_l,
                                                         Ref* __restrict__ box_r) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t ns = *n_strad;
   if ((t - (threadIdx.x & 63)) >= 2 * ns) return;  // whole waves past the list leave together
-  const bool in = t < 2 * ns;
-  int key = -1, ok = 0;
+  int ok = 0;
   const int side = (int)(t & 1);
-  if (in) {
-    const int64_t i = strad[t >> 1];
-    key = ref_node[i];
-    const LNode& nd = nodes[key];
+  int64_t i = 0;
+  if (t < 2 * ns) {
+    i = strad[t >> 1];
+    const LNode& nd = nodes[ref_node[i]];
     float lo[3] = {nd.lo[0], nd.lo[1], nd.lo[2]}, hi[3] = {nd.hi[0], nd.hi[1], nd.hi[2]};
     if (side == 0) {
       if (nd.axis == 0) hi[0] = nd.pos;
@@ -428,40 +450,55 @@ __global__ void __launch_bounds__(256) part_clip_kernel(const float* __restrict_
     }
     Ref c;
     ok = clip_box(tv, refs[i].prim, lo, hi, c) ? 1 : 0;
-    if (side == 0) {
-      fl[i] = ok;
-      if (ok) box_l[i] = c;
-    } else {
-      fr[i] = ok;
-      if (ok) box_r[i] = c;
-    }
+    if (ok) (side == 0 ? box_l : box_r)[i] = c;
   }
-  wave_count(nodes, key, side == 0 ? ok : 0, side == 1 ? ok : 0);
-}
-
-// Totals of the three exclusive scans over a level's nodes.
-__global__ void totals_kernel(const int32_t* kids, const int32_t* kx, const int32_t* crefs, const int32_t* cx,
-                              const int32_t* leafn, const int32_t* lx, int64_t nn, int64_t* out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    out[0] = (int64_t)kx[nn - 1] + kids[nn - 1];
-    out[1] = (int64_t)cx[nn - 1] + crefs[nn - 1];
-    out[2] = (int64_t)lx[nn - 1] + leafn[nn - 1];
+  const unsigned long long m = __ballot(ok);
+  if (t < 2 * ns && side == 0) {
+    const unsigned long long two = m >> (threadIdx.x & 63);
+    flags[i] = ((two & 1ull) ? kBelow : 0) | ((two & 2ull) ? kAbove : 0);
   }
 }
 
-__global__ void decide_kernel(LNode* __restrict__ nodes, int32_t nn, int32_t* __restrict__ kids,
-                              int32_t* __restrict__ crefs, int32_t* __restrict__ leafn) {
+// What a node adds to the next level and to the leaf pool, scanned together:
+// next-level nodes, next-level references, leaf-pool references.
+struct Adds {
+  int32_t kids, refs, leaf, pad;
+};
+struct AddsSum {
+  __host__ __device__ Adds operator()(const Adds& a, const Adds& b) const {
+    return Adds{a.kids + b.kids, a.refs + b.refs, a.leaf + b.leaf, 0};
+  }
+};
+
+// The split decision of every node, its below and above counts taken from
+// the scan of its references' flags (flags_x exclusive; a node's references
+// are contiguous).
+__global__ void decide_kernel(LNode* __restrict__ nodes, int32_t nn, const uint64_t* __restrict__ flags,
+                              const uint64_t* __restrict__ flags_x, Adds* __restrict__ adds) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nn) return;
   LNode& nd = nodes[i];
+  if (nd.n > 0) {
+    const int64_t last = nd.rbegin + nd.n - 1;
+    const uint64_t c = flags_x[last] + flags[last] - flags_x[nd.rbegin];
+    nd.cl = (int32_t)(uint32_t)c;
+    nd.cr = (int32_t)(c >> 32);
+  }
   nd.split = (will_try(nd) && !(nd.cl == nd.n && nd.cr == nd.n)) ? 1 : 0;
-  kids[i] = nd.split ? 2 : 0;
-  crefs[i] = nd.split ? nd.cl + nd.cr : 0;
-  leafn[i] = nd.split ? 0 : nd.n;
+  adds[i] = Adds{nd.split ? 2 : 0, nd.split ? nd.cl + nd.cr : 0, nd.split ? 0 : nd.n, 0};
 }
 
-__global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const int32_t* __restrict__ kids_x,
-                            const int32_t* __restrict__ crefs_x, const int32_t* __restrict__ leafn_x,
+// Totals of the scan over a level's nodes.
+__global__ void totals_kernel(const Adds* adds, const Adds* adds_x, int64_t nn, int64_t* out) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    const Adds a = adds[nn - 1], x = adds_x[nn - 1];
+    out[0] = (int64_t)x.kids + a.kids;
+    out[1] = (int64_t)x.refs + a.refs;
+    out[2] = (int64_t)x.leaf + a.leaf;
+  }
+}
+
+__global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const Adds* __restrict__ adds_x,
                             LNode* __restrict__ next, int32_t next_gid, int64_t pool_base, GNode* __restrict__ gn) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nn) return;
@@ -473,9 +510,9 @@ __global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const int32_t
   }
   g.depth = nd.depth;
   if (nd.split) {
-    const int c = kids_x[i];
+    const int c = adds_x[i].kids;
     nd.child = c;
-    nd.crbegin = crefs_x[i];
+    nd.crbegin = adds_x[i].refs;
     LNode b{}, u{};
     for (int a = 0; a < 3; ++a) {
       b.lo[a] = u.lo[a] = nd.lo[a];
@@ -500,7 +537,7 @@ __global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const int32_t
     g.pool_n = 0;
     g.pool = 0;
   } else {
-    nd.pool = pool_base + leafn_x[i];
+    nd.pool = pool_base + adds_x[i].leaf;
     g.axis = -1;
     g.split = 0.0f;
     g.child0 = g.child1 = -1;
@@ -510,24 +547,29 @@ __global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const int32_t
   gn[nd.gid] = g;
 }
 
+// Each reference to its place in the children (the clipped boxes are those
+// of the straddlers only; every other reference keeps its box) or, in a leaf,
+// to the pool.
 __global__ void scatter_kernel(const Ref* __restrict__ refs, const int32_t* __restrict__ ref_node, int64_t nref,
-                               const LNode* __restrict__ nodes, const int32_t* __restrict__ fl,
-                               const int32_t* __restrict__ fr, const int32_t* __restrict__ fl_x,
-                               const int32_t* __restrict__ fr_x, const Ref* __restrict__ box_l,
-                               const Ref* __restrict__ box_r, Ref* __restrict__ next_refs,
+                               const LNode* __restrict__ nodes, const uint64_t* __restrict__ flags,
+                               const uint64_t* __restrict__ flags_x, const Ref* __restrict__ box_l,
+                               const Ref* __restrict__ box_r, Params P, Ref* __restrict__ next_refs,
                                int32_t* __restrict__ next_node, int32_t* __restrict__ pool) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nref) return;
   const LNode& nd = nodes[ref_node[i]];
   if (nd.split) {
-    if (fl[i]) {
-      const int64_t k = nd.crbegin + (fl_x[i] - fl_x[nd.rbegin]);
-      next_refs[k] = box_l[i];
+    const uint64_t f = flags[i], rank = flags_x[i] - flags_x[nd.rbegin];
+    const Ref r = refs[i];
+    const bool clipped = P.clip && get3(r.lo, nd.axis) < nd.pos && get3(r.hi, nd.axis) >= nd.pos;
+    if (f & kBelow) {
+      const int64_t k = nd.crbegin + (int64_t)(uint32_t)rank;
+      next_refs[k] = clipped ? box_l[i] : r;
       next_node[k] = nd.child;
     }
-    if (fr[i]) {
-      const int64_t k = nd.crbegin + nd.cl + (fr_x[i] - fr_x[nd.rbegin]);
-      next_refs[k] = box_r[i];
+    if (f & kAbove) {
+      const int64_t k = nd.crbegin + nd.cl + (int64_t)(rank >> 32);
+      next_refs[k] = clipped ? box_r[i] : r;
       next_node[k] = nd.child + 1;
     }
   } else {
@@ -722,13 +764,13 @@ struct Arr {
 // Exclusive prefix sum with a reusable temporary buffer.
 struct Scanner {
   Arr<char> tmp;
-  template <typename T>
-  hipError_t run(Bufs& B, const T* in, T* out, int64_t n, hipStream_t s) {
+  template <typename T, typename Op = hipcub::Sum>
+  hipError_t run(Bufs& B, const T* in, T* out, int64_t n, hipStream_t s, Op op = Op{}, T zero = T{}) {
     if (n <= 0) return hipSuccess;
     size_t bytes = 0;
-    hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, in, out, (int)n, s);
+    hipError_t e = hipcub::DeviceScan::ExclusiveScan(nullptr, bytes, in, out, op, zero, (int)n, s);
     if (e == hipSuccess) e = tmp.ensure(B, (int64_t)bytes, s);
-    if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(tmp.p, bytes, in, out, (int)n, s);
+    if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveScan(tmp.p, bytes, in, out, op, zero, (int)n, s);
     return e;
   }
 };
@@ -766,9 +808,11 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
 
   // Level arrays: current and next references / nodes swap every level.
   Arr<Ref> refs, nrefs, box_l, box_r;
-  Arr<int32_t> ref_node, nnode, fl, fr, flx, frx, strad;
+  Arr<int32_t> ref_node, nnode, strad;
+  Arr<uint64_t> flags, flags_x;
   Arr<LNode> lv, next;
-  Arr<int32_t> kids, crefs, leafn, kx, cx, lx, hist;
+  Arr<int32_t> hist;
+  Arr<Adds> adds, adds_x;
   Arr<GNode> gn;
   Arr<int32_t> pool;
   Scanner scan;
@@ -812,27 +856,27 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
                        P);
     KDB_TRY(hipGetLastError());
 
-    for (Arr<int32_t>* a : {&fl, &fr, &flx, &frx, &strad}) KDB_TRY(a->ensure(B, nref, s));
+    KDB_TRY(strad.ensure(B, nref, s));
+    KDB_TRY(flags.ensure(B, nref, s));
+    KDB_TRY(flags_x.ensure(B, nref, s));
     KDB_TRY(box_l.ensure(B, nref, s));
     KDB_TRY(box_r.ensure(B, nref, s));
     KDB_TRY(hipMemsetAsync(n_strad, 0, sizeof(int32_t), s));
-    hipLaunchKernelGGL(part_flags_kernel, dim3(blocks(nref, 256)), dim3(256), 0, s, refs.p, ref_node.p, nref, lv.p, P,
-                       fl.p, fr.p, box_l.p, box_r.p, strad.p, n_strad);
+    hipLaunchKernelGGL(part_flags_kernel, dim3(blocks(nref, kFlagChunk)), dim3(256), 0, s, refs.p, ref_node.p, nref,
+                       lv.p, P, flags.p, strad.p, n_strad);
     if (P.clip)
       hipLaunchKernelGGL(part_clip_kernel, dim3(blocks(2 * nref, 256)), dim3(256), 0, s, tv, refs.p, ref_node.p,
-                         lv.p, strad.p, n_strad, fl.p, fr.p, box_l.p, box_r.p);
+                         lv.p, strad.p, n_strad, flags.p, box_l.p, box_r.p);
     KDB_TRY(hipGetLastError());
-    KDB_TRY(scan.run(B, fl.p, flx.p, nref, s));
-    KDB_TRY(scan.run(B, fr.p, frx.p, nref, s));
+    KDB_TRY(scan.run(B, flags.p, flags_x.p, nref, s));
 
-    for (Arr<int32_t>* a : {&kids, &crefs, &leafn, &kx, &cx, &lx}) KDB_TRY(a->ensure(B, nn, s));
-    hipLaunchKernelGGL(decide_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, kids.p, crefs.p,
-                       leafn.p);
+    KDB_TRY(adds.ensure(B, nn, s));
+    KDB_TRY(adds_x.ensure(B, nn, s));
+    hipLaunchKernelGGL(decide_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, flags.p, flags_x.p,
+                       adds.p);
     KDB_TRY(hipGetLastError());
-    KDB_TRY(scan.run(B, kids.p, kx.p, nn, s));
-    KDB_TRY(scan.run(B, crefs.p, cx.p, nn, s));
-    KDB_TRY(scan.run(B, leafn.p, lx.p, nn, s));
-    hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, kids.p, kx.p, crefs.p, cx.p, leafn.p, lx.p, nn, tot);
+    KDB_TRY(scan.run(B, adds.p, adds_x.p, nn, s, AddsSum{}, Adds{0, 0, 0, 0}));
+    hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, adds.p, adds_x.p, nn, tot);
     int64_t t3[3] = {0, 0, 0};
     KDB_TRY(hipMemcpyAsync(t3, tot, sizeof(t3), hipMemcpyDeviceToHost, s));
     KDB_TRY(hipStreamSynchronize(s));
@@ -845,10 +889,10 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
     KDB_TRY(nrefs.ensure(B, r_next, s));
     KDB_TRY(nnode.ensure(B, r_next, s));
     const int32_t next_gid = gbase + (int32_t)nn;
-    hipLaunchKernelGGL(emit_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, kx.p, cx.p, lx.p,
-                       next.p, next_gid, pused, gn.p);
+    hipLaunchKernelGGL(emit_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, adds_x.p, next.p, next_gid,
+                       pused, gn.p);
     hipLaunchKernelGGL(scatter_kernel, dim3(blocks(nref, 256)), dim3(256), 0, s, refs.p, ref_node.p, nref, lv.p,
-                       fl.p, fr.p, flx.p, frx.p, box_l.p, box_r.p, nrefs.p, nnode.p, pool.p);
+                       flags.p, flags_x.p, box_l.p, box_r.p, P, nrefs.p, nnode.p, pool.p);
     KDB_TRY(hipGetLastError());
     std::swap(lv, next);
     std::swap(refs, nrefs);
