@@ -16,8 +16,10 @@ struct Ref {
   float lo[3], hi[3];
 };
 
-// Node modes of a level.
-enum : int32_t { kModeLeaf = 0, kModeExact = 1, kModeBinned = 2 };
+// Node modes of a level: a leaf by size or depth, every candidate plane
+// (at most kExactMax references), binned by one wave (at most kWaveBinMax),
+// binned by many blocks.
+enum : int32_t { kModeLeaf = 0, kModeExact = 1, kModeBinned = 2, kModeBig = 3 };
 
 // An active node of the current level.
 struct LNode {
@@ -55,6 +57,17 @@ struct Params {
 
 constexpr int kExactMax = 64;  // nodes with at most this many references test every candidate plane
 constexpr int kMaxBins = 64;
+// References per block of the many-block binning, and the most that one wave
+// bins by itself.  Equal, so that a chunk's references belong to at most two
+// big nodes (its first and its last) and each chunk index is at most one big
+// node's rbegin / kBinChunk, which numbers the histograms.
+constexpr int kBinChunk = 1024;
+constexpr int kWaveBinMax = kBinChunk;
+
+RE_HD int32_t mode_of(int32_t n, int32_t depth, const Params& P) {
+  if (n <= P.max_leaf || depth >= P.max_depth) return kModeLeaf;
+  return n <= kExactMax ? kModeExact : (n <= kWaveBinMax ? kModeBinned : kModeBig);
+}
 
 }  // namespace kdb
 }  // namespace re

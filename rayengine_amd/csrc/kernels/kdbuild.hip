@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../capi_util.hpp"
+#include "../device_paths.hpp"
 #include "../kdbuild.hpp"
 
 namespace re {
@@ -152,53 +153,124 @@ __global__ void init_refs_kernel(const float* __restrict__ tv, int64_t n, Ref* _
   ref_node[i] = 0;
 }
 
-__global__ void classify_kernel(LNode* __restrict__ nodes, int32_t nn, Params P) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nn) return;
-  LNode& nd = nodes[i];
-  nd.mode = (nd.n <= P.max_leaf || nd.depth >= P.max_depth) ? kModeLeaf
-                                                             : (nd.n <= kExactMax ? kModeExact : kModeBinned);
-  nd.axis = -1;
-  nd.pos = 0.0f;
-  nd.nl = nd.nr = 0;
-  nd.cl = nd.cr = 0;
-  nd.split = 0;
+__device__ __forceinline__ int bin_of(float v, float lo, float hi, float scale, int nb) {
+  const float pc = smin(smax(v, lo), hi);
+  return min(nb - 1, max(0, (int)((pc - lo) * scale)));
 }
 
-// One wave per node with at most 64 references: every reference's minimum
-// and the float just past its maximum are candidate planes (host:
+// Adds a reference to its node's bin counts: per axis a, the bin of its
+// clamped minimum (row 2 a) and of its clamped maximum (row 2 a + 1).
+__device__ __forceinline__ void bin_ref(const Ref& r, const LNode& nd, int nb, int32_t* h) {
+  for (int a = 0; a < 3; ++a) {
+    const float lo = get3(nd.lo, a), hi = get3(nd.hi, a), ext = hi - lo;
+    if (!(ext > 0.0f)) continue;
+    const float scale = (float)nb / ext;
+    atomicAdd(&h[(2 * a) * nb + bin_of(get3(r.lo, a), lo, hi, scale, nb)], 1);
+    atomicAdd(&h[(2 * a + 1) * nb + bin_of(get3(r.hi, a), lo, hi, scale, nb)], 1);
+  }
+}
+
+// Bin counts of the nodes too large for one wave (host: find_split, binned
+// branch).  A chunk of kBinChunk references belongs to at most two of them,
+// its first reference's node and its last's: both are counted in LDS and
+// added to the node's histogram once per chunk.  (Counting the references of
+// mixed chunks, most of them once nodes are a few thousand references large,
+// with global atomics took 26 us per level on a 2^18-triangle soup; 10 us
+// now, in the two thirds of the levels that have such nodes.)
+__global__ void __launch_bounds__(256) bin_count_kernel(const Ref* __restrict__ refs,
+                                                        const int32_t* __restrict__ ref_node, int64_t nref,
+                                                        const LNode* __restrict__ nodes, int32_t* __restrict__ hist,
+                                                        Params P) {
+  __shared__ int32_t sh[2][6 * kMaxBins];
+  const int nb = max(4, P.n_bins);
+  const int64_t c0 = (int64_t)blockIdx.x * kBinChunk;
+  const int64_t c1 = min(c0 + (int64_t)kBinChunk, nref);
+  const int32_t first = ref_node[c0], last = ref_node[c1 - 1];
+  const bool big0 = nodes[first].mode == kModeBig, big1 = last != first && nodes[last].mode == kModeBig;
+  if (!big0 && !big1) return;
+  for (int k = threadIdx.x; k < 6 * nb; k += blockDim.x) sh[0][k] = sh[1][k] = 0;
+  __syncthreads();
+  for (int64_t i = c0 + threadIdx.x; i < c1; i += blockDim.x) {
+    const int32_t node = ref_node[i];
+    if (node == first ? big0 : (node == last && big1)) bin_ref(refs[i], nodes[node], nb, sh[node == first ? 0 : 1]);
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < 6 * nb; k += blockDim.x) {
+    if (sh[0][k]) atomicAdd(&hist[nodes[first].rbegin / kBinChunk * (6 * nb) + k], sh[0][k]);
+    if (sh[1][k]) atomicAdd(&hist[nodes[last].rbegin / kBinChunk * (6 * nb) + k], sh[1][k]);
+  }
+}
+
+struct Plane {
+  float cost, pos;
+  int axis, nl, nr;
+};
+
+// The best bin plane of a node from its bin counts h (LDS): lane k costs the
+// plane between bins k - 1 and k.
+__device__ __forceinline__ Plane binned_plane(const float* nlo, const float* nhi, int n, const int32_t* h, int nb,
+                                              float inv_sa, const Params& P) {
+  const int k = threadIdx.x & 63;
+  Plane best{kInf, 0.0f, -1, 0, 0};
+  for (int a = 0; a < 3; ++a) {
+    const float lo = nlo[a], hi = nhi[a];
+    const float ext = hi - lo;
+    if (!(ext > 0.0f)) continue;
+    // references with their minimum below the plane, and all but those with
+    // their maximum below it
+    const uint32_t cmin = k < nb ? (uint32_t)h[(2 * a) * nb + k] : 0u;
+    const uint32_t cmax = k < nb ? (uint32_t)h[(2 * a + 1) * nb + k] : 0u;
+    const int nl = (int)(wave_incl_scan(cmin) - cmin), nr = n - (int)(wave_incl_scan(cmax) - cmax);
+    float c = kInf, pos = 0.0f;
+    if (k >= 1 && k < nb) {
+      pos = lo + ext * (float)k / (float)nb;
+      if (pos > lo && pos < hi) c = split_cost(P, nlo, nhi, a, pos, nl, nr, inv_sa);
+      if (!(c < kInf)) c = kInf;  // NaN never wins; keep the reduction's order total
+    }
+    // lowest cost, then lowest k, across the wave
+    float wc = c;
+    int wk = (c < kInf) ? k : 1 << 20;
+    for (int off = 32; off >= 1; off >>= 1) {
+      const float oc = __shfl_xor(wc, off);
+      const int ok = __shfl_xor(wk, off);
+      if (oc < wc || (oc == wc && ok < wk)) {
+        wc = oc;
+        wk = ok;
+      }
+    }
+    if (wk < (1 << 20)) {
+      const float wpos = __shfl(pos, wk);
+      const int wnl = __shfl(nl, wk), wnr = __shfl(nr, wk);
+      if (better(wc, a, wpos, best.cost, best.axis, best.pos)) best = Plane{wc, wpos, a, wnl, wnr};
+    }
+  }
+  return best;
+}
+
+struct ExactLds {
+  float2 iv[3][kExactMax + 1];  // per axis: {lo, hi} of each reference; the pad spreads the axes over the banks
+};
+
+// The best plane of a node with at most 64 references: every reference's
+// minimum and the float just past its maximum are candidate planes (host:
 // find_split, exact branch).  The node's 6 n candidates (axis, reference,
 // side) are dealt to the lanes; each lane counts the references below and
 // above its own plane by walking the n reference intervals of its axis in LDS
 // (the lanes of an axis read one address, a broadcast) and costs the plane
 // once, and the wave then reduces to the winner.  Bound by vector-instruction
 // issue.  The form before took the candidates one at a time with every lane
-// costing the same plane: 6 n rounds of two ballots, a cross-lane read and
-// the cost, where this one takes 6 n / 64 rounds of n short steps.
-struct SplitLds {
-  float2 iv[3][kExactMax + 1];  // per axis: {lo, hi} of each reference; the pad spreads the axes over the banks
-};
-
-__global__ void __launch_bounds__(256) exact_split_kernel(LNode* __restrict__ nodes, int32_t nn,
-                                                          const Ref* __restrict__ refs, Params P) {
-  __shared__ SplitLds lds[4];
+// costing the same plane, 6 n rounds of two ballots, a cross-lane read and
+// the cost: 109 us per level on a 2^18-triangle soup against 14 us.
+__device__ __forceinline__ Plane exact_plane(const float* nlo, const float* nhi, int n, const Ref* __restrict__ refs,
+                                             ExactLds& S, float inv_sa, const Params& P) {
   const int lane = threadIdx.x & 63;
-  const int w = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  if (w >= nn) return;
-  LNode& nd = nodes[w];
-  if (nd.mode != kModeExact) return;
-  SplitLds& S = lds[threadIdx.x >> 6];
-  const int n = nd.n;
   if (lane < n) {
-    const Ref r = refs[nd.rbegin + lane];
+    const Ref r = refs[lane];
     for (int a = 0; a < 3; ++a) S.iv[a][lane] = make_float2(r.lo[a], r.hi[a]);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const float nlo[3] = {nd.lo[0], nd.lo[1], nd.lo[2]}, nhi[3] = {nd.hi[0], nd.hi[1], nd.hi[2]};
-  const float sa = area_of(nhi[0] - nlo[0], nhi[1] - nlo[1], nhi[2] - nlo[2]);
-  const float inv_sa = sa > 0.0f ? 1.0f / sa : 0.0f;
   float bc = kInf, bp = 0.0f;
   int ba = 3, bq = 0, bnl = 0, bnr = 0;  // axis 3: none
   for (int e = lane; e < 6 * n; e += 64) {
@@ -240,127 +312,55 @@ __global__ void __launch_bounds__(256) exact_split_kernel(LNode* __restrict__ no
       bnr = orr;
     }
   }
-  if (lane == 0) {
-    nd.axis = ba == 3 ? -1 : ba;
-    nd.pos = bp;
-    nd.nl = bnl;
-    nd.nr = bnr;
-  }
+  return Plane{bc, bp, ba == 3 ? -1 : ba, bnl, bnr};
 }
 
-// Bin counts of the nodes with more than 64 references: per axis, the bin
-// of every reference's clamped minimum and of its clamped maximum (host:
-// find_split, binned branch).  A block whose chunk of references belongs to
-// one node counts in LDS and adds its histogram once.
-constexpr int kBinChunk = 1024;
+// One wave per node: its split plane, by every candidate or by bins.  A node
+// of 65 to kWaveBinMax references is binned here, in the wave's own LDS
+// histogram, a larger one's counts come from bin_count_kernel.
+union SplitLds {
+  ExactLds exact;
+  int32_t hist[6 * kMaxBins];
+};
 
-__device__ __forceinline__ int bin_of(float v, float lo, float hi, float scale, int nb) {
-  const float pc = smin(smax(v, lo), hi);
-  return min(nb - 1, max(0, (int)((pc - lo) * scale)));
-}
-
-__global__ void __launch_bounds__(256) bin_count_kernel(const Ref* __restrict__ refs,
-                                                        const int32_t* __restrict__ ref_node, int64_t nref,
-                                                        const LNode* __restrict__ nodes, int32_t* __restrict__ hist,
-                                                        Params P) {
-  __shared__ int32_t sh[3 * 2 * kMaxBins];
-  const int nb = max(4, P.n_bins);
-  const int64_t c0 = (int64_t)blockIdx.x * kBinChunk;
-  if (c0 >= nref) return;
-  const int64_t c1 = min(c0 + (int64_t)kBinChunk, nref);
-  const int32_t first = ref_node[c0], last = ref_node[c1 - 1];
-  const bool one = first == last;
-  if (one && nodes[first].mode != kModeBinned) return;
-  if (one)
-    for (int k = threadIdx.x; k < 6 * nb; k += blockDim.x) sh[k] = 0;
-  __syncthreads();
-  for (int64_t i = c0 + threadIdx.x; i < c1; i += blockDim.x) {
-    const int32_t node = one ? first : ref_node[i];
-    const LNode& nd = nodes[node];
-    if (nd.mode != kModeBinned) continue;
-    const Ref r = refs[i];
-    int32_t* g = hist + (int64_t)node * 6 * nb;
-    for (int a = 0; a < 3; ++a) {
-      const float lo = get3(nd.lo, a), hi = get3(nd.hi, a), ext = hi - lo;
-      if (!(ext > 0.0f)) continue;
-      const float scale = (float)nb / ext;
-      const int bl = bin_of(get3(r.lo, a), lo, hi, scale, nb), bh = bin_of(get3(r.hi, a), lo, hi, scale, nb);
-      if (one) {
-        atomicAdd(&sh[(2 * a) * nb + bl], 1);
-        atomicAdd(&sh[(2 * a + 1) * nb + bh], 1);
-      } else {
-        atomicAdd(&g[(2 * a) * nb + bl], 1);
-        atomicAdd(&g[(2 * a + 1) * nb + bh], 1);
-      }
-    }
-  }
-  if (!one) return;
-  __syncthreads();
-  int32_t* g = hist + (int64_t)first * 6 * nb;
-  for (int k = threadIdx.x; k < 6 * nb; k += blockDim.x)
-    if (sh[k]) atomicAdd(&g[k], sh[k]);
-}
-
-// One wave per binned node: lane k costs the plane between bins k-1 and k.
-__global__ void __launch_bounds__(256) binned_split_kernel(LNode* __restrict__ nodes, int32_t nn,
-                                                           const int32_t* __restrict__ hist, Params P) {
+__global__ void __launch_bounds__(256) split_kernel(LNode* __restrict__ nodes, int32_t nn,
+                                                    const Ref* __restrict__ refs, const int32_t* __restrict__ hist,
+                                                    Params P) {
+  __shared__ SplitLds lds[4];
   const int lane = threadIdx.x & 63;
-  const int w = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+  const int w = __builtin_amdgcn_readfirstlane((int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6));
   if (w >= nn) return;
   LNode& nd = nodes[w];
-  if (nd.mode != kModeBinned) return;
-  const int nb = max(4, P.n_bins);
-  const int64_t n = nd.n;
-  const int32_t* g = hist + (int64_t)w * 6 * nb;
-  const float sa = area_of(nd.hi[0] - nd.lo[0], nd.hi[1] - nd.lo[1], nd.hi[2] - nd.lo[2]);
+  const int mode = nd.mode;
+  if (mode == kModeLeaf) return;
+  SplitLds& S = lds[threadIdx.x >> 6];
+  const int n = nd.n;
+  const float nlo[3] = {nd.lo[0], nd.lo[1], nd.lo[2]}, nhi[3] = {nd.hi[0], nd.hi[1], nd.hi[2]};
+  const float sa = area_of(nhi[0] - nlo[0], nhi[1] - nlo[1], nhi[2] - nlo[2]);
   const float inv_sa = sa > 0.0f ? 1.0f / sa : 0.0f;
-  float bc = kInf, bp = 0.0f;
-  int ba = -1;
-  int64_t bnl = 0, bnr = 0;
-  for (int a = 0; a < 3; ++a) {
-    const float lo = get3(nd.lo, a), hi = get3(nd.hi, a);
-    const float ext = hi - lo;
-    if (!(ext > 0.0f)) continue;
-    const int k = lane;
-    float c = kInf, pos = 0.0f;
-    int64_t nl = 0, nr = n;
-    if (k >= 1 && k < nb) {
-      for (int j = 0; j < k; ++j) {
-        nl += g[(2 * a) * nb + j];
-        nr -= g[(2 * a + 1) * nb + j];
-      }
-      pos = lo + ext * (float)k / (float)nb;
-      if (pos > lo && pos < hi) c = split_cost(P, nd.lo, nd.hi, a, pos, nl, nr, inv_sa);
-      if (!(c < kInf)) c = kInf;  // NaN never wins; keep the reduction's order total
+  Plane best;
+  if (mode == kModeExact) {
+    best = exact_plane(nlo, nhi, n, refs + nd.rbegin, S.exact, inv_sa, P);
+  } else {
+    const int nb = max(4, P.n_bins);
+    const int32_t* g = hist + nd.rbegin / kBinChunk * (6 * nb);
+    for (int k = lane; k < 6 * nb; k += 64) S.hist[k] = mode == kModeBig ? g[k] : 0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (mode == kModeBinned) {
+      for (int i = lane; i < n; i += 64) bin_ref(refs[nd.rbegin + i], nd, nb, S.hist);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    // lowest cost, then lowest k, across the wave
-    float wc = c;
-    int wk = (c < kInf) ? k : 1 << 20;
-    for (int off = 32; off >= 1; off >>= 1) {
-      const float oc = __shfl_xor(wc, off);
-      const int ok = __shfl_xor(wk, off);
-      if (oc < wc || (oc == wc && ok < wk)) {
-        wc = oc;
-        wk = ok;
-      }
-    }
-    if (wk < (1 << 20)) {
-      const float wpos = __shfl(pos, wk);
-      const int64_t wnl = __shfl(nl, wk), wnr = __shfl(nr, wk);
-      if (better(wc, a, wpos, bc, ba, bp)) {
-        bc = wc;
-        ba = a;
-        bp = wpos;
-        bnl = wnl;
-        bnr = wnr;
-      }
-    }
+    best = binned_plane(nlo, nhi, n, S.hist, nb, inv_sa, P);
   }
   if (lane == 0) {
-    nd.axis = ba;
-    nd.pos = bp;
-    nd.nl = (int32_t)bnl;
-    nd.nr = (int32_t)bnr;
+    nd.axis = best.axis;
+    nd.pos = best.pos;
+    nd.nl = best.nl;
+    nd.nr = best.nr;
   }
 }
 
@@ -460,13 +460,18 @@ __global__ void __launch_bounds__(256) part_clip_kernel(const float* __restrict_
 }
 
 // What a node adds to the next level and to the leaf pool, scanned together:
-// next-level nodes, next-level references, leaf-pool references.
+// next-level nodes, next-level references, leaf-pool references; and, in
+// `last`, the largest leaf in the low 31 bits, with bit 31 set when a
+// next-level node is to be binned by bin_count_kernel (their maximum and or).
 struct Adds {
-  int32_t kids, refs, leaf, pad;
+  int32_t kids, refs, leaf;
+  uint32_t last;
 };
+constexpr uint32_t kBigBit = 0x80000000u;
 struct AddsSum {
   __host__ __device__ Adds operator()(const Adds& a, const Adds& b) const {
-    return Adds{a.kids + b.kids, a.refs + b.refs, a.leaf + b.leaf, 0};
+    return Adds{a.kids + b.kids, a.refs + b.refs, a.leaf + b.leaf,
+                ((a.last | b.last) & kBigBit) | max(a.last & ~kBigBit, b.last & ~kBigBit)};
   }
 };
 
@@ -474,7 +479,7 @@ struct AddsSum {
 // the scan of its references' flags (flags_x exclusive; a node's references
 // are contiguous).
 __global__ void decide_kernel(LNode* __restrict__ nodes, int32_t nn, const uint64_t* __restrict__ flags,
-                              const uint64_t* __restrict__ flags_x, Adds* __restrict__ adds) {
+                              const uint64_t* __restrict__ flags_x, Params P, Adds* __restrict__ adds) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nn) return;
   LNode& nd = nodes[i];
@@ -485,21 +490,30 @@ __global__ void decide_kernel(LNode* __restrict__ nodes, int32_t nn, const uint6
     nd.cr = (int32_t)(c >> 32);
   }
   nd.split = (will_try(nd) && !(nd.cl == nd.n && nd.cr == nd.n)) ? 1 : 0;
-  adds[i] = Adds{nd.split ? 2 : 0, nd.split ? nd.cl + nd.cr : 0, nd.split ? 0 : nd.n, 0};
+  Adds a{0, 0, nd.n, (uint32_t)nd.n};
+  if (nd.split) {
+    const bool big = mode_of(nd.cl, nd.depth + 1, P) == kModeBig || mode_of(nd.cr, nd.depth + 1, P) == kModeBig;
+    a = Adds{2, nd.cl + nd.cr, 0, big ? kBigBit : 0u};
+  }
+  adds[i] = a;
 }
 
-// Totals of the scan over a level's nodes.
-__global__ void totals_kernel(const Adds* adds, const Adds* adds_x, int64_t nn, int64_t* out) {
+// Totals of the scan over a level's nodes; the straddler list starts empty
+// again for the next level.
+__global__ void totals_kernel(const Adds* adds, const Adds* adds_x, int64_t nn, int64_t* out, int32_t* n_strad) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
-    const Adds a = adds[nn - 1], x = adds_x[nn - 1];
-    out[0] = (int64_t)x.kids + a.kids;
-    out[1] = (int64_t)x.refs + a.refs;
-    out[2] = (int64_t)x.leaf + a.leaf;
+    const Adds a = AddsSum{}(adds_x[nn - 1], adds[nn - 1]);
+    out[0] = a.kids;
+    out[1] = a.refs;
+    out[2] = a.leaf;
+    out[3] = a.last;
+    *n_strad = 0;
   }
 }
 
 __global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const Adds* __restrict__ adds_x,
-                            LNode* __restrict__ next, int32_t next_gid, int64_t pool_base, GNode* __restrict__ gn) {
+                            LNode* __restrict__ next, int32_t next_gid, int64_t pool_base, GNode* __restrict__ gn,
+                            Params P) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nn) return;
   LNode& nd = nodes[i];
@@ -526,6 +540,8 @@ __global__ void emit_kernel(LNode* __restrict__ nodes, int32_t nn, const Adds* _
     u.rbegin = nd.crbegin + nd.cl;
     u.n = nd.cr;
     b.depth = u.depth = nd.depth + 1;
+    b.mode = mode_of(b.n, b.depth, P);
+    u.mode = mode_of(u.n, u.depth, P);
     b.gid = next_gid + c;
     u.gid = next_gid + c + 1;
     next[c] = b;
@@ -626,45 +642,53 @@ __constant__ int kFaceAxisD[6] = {0, 2, 0, 2, 1, 1};
 __constant__ int kFaceHighD[6] = {0, 1, 1, 0, 1, 0};
 
 // Leaf records: box, ropes pushed down to the deepest node covering the whole
-// face (host: Builder::push_down), and the per-leaf reference counts.
-__global__ void leaves_kernel(const GNode* __restrict__ gn, int32_t total, const int32_t* __restrict__ entry,
-                              const int32_t* __restrict__ lbase, const int32_t* __restrict__ ropes,
-                              LeafRec* __restrict__ leaves, int32_t* __restrict__ leaf_cnt,
-                              int32_t* __restrict__ leaf_gid, int32_t* __restrict__ stats) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= total) return;
+// face (host: Builder::push_down), and the per-leaf reference counts.  Eight
+// threads per node: thread f < 6 of a leaf's eight walks down face f's rope,
+// the last writes the rest of the record.  Bound by the walks' chains of
+// dependent loads; with one thread per leaf, its six walks one after another
+// and an atomic maximum of the depth and leaf size at the end, it took 110 us
+// on a 2^18-triangle soup, and 465 us with eight threads and those atomics.
+__global__ void __launch_bounds__(256) leaves_kernel(const GNode* __restrict__ gn, int32_t total,
+                                                     const int32_t* __restrict__ entry,
+                                                     const int32_t* __restrict__ lbase,
+                                                     const int32_t* __restrict__ ropes, LeafRec* __restrict__ leaves,
+                                                     int32_t* __restrict__ leaf_cnt,
+                                                     int32_t* __restrict__ leaf_gid) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 8 * (int64_t)total) return;
+  const int g = (int)(i >> 3), f = (int)(i & 7);
   const GNode& n = gn[g];
-  if (n.axis >= 0) return;
+  if (n.axis >= 0 || f == 6) return;
   const int lid = lbase[g];
-  LeafRec lr;
-  for (int a = 0; a < 3; ++a) {
-    lr.bmin[a] = n.lo[a];
-    lr.bmax[a] = n.hi[a];
-  }
-  for (int f = 0; f < 6; ++f) {
-    int r = ropes[6 * g + f];
-    while (r >= 0 && gn[r].axis >= 0) {
-      const GNode& t = gn[r];
-      if (t.axis == kFaceAxisD[f]) {
-        r = kFaceHighD[f] ? t.child0 : t.child1;
-      } else if (t.split <= get3(n.lo, t.axis)) {
-        r = t.child1;
-      } else if (t.split >= get3(n.hi, t.axis)) {
-        r = t.child0;
-      } else {
-        break;
-      }
+  LeafRec& lr = leaves[lid];
+  if (f == 7) {
+    for (int a = 0; a < 3; ++a) {
+      lr.bmin[a] = n.lo[a];
+      lr.bmax[a] = n.hi[a];
     }
-    lr.rope[f] = r < 0 ? kNoRope : (gn[r].axis < 0 ? leaf_ref((uint32_t)lbase[r]) : entry[r]);
+    lr.first = 0;
+    lr.count = (uint32_t)n.pool_n;
+    lr.pad[0] = lr.pad[1] = 0;
+    leaf_cnt[lid] = n.pool_n;
+    leaf_gid[lid] = g;
+    return;
   }
-  lr.first = 0;
-  lr.count = (uint32_t)n.pool_n;
-  lr.pad[0] = lr.pad[1] = 0;
-  leaves[lid] = lr;
-  leaf_cnt[lid] = n.pool_n;
-  leaf_gid[lid] = g;
-  atomicMax(&stats[0], n.depth);
-  atomicMax(&stats[1], n.pool_n);
+  const int axis = kFaceAxisD[f];
+  const bool high = kFaceHighD[f] != 0;
+  int r = ropes[6 * (int64_t)g + f];
+  while (r >= 0 && gn[r].axis >= 0) {
+    const GNode& t = gn[r];
+    if (t.axis == axis) {
+      r = high ? t.child0 : t.child1;
+    } else if (t.split <= get3(n.lo, t.axis)) {
+      r = t.child1;
+    } else if (t.split >= get3(n.hi, t.axis)) {
+      r = t.child0;
+    } else {
+      break;
+    }
+  }
+  lr.rope[f] = r < 0 ? kNoRope : (gn[r].axis < 0 ? leaf_ref((uint32_t)lbase[r]) : entry[r]);
 }
 
 __global__ void entries_kernel(const GNode* __restrict__ gn, int32_t total, const int32_t* __restrict__ entry,
@@ -818,13 +842,16 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
   Scanner scan;
   int64_t* tot = nullptr;
   int32_t* n_strad = nullptr;
-  KDB_TRY(B.alloc(&tot, 3));
+  KDB_TRY(B.alloc(&tot, 4));
   KDB_TRY(B.alloc(&n_strad, 1));
   KDB_TRY(refs.ensure(B, n, s));
   KDB_TRY(ref_node.ensure(B, n, s));
   hipLaunchKernelGGL(init_refs_kernel, dim3(blocks(n, 256)), dim3(256), 0, s, tv, n, refs.p, ref_node.p);
   KDB_TRY(hipGetLastError());
   KDB_TRY(lv.ensure(B, 1, s));
+  bool any_big = false;  // the level holds a node that many blocks bin
+  max_leaf = 0;
+  KDB_TRY(hipMemsetAsync(n_strad, 0, sizeof(int32_t), s));
   {
     LNode root{};
     for (int a = 0; a < 3; ++a) {
@@ -835,6 +862,8 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
     root.n = (int32_t)n;
     root.depth = 1;
     root.gid = 0;
+    root.mode = mode_of(root.n, root.depth, P);
+    any_big = root.mode == kModeBig;
     KDB_TRY(hipMemcpyAsync(lv.p, &root, sizeof(root), hipMemcpyHostToDevice, s));
   }
   int64_t nn = 1, nref = n, gused = 1, pused = 0;
@@ -845,14 +874,13 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
 
   while (nn > 0) {
     levels.emplace_back(gbase, (int32_t)nn);
-    hipLaunchKernelGGL(classify_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, P);
-    hipLaunchKernelGGL(exact_split_kernel, dim3(blocks(nn * 64, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, refs.p,
-                       P);
-    KDB_TRY(hist.ensure(B, nn * 6 * nb, s));
-    KDB_TRY(hipMemsetAsync(hist.p, 0, (size_t)(nn * 6 * nb) * sizeof(int32_t), s));
-    hipLaunchKernelGGL(bin_count_kernel, dim3(blocks(nref, kBinChunk)), dim3(256), 0, s, refs.p, ref_node.p, nref,
-                       lv.p, hist.p, P);
-    hipLaunchKernelGGL(binned_split_kernel, dim3(blocks(nn * 64, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, hist.p,
+    KDB_TRY(hist.ensure(B, (nref / kBinChunk + 1) * 6 * nb, s));
+    if (any_big) {
+      KDB_TRY(hipMemsetAsync(hist.p, 0, (size_t)((nref / kBinChunk + 1) * 6 * nb) * sizeof(int32_t), s));
+      hipLaunchKernelGGL(bin_count_kernel, dim3(blocks(nref, kBinChunk)), dim3(256), 0, s, refs.p, ref_node.p, nref,
+                         lv.p, hist.p, P);
+    }
+    hipLaunchKernelGGL(split_kernel, dim3(blocks(nn * 64, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, refs.p, hist.p,
                        P);
     KDB_TRY(hipGetLastError());
 
@@ -861,7 +889,6 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
     KDB_TRY(flags_x.ensure(B, nref, s));
     KDB_TRY(box_l.ensure(B, nref, s));
     KDB_TRY(box_r.ensure(B, nref, s));
-    KDB_TRY(hipMemsetAsync(n_strad, 0, sizeof(int32_t), s));
     hipLaunchKernelGGL(part_flags_kernel, dim3(blocks(nref, kFlagChunk)), dim3(256), 0, s, refs.p, ref_node.p, nref,
                        lv.p, P, flags.p, strad.p, n_strad);
     if (P.clip)
@@ -873,14 +900,16 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
     KDB_TRY(adds.ensure(B, nn, s));
     KDB_TRY(adds_x.ensure(B, nn, s));
     hipLaunchKernelGGL(decide_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, flags.p, flags_x.p,
-                       adds.p);
+                       P, adds.p);
     KDB_TRY(hipGetLastError());
     KDB_TRY(scan.run(B, adds.p, adds_x.p, nn, s, AddsSum{}, Adds{0, 0, 0, 0}));
-    hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, adds.p, adds_x.p, nn, tot);
-    int64_t t3[3] = {0, 0, 0};
-    KDB_TRY(hipMemcpyAsync(t3, tot, sizeof(t3), hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, adds.p, adds_x.p, nn, tot, n_strad);
+    int64_t t4[4] = {0, 0, 0, 0};
+    KDB_TRY(hipMemcpyAsync(t4, tot, sizeof(t4), hipMemcpyDeviceToHost, s));
     KDB_TRY(hipStreamSynchronize(s));
-    const int64_t n_next = t3[0], r_next = t3[1], l_now = t3[2];
+    const int64_t n_next = t4[0], r_next = t4[1], l_now = t4[2];
+    any_big = (t4[3] & kBigBit) != 0;
+    max_leaf = std::max(max_leaf, (int32_t)(t4[3] & ~(int64_t)kBigBit));
     if (gbase + nn + n_next > (int64_t)0x3fffffff || r_next > (int64_t)0x7fffffff) return hipErrorInvalidValue;
 
     KDB_TRY(gn.ensure(B, gused + n_next, s, gused));
@@ -890,7 +919,7 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
     KDB_TRY(nnode.ensure(B, r_next, s));
     const int32_t next_gid = gbase + (int32_t)nn;
     hipLaunchKernelGGL(emit_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, adds_x.p, next.p, next_gid,
-                       pused, gn.p);
+                       pused, gn.p, P);
     hipLaunchKernelGGL(scatter_kernel, dim3(blocks(nref, 256)), dim3(256), 0, s, refs.p, ref_node.p, nref, lv.p,
                        flags.p, flags_x.p, box_l.p, box_r.p, P, nrefs.p, nnode.p, pool.p);
     KDB_TRY(hipGetLastError());
@@ -932,16 +961,14 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
 
   LeafRec* leaves = nullptr;
   NodeEntry* entries = nullptr;
-  int32_t *leaf_cnt = nullptr, *leaf_gid = nullptr, *first = nullptr, *stats = nullptr;
+  int32_t *leaf_cnt = nullptr, *leaf_gid = nullptr, *first = nullptr;
   KDB_TRY(B.alloc(&leaves, (size_t)n_leaves));
   KDB_TRY(B.alloc(&entries, (size_t)total));
   KDB_TRY(B.alloc(&leaf_cnt, (size_t)n_leaves));
   KDB_TRY(B.alloc(&leaf_gid, (size_t)n_leaves));
   KDB_TRY(B.alloc(&first, (size_t)n_leaves + 1));
-  KDB_TRY(B.alloc(&stats, 2));
-  KDB_TRY(hipMemsetAsync(stats, 0, 2 * sizeof(int32_t), s));
-  hipLaunchKernelGGL(leaves_kernel, dim3(blocks(total, 256)), dim3(256), 0, s, gn.p, total, entry, lbase, ropes,
-                     leaves, leaf_cnt, leaf_gid, stats);
+  hipLaunchKernelGGL(leaves_kernel, dim3(blocks(8 * (int64_t)total, 256)), dim3(256), 0, s, gn.p, total, entry, lbase, ropes,
+                     leaves, leaf_cnt, leaf_gid);
   hipLaunchKernelGGL(entries_kernel, dim3(blocks(total, 256)), dim3(256), 0, s, gn.p, total, entry, lbase, entries);
   KDB_TRY(hipGetLastError());
   KDB_TRY(scan.run(B, leaf_cnt, first, n_leaves, s));
@@ -956,15 +983,12 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
   out_nodes.resize((size_t)total);
   out_leaves.resize((size_t)n_leaves);
   out_tris.resize((size_t)n_tris);
-  int32_t st[2] = {0, 0};
   KDB_TRY(hipMemcpyAsync(out_nodes.data(), entries, (size_t)total * sizeof(NodeEntry), hipMemcpyDeviceToHost, s));
   KDB_TRY(hipMemcpyAsync(out_leaves.data(), leaves, (size_t)n_leaves * sizeof(LeafRec), hipMemcpyDeviceToHost, s));
   KDB_TRY(hipMemcpyAsync(out_tris.data(), tris, (size_t)n_tris * sizeof(TriRec), hipMemcpyDeviceToHost, s));
-  KDB_TRY(hipMemcpyAsync(st, stats, sizeof(st), hipMemcpyDeviceToHost, s));
   KDB_TRY(hipStreamSynchronize(s));
   KDB_TRY(hipEventElapsedTime(&device_ms, ev0, ev1));
-  depth = st[0];
-  max_leaf = st[1];
+  depth = (int32_t)levels.size();  // the last level holds leaves only
   return hipSuccess;
 }
 
