@@ -94,42 +94,30 @@ RE_API re_status re_scene_upload(re_ctx* ctx, const re_object* objs, int32_t n_o
   for (int32_t k = 0; k < n_obj; ++k)
     if (!objs[k].tree) return set_err(ctx, RE_ERR_INVALID, "re_scene_upload: object without a tree");
   HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
-  // Concatenate, offsetting entry indices, leaf ids, triangle indices and
-  // prim ids per object (RayEngine/src/World/RTScene.cpp:263-279).
-  std::vector<NodeEntry> nodes;
-  std::vector<LeafRec> leaves;
-  std::vector<TriRec> tris;
+  // The objects' records one after another; their entry indices, leaf ids,
+  // triangle indices and prim ids are offset on the device.
+  DevScene s;
+  s.n_obj = n_obj;
   std::vector<ObjXform> xf(n_obj);
-  std::vector<size_t> leaf_end(n_obj);  // one past each object's last leaf
+  std::vector<ScenePlace> place(n_obj);
   for (int32_t k = 0; k < n_obj; ++k) {
     const re_object& ob = objs[k];
-    const auto& tn = kd_nodes(ob.tree);
-    const auto& tl = kd_leaves(ob.tree);
-    const auto& tt = kd_tris(ob.tree);
     re_kd_info info;
     re_kd_get_info(ob.tree, &info);
-    const uint32_t nb = (uint32_t)nodes.size(), lb = (uint32_t)leaves.size(), tb = (uint32_t)tris.size();
-    if ((uint64_t)nb + tn.size() >= 0x3fffffffull || (uint64_t)lb + tl.size() >= 0x3fffffffull)
+    ScenePlace& p = place[k];
+    p.n_nodes = (int64_t)kd_nodes(ob.tree).size();
+    p.n_leaves = (int64_t)kd_leaves(ob.tree).size();
+    p.n_tris = (int64_t)kd_tris(ob.tree).size();
+    if (s.n_nodes + p.n_nodes >= 0x3fffffffll || s.n_leaves + p.n_leaves >= 0x3fffffffll)
       return set_err(ctx, RE_ERR_INVALID, "re_scene_upload: scene too large for 30-bit node indices");
-    for (NodeEntry e : tn) {
-      if ((e.meta >> 30) == 3u) e.meta = kLeafMeta | ((e.meta & 0x3fffffffu) + lb);
-      else e.meta = (e.meta & 0xc0000000u) | ((e.meta & 0x3fffffffu) + nb);
-      nodes.push_back(e);
-    }
-    for (LeafRec l : tl) {
-      for (int f = 0; f < 6; ++f) {
-        int32_t r = l.rope[f];
-        if (r == kNoRope) continue;
-        l.rope[f] = ref_is_leaf(r) ? leaf_ref(ref_leaf_id(r) + lb) : r + (int32_t)nb;
-      }
-      l.first += tb;
-      leaves.push_back(l);
-    }
-    leaf_end[k] = leaves.size();
-    for (TriRec t : tt) {
-      t.prim += ob.prim_offset;
-      tris.push_back(t);
-    }
+    p.node_base = (uint32_t)s.n_nodes;
+    p.leaf_base = (uint32_t)s.n_leaves;
+    p.tri_base = (uint32_t)s.n_trirecs;
+    p.prim_offset = ob.prim_offset;
+    p.object = k;
+    s.n_nodes += p.n_nodes;
+    s.n_leaves += p.n_leaves;
+    s.n_trirecs += p.n_tris;
     ObjXform& x = xf[k];
     for (int a = 0; a < 3; ++a) {
       x.loc[a] = ob.location[a];
@@ -139,49 +127,41 @@ RE_API re_status re_scene_upload(re_ctx* ctx, const re_object* objs, int32_t n_o
     x.sin_y = ob.sin_rot_y;
     x.cos_y = ob.cos_rot_y;
     x.is_character = ob.is_character;
-    x.root = (int32_t)nb;
+    x.root = (int32_t)p.node_base;
   }
-  DevScene s;
-  s.n_obj = n_obj;
-  s.n_nodes = (int64_t)nodes.size();
-  s.n_leaves = (int64_t)leaves.size();
-  s.n_trirecs = (int64_t)tris.size();
-  // Trailing pad entries (leaf entries of leaf 0) for window reads at the end.
-  nodes.resize(nodes.size() + kNodePad, NodeEntry{0.0f, kLeafMeta});
-  std::vector<DevLeaf> dleaves(leaves.size());
-  // pad[0] of a device leaf record holds its object's index (the walk-start
-  // hint check reads it)
-  for (int32_t k = 0, i = 0; k < n_obj; ++k)
-    for (; (size_t)i < leaf_end[k]; ++i) {
-      dleaves[i] = dev_leaf(leaves[i]);
-      dleaves[i].pad[0] = (uint32_t)k;
-    }
-  auto up =[&](void** dst, const void* src, size_t bytes, const char* what) -> re_status {
+  hipError_t e = hipSuccess;
+  auto alloc = [&](void** dst, size_t bytes) {
     if (bytes == 0) bytes = 64;  // keep every pointer valid
-    hipError_t e = hipMalloc(dst, bytes);
-    if (e != hipSuccess) return hip_err(ctx, e, what);
-    if (src) {
-      e = hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
-      if (e != hipSuccess) return hip_err(ctx, e, what);
-    }
+    if (e == hipSuccess) e = hipMalloc(dst, bytes);
     s.bytes += (int64_t)bytes;
-    return RE_OK;
   };
-  re_status st;
-  if ((st = up((void**)&s.nodes, nodes.empty() ? nullptr : nodes.data(), nodes.size() * sizeof(NodeEntry), "upload nodes")) ||
-      (st = up((void**)&s.leaves, dleaves.empty() ? nullptr : dleaves.data(), dleaves.size() * sizeof(DevLeaf), "upload leaves")) ||
-      (st = up((void**)&s.tris, tris.empty() ? nullptr : tris.data(), tris.size() * sizeof(TriRec), "upload tris")) ||
-      (st = up((void**)&s.objs, xf.data(), xf.size() * sizeof(ObjXform), "upload objects"))) {
-    (void)hipStreamSynchronize(ctx->stream);
-    free_scene(s);
-    return st;
+  auto copy = [&](void* dst, const void* src, size_t bytes) {
+    if (e == hipSuccess && bytes > 0) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
+  };
+  // Trailing pad entries (leaf entries of leaf 0) for window reads at the end.
+  const NodeEntry pad[kNodePad] = {{0.0f, kLeafMeta}, {0.0f, kLeafMeta}};
+  alloc((void**)&s.nodes, (size_t)(s.n_nodes + kNodePad) * sizeof(NodeEntry));
+  alloc((void**)&s.leaves, (size_t)s.n_leaves * sizeof(DevLeaf));
+  alloc((void**)&s.tris, (size_t)s.n_trirecs * sizeof(TriRec));
+  alloc((void**)&s.objs, xf.size() * sizeof(ObjXform));
+  for (int32_t k = 0; k < n_obj && e == hipSuccess; ++k) {
+    ScenePlace& p = place[k];
+    p.nodes = s.nodes + p.node_base;
+    p.leaves = s.leaves + p.leaf_base;
+    p.tris = s.tris + p.tri_base;
+    copy(p.nodes, kd_nodes(objs[k].tree).data(), (size_t)p.n_nodes * sizeof(NodeEntry));
+    copy(p.leaves, kd_leaves(objs[k].tree).data(), (size_t)p.n_leaves * sizeof(LeafRec));
+    copy(p.tris, kd_tris(objs[k].tree).data(), (size_t)p.n_tris * sizeof(TriRec));
+    if (e == hipSuccess) e = launch_scene_place(p, ctx->stream);
   }
-  hipError_t e = hipStreamSynchronize(ctx->stream);
+  copy(s.nodes + s.n_nodes, pad, sizeof(pad));
+  copy(s.objs, xf.data(), xf.size() * sizeof(ObjXform));
+  const hipError_t es = hipStreamSynchronize(ctx->stream);  // also after an error: nothing is in flight when it is freed
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) {
     free_scene(s);
-    return hip_err(ctx, e, "re_scene_upload sync");
+    return hip_err(ctx, e, "re_scene_upload");
   }
-  s.h_leaves = std::move(leaves);
   int32_t id = ctx->next_id++;
   ctx->scenes[id] = std::move(s);
   *scene_id = id;
@@ -240,20 +220,25 @@ RE_API re_status re_scene_info(re_ctx* ctx, int32_t scene_id, int64_t sizes[4]) 
 
 RE_API re_status re_scene_export(re_ctx* ctx, int32_t scene_id, void* nodes, void* leaves, void* tris, void* objs) {
   if (!ctx) return fail(RE_ERR_INVALID, "re_scene_export: null ctx");
+  return guarded(ctx, "re_scene_export", [&]() -> re_status {
   auto it = ctx->scenes.find(scene_id);
   if (it == ctx->scenes.end()) return set_err(ctx, RE_ERR_NOT_FOUND, "re_scene_export: unknown scene");
   const DevScene& s = it->second;
   HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
   if (nodes && s.n_nodes)
     HIP_TRY(ctx, hipMemcpyAsync(nodes, s.nodes, s.n_nodes * sizeof(NodeEntry), hipMemcpyDeviceToHost, ctx->stream), "export nodes");
-  // Leaf records in the flat field order (host copy; the device holds them as DevLeaf).
-  if (leaves && s.n_leaves) std::memcpy(leaves, s.h_leaves.data(), s.n_leaves * sizeof(LeafRec));
+  // Leaf records in the flat field order (the device holds them as DevLeaf).
+  std::vector<DevLeaf> dl(leaves ? (size_t)s.n_leaves : 0);
+  if (!dl.empty())
+    HIP_TRY(ctx, hipMemcpyAsync(dl.data(), s.leaves, dl.size() * sizeof(DevLeaf), hipMemcpyDeviceToHost, ctx->stream), "export leaves");
   if (tris && s.n_trirecs)
     HIP_TRY(ctx, hipMemcpyAsync(tris, s.tris, s.n_trirecs * sizeof(TriRec), hipMemcpyDeviceToHost, ctx->stream), "export tris");
   if (objs)
     HIP_TRY(ctx, hipMemcpyAsync(objs, s.objs, s.n_obj * sizeof(ObjXform), hipMemcpyDeviceToHost, ctx->stream), "export objs");
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream), "export sync");
+  for (size_t i = 0; i < dl.size(); ++i) static_cast<LeafRec*>(leaves)[i] = flat_leaf(dl[i]);
   return RE_OK;
+  });
 }
 
 RE_API void re_trace_default_params(re_trace_params* p) {

@@ -23,8 +23,7 @@ const std::vector<LeafRec>& kd_leaves(const re_kdtree* t);
 const std::vector<TriRec>& kd_tris(const re_kdtree* t);
 
 // A scene resident in HBM: the concatenated trees of its objects (leaf
-// records in the device order of DevLeaf; the host keeps the flat records for
-// re_scene_export).
+// records in the device order of DevLeaf).
 struct DevScene {
   NodeEntry* nodes = nullptr;
   DevLeaf* leaves = nullptr;
@@ -33,13 +32,25 @@ struct DevScene {
   int32_t n_obj = 0;
   int64_t n_nodes = 0, n_leaves = 0, n_trirecs = 0;
   int64_t bytes = 0;
-  std::vector<LeafRec> h_leaves;
   // hit attributes (re_scene_set_attributes), indexed by prim id
   float* attr_geom = nullptr;  // v0, e1, e2 (9 floats) per prim
   float* attr_nrm = nullptr;   // vertex normals n0, n1, n2 (9 floats) per prim
   float* attr_uv = nullptr;    // vertex uvs uv0, uv1, uv2 (6 floats) per prim, or null
   int64_t n_attr = 0;
 };
+
+// One object's tree records inside a scene's arrays, copied as the builder
+// left them, and their place: the bases are the counts of the records before
+// them (kernels/scene.hip).
+struct ScenePlace {
+  NodeEntry* nodes;
+  DevLeaf* leaves;  // LeafRec records until placed
+  TriRec* tris;
+  int64_t n_nodes, n_leaves, n_tris;
+  uint32_t node_base, leaf_base, tri_base;
+  int32_t prim_offset, object;
+};
+hipError_t launch_scene_place(const ScenePlace& P, hipStream_t s);
 
 struct AttrLaunch {
   const DevScene* scene;

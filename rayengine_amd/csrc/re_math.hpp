@@ -246,6 +246,19 @@ RE_HD DevLeaf dev_leaf(const LeafRec& l) {
   return d;
 }
 
+RE_HD LeafRec flat_leaf(const DevLeaf& d) {
+  LeafRec l;
+  for (int a = 0; a < 3; ++a) {
+    l.bmin[a] = d.bmin[a];
+    l.bmax[a] = d.bmax[a];
+  }
+  for (int f = 0; f < 6; ++f) l.rope[f] = d.rope[f];
+  l.first = d.first;
+  l.count = d.count;
+  l.pad[0] = l.pad[1] = 0;
+  return l;
+}
+
 static_assert(sizeof(NodeEntry) == 8, "node entry is 8 bytes");
 static_assert(sizeof(LeafRec) == 64, "leaf record is 64 bytes");
 static_assert(sizeof(DevLeaf) == 64, "device leaf record is 64 bytes");
