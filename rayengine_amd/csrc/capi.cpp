@@ -76,6 +76,8 @@ RE_API void re_destroy(re_ctx* ctx) {
                     (void*)kv.second.small, (void*)kv.second.partial, (void*)kv.second.grad, (void*)kv.second.loss})
       if (p) (void)hipFree(p);
   if (ctx->stage) (void)hipFree(ctx->stage);
+  if (ctx->kd_build.chunk) (void)hipFree(ctx->kd_build.chunk);
+  if (ctx->kd_build.totals) (void)hipHostFree(ctx->kd_build.totals);
   if (ctx->counts_buf) (void)hipFree(ctx->counts_buf);
   for (int i = 0; i < 2 * re_ctx::kRing; ++i)
     if (ctx->ring[i]) (void)hipEventDestroy(ctx->ring[i]);

@@ -11,12 +11,12 @@
 using namespace re;
 
 namespace re {
-re_kdtree* kd_from_arrays(std::vector<NodeEntry>&& nodes, std::vector<LeafRec>&& leaves, std::vector<TriRec>&& tris,
+re_kdtree* kd_from_arrays(RecVec<NodeEntry>&& nodes, RecVec<LeafRec>&& leaves, RecVec<TriRec>&& tris,
                           const re_kd_info& info);
 namespace kdb {
 hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, const float* root_max,
-                        const Params& P, hipStream_t s, std::vector<NodeEntry>& out_nodes,
-                        std::vector<LeafRec>& out_leaves, std::vector<TriRec>& out_tris, int32_t& depth,
+                        const Params& P, Workspace& ws, hipStream_t s, RecVec<NodeEntry>& out_nodes,
+                        RecVec<LeafRec>& out_leaves, RecVec<TriRec>& out_tris, int32_t& depth,
                         int32_t& max_leaf, float& device_ms);
 }  // namespace kdb
 }  // namespace re
@@ -54,13 +54,13 @@ RE_API re_status re_kd_build_gpu(re_ctx* ctx, const float* tri_v, int64_t n_tris
   HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
   kdb::Params P{p.max_leaf_tris, p.max_depth, p.n_bins, p.clip ? 1 : 0, p.cost_traversal, p.cost_intersect,
                 p.empty_bonus};
-  std::vector<NodeEntry> nodes;
-  std::vector<LeafRec> leaves;
-  std::vector<TriRec> tris;
+  RecVec<NodeEntry> nodes;
+  RecVec<LeafRec> leaves;
+  RecVec<TriRec> tris;
   int32_t depth = 0, max_leaf = 0;
   float ms = 0.0f;
   try {
-    hipError_t e = kdb::build_device(tri_v, n_tris, rmin, rmax, P, ctx->stream, nodes, leaves, tris, depth, max_leaf, ms);
+    hipError_t e = kdb::build_device(tri_v, n_tris, rmin, rmax, P, ctx->kd_build, ctx->stream, nodes, leaves, tris, depth, max_leaf, ms);
     if (e != hipSuccess) return hip_err(ctx, e, "re_kd_build_gpu");
   } catch (const std::bad_alloc&) {
     return set_err(ctx, RE_ERR_OOM, "re_kd_build_gpu: out of host memory");

@@ -21,13 +21,14 @@
 
 #include "errors.hpp"
 #include "../re_math.hpp"
+#include "../rec_vec.hpp"
 
 using namespace re;
 
 struct re_kdtree {
-  std::vector<NodeEntry> nodes;
-  std::vector<LeafRec> leaves;
-  std::vector<TriRec> tris;
+  RecVec<NodeEntry> nodes;
+  RecVec<LeafRec> leaves;
+  RecVec<TriRec> tris;
   re_kd_info info;
 };
 
@@ -477,7 +478,7 @@ RE_API re_status re_kd_export(const re_kdtree* tree, void* nodes, void* leaves, 
 
 // Internal accessors for the device upload (capi.cpp).
 namespace re {
-re_kdtree* kd_from_arrays(std::vector<NodeEntry>&& nodes, std::vector<LeafRec>&& leaves, std::vector<TriRec>&& tris,
+re_kdtree* kd_from_arrays(RecVec<NodeEntry>&& nodes, RecVec<LeafRec>&& leaves, RecVec<TriRec>&& tris,
                           const re_kd_info& info) {
   re_kdtree* t = new (std::nothrow) re_kdtree();
   if (!t) return nullptr;
@@ -487,7 +488,7 @@ re_kdtree* kd_from_arrays(std::vector<NodeEntry>&& nodes, std::vector<LeafRec>&&
   t->info = info;
   return t;
 }
-const std::vector<NodeEntry>& kd_nodes(const re_kdtree* t) { return t->nodes; }
-const std::vector<LeafRec>& kd_leaves(const re_kdtree* t) { return t->leaves; }
-const std::vector<TriRec>& kd_tris(const re_kdtree* t) { return t->tris; }
+const RecVec<NodeEntry>& kd_nodes(const re_kdtree* t) { return t->nodes; }
+const RecVec<LeafRec>& kd_leaves(const re_kdtree* t) { return t->leaves; }
+const RecVec<TriRec>& kd_tris(const re_kdtree* t) { return t->tris; }
 }  // namespace re

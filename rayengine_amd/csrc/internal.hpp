@@ -10,17 +10,19 @@
 
 #include "../../include/rayengine.h"
 #include "host/batch_plan.hpp"
+#include "kdbuild.hpp"
 #include "mlp_layout.hpp"
 #include "re_math.hpp"
+#include "rec_vec.hpp"
 #include "terrain_math.hpp"
 
 struct re_kdtree;
 
 namespace re {
 
-const std::vector<NodeEntry>& kd_nodes(const re_kdtree* t);
-const std::vector<LeafRec>& kd_leaves(const re_kdtree* t);
-const std::vector<TriRec>& kd_tris(const re_kdtree* t);
+const RecVec<NodeEntry>& kd_nodes(const re_kdtree* t);
+const RecVec<LeafRec>& kd_leaves(const re_kdtree* t);
+const RecVec<TriRec>& kd_tris(const re_kdtree* t);
 
 // A scene resident in HBM: the concatenated trees of its objects (leaf
 // records in the device order of DevLeaf).
@@ -400,6 +402,7 @@ struct re_ctx {
   int64_t coop_refill_grid[3] = {0, 0, 0};  // the same for variant 5
   void* stage = nullptr;
   size_t stage_bytes = 0;
+  re::kdb::Workspace kd_build;  // re_kd_build_gpu
   std::string err;
 
   hipError_t launch_begin() { return hipEventRecord(ring[2 * (n_launch % kRing)], stream); }

@@ -64,6 +64,17 @@ constexpr int kMaxBins = 64;
 constexpr int kBinChunk = 1024;
 constexpr int kWaveBinMax = kBinChunk;
 
+// Device and pinned host memory that a context keeps between its device
+// builds: one chunk of what the last build took, at most kKeepBytes, and the
+// words a level's totals are written to.  A build that needs more takes and
+// frees the rest itself.
+constexpr size_t kKeepBytes = (size_t)256 << 20;
+struct Workspace {
+  char* chunk = nullptr;
+  size_t bytes = 0;
+  int64_t* totals = nullptr;  // pinned, 4 words
+};
+
 RE_HD int32_t mode_of(int32_t n, int32_t depth, const Params& P) {
   if (n <= P.max_leaf || depth >= P.max_depth) return kModeLeaf;
   return n <= kExactMax ? kModeExact : (n <= kWaveBinMax ? kModeBinned : kModeBig);

@@ -498,8 +498,9 @@ __global__ void decide_kernel(LNode* __restrict__ nodes, int32_t nn, const uint6
   adds[i] = a;
 }
 
-// Totals of the scan over a level's nodes; the straddler list starts empty
-// again for the next level.
+// Totals of the scan over a level's nodes, to pinned host memory (read after
+// the stream's synchronisation); the straddler list starts empty again for
+// the next level.
 __global__ void totals_kernel(const Adds* adds, const Adds* adds_x, int64_t nn, int64_t* out, int32_t* n_strad) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     const Adds a = AddsSum{}(adds_x[nn - 1], adds[nn - 1]);
@@ -737,20 +738,63 @@ __global__ void tris_kernel(const GNode* __restrict__ gn, int32_t n_leaves, cons
 
 unsigned blocks(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
-// Device buffers freed on scope exit.  release() only marks a buffer; it is
-// freed by flush(), which the caller calls after synchronizing the stream,
-// so no buffer is freed while queued work may still use it.
+// Device buffers of one build.  Those below kOwnBytes are carved from chunks,
+// first the one the context keeps, and are reused only by the next build (a
+// level's hipMalloc and hipFree calls, 157 of each on a 2^18-triangle soup,
+// took longer than its kernels); larger ones are allocated one by one, so
+// that a large build holds no more than its live arrays.  release() only
+// marks such a buffer; it is freed by flush(), which the caller calls after
+// synchronizing the stream, so no buffer is freed while queued work may still
+// use it.
 struct Bufs {
-  std::vector<void*> ptrs, dead;
+  static constexpr size_t kOwnBytes = (size_t)64 << 20, kMinChunk = (size_t)8 << 20;
+  Workspace& ws;
+  hipStream_t s;
+  std::vector<void*> chunks, ptrs, dead;  // allocated here; ptrs: one buffer each
+  char* at = nullptr;
+  size_t left = 0, carved = 0;    // of the current chunk; of all chunks
+  Bufs(Workspace& w, hipStream_t st) : ws(w), s(st), at(w.chunk), left(w.bytes) {}
   ~Bufs() {
+    // The end of the build, or an error on the way: nothing may use the
+    // buffers any more.  The kept chunk becomes one of what was carved.
+    (void)hipStreamSynchronize(s);
+    for (void* p : chunks) (void)hipFree(p);
     for (void* p : ptrs) (void)hipFree(p);
+    if (carved > ws.bytes && ws.bytes < kKeepBytes) {
+      if (ws.chunk) (void)hipFree(ws.chunk);
+      ws.chunk = nullptr;
+      ws.bytes = 0;
+      const size_t want = std::min(carved + carved / 8, kKeepBytes);
+      if (hipMalloc((void**)&ws.chunk, want) == hipSuccess) ws.bytes = want;
+      else (void)hipGetLastError();  // the next build allocates its own
+    }
+  }
+  hipError_t take(void** p, size_t bytes) {
+    *p = nullptr;
+    bytes = (bytes + 255) & ~(size_t)255;
+    if (bytes >= kOwnBytes) {
+      const hipError_t e = hipMalloc(p, bytes);
+      if (e == hipSuccess) ptrs.push_back(*p);
+      return e;
+    }
+    if (bytes > left) {
+      const size_t chunk = std::max(bytes, std::min(std::max(kMinChunk, carved), kOwnBytes));
+      void* q = nullptr;
+      const hipError_t e = hipMalloc(&q, chunk);
+      if (e != hipSuccess) return e;
+      chunks.push_back(q);
+      at = (char*)q;
+      left = chunk;
+    }
+    *p = at;
+    at += bytes;
+    left -= bytes;
+    carved += bytes;
+    return hipSuccess;
   }
   template <typename T>
   hipError_t alloc(T** p, size_t count) {
-    *p = nullptr;
-    hipError_t e = hipMalloc((void**)p, std::max<size_t>(count, 1) * sizeof(T));
-    if (e == hipSuccess) ptrs.push_back(*p);
-    return e;
+    return take((void**)p, std::max<size_t>(count, 1) * sizeof(T));
   }
   void release(void* p) {
     if (p && std::find(ptrs.begin(), ptrs.end(), p) != ptrs.end()) dead.push_back(p);
@@ -811,10 +855,11 @@ struct Scanner {
 // Builds the tree of n (> 0) triangles; the outputs are host vectors.
 // device_ms gets the device time of the build (events around all of it).
 hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, const float* root_max,
-                        const Params& P, hipStream_t s, std::vector<NodeEntry>& out_nodes,
-                        std::vector<LeafRec>& out_leaves, std::vector<TriRec>& out_tris, int32_t& depth,
+                        const Params& P, Workspace& ws, hipStream_t s, RecVec<NodeEntry>& out_nodes,
+                        RecVec<LeafRec>& out_leaves, RecVec<TriRec>& out_tris, int32_t& depth,
                         int32_t& max_leaf, float& device_ms) {
-  Bufs B;
+  if (!ws.totals) KDB_TRY(hipHostMalloc((void**)&ws.totals, 4 * sizeof(int64_t), hipHostMallocDefault));
+  Bufs B(ws, s);
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   KDB_TRY(hipEventCreate(&ev0));
   KDB_TRY(hipEventCreate(&ev1));
@@ -841,9 +886,7 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
   Arr<GNode> gn;
   Arr<int32_t> pool;
   Scanner scan;
-  int64_t* tot = nullptr;
   int32_t* n_strad = nullptr;
-  KDB_TRY(B.alloc(&tot, 4));
   KDB_TRY(B.alloc(&n_strad, 1));
   KDB_TRY(refs.ensure(B, n, s));
   KDB_TRY(ref_node.ensure(B, n, s));
@@ -904,10 +947,10 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
                        P, adds.p);
     KDB_TRY(hipGetLastError());
     KDB_TRY(scan.run(B, adds.p, adds_x.p, nn, s, AddsSum{}, Adds{0, 0, 0, 0}));
-    hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, adds.p, adds_x.p, nn, tot, n_strad);
-    int64_t t4[4] = {0, 0, 0, 0};
-    KDB_TRY(hipMemcpyAsync(t4, tot, sizeof(t4), hipMemcpyDeviceToHost, s));
+    hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, adds.p, adds_x.p, nn, ws.totals, n_strad);
+    KDB_TRY(hipGetLastError());
     KDB_TRY(hipStreamSynchronize(s));
+    const int64_t* t4 = ws.totals;
     const int64_t n_next = t4[0], r_next = t4[1], l_now = t4[2];
     any_big = (t4[3] & kBigBit) != 0;
     max_leaf = std::max(max_leaf, (int32_t)(t4[3] & ~(int64_t)kBigBit));
