@@ -14,7 +14,7 @@ namespace re {
 re_kdtree* kd_from_arrays(RecVec<NodeEntry>&& nodes, RecVec<LeafRec>&& leaves, RecVec<TriRec>&& tris,
                           const re_kd_info& info);
 namespace kdb {
-hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, const float* root_max,
+hipError_t build_device(const float* tri_v, int64_t n, float* root_min, float* root_max, bool& finite,
                         const Params& P, Workspace& ws, hipStream_t s, RecVec<NodeEntry>& out_nodes,
                         RecVec<LeafRec>& out_leaves, RecVec<TriRec>& out_tris, int32_t& depth,
                         int32_t& max_leaf, float& device_ms);
@@ -36,17 +36,6 @@ RE_API re_status re_kd_build_gpu(re_ctx* ctx, const float* tri_v, int64_t n_tris
   if (p.split_rule != 0)
     return set_err(ctx, RE_ERR_UNSUPPORTED, "re_kd_build_gpu: the spatial-median rule is built on the host (re_kd_build)");
   if (device_ms) *device_ms = 0.0f;
-  // Root box and input check on the host, as re_kd_build does them.
-  float rmin[3] = {kInf, kInf, kInf}, rmax[3] = {-kInf, -kInf, -kInf};
-  for (int64_t i = 0; i < n_tris; ++i) {
-    const float* t = tri_v + 9 * i;
-    for (int k = 0; k < 9; ++k)
-      if (!std::isfinite(t[k])) return set_err(ctx, RE_ERR_INVALID, "re_kd_build_gpu: non-finite vertex");
-    for (int a = 0; a < 3; ++a) {
-      rmin[a] = std::min(rmin[a], std::min(std::min(t[a], t[3 + a]), t[6 + a]));
-      rmax[a] = std::max(rmax[a], std::max(std::max(t[a], t[3 + a]), t[6 + a]));
-    }
-  }
   if (n_tris == 0) {  // a single empty leaf: nothing for the device to do
     re_status st = re_kd_build(tri_v, 0, &p, out);
     return st ? set_err(ctx, st, "re_kd_build_gpu: empty build failed") : RE_OK;
@@ -58,10 +47,12 @@ RE_API re_status re_kd_build_gpu(re_ctx* ctx, const float* tri_v, int64_t n_tris
   RecVec<LeafRec> leaves;
   RecVec<TriRec> tris;
   int32_t depth = 0, max_leaf = 0;
-  float ms = 0.0f;
+  float ms = 0.0f, rmin[3] = {kInf, kInf, kInf}, rmax[3] = {-kInf, -kInf, -kInf};
+  bool finite = true;
   try {
-    hipError_t e = kdb::build_device(tri_v, n_tris, rmin, rmax, P, ctx->kd_build, ctx->stream, nodes, leaves, tris, depth, max_leaf, ms);
+    hipError_t e = kdb::build_device(tri_v, n_tris, rmin, rmax, finite, P, ctx->kd_build, ctx->stream, nodes, leaves, tris, depth, max_leaf, ms);
     if (e != hipSuccess) return hip_err(ctx, e, "re_kd_build_gpu");
+    if (!finite) return set_err(ctx, RE_ERR_INVALID, "re_kd_build_gpu: non-finite vertex");
   } catch (const std::bad_alloc&) {
     return set_err(ctx, RE_ERR_OOM, "re_kd_build_gpu: out of host memory");
   }

@@ -138,19 +138,76 @@ __device__ bool clip_box(const float* __restrict__ tv, int32_t prim, const float
 
 // ---------------------------------------------------------------- per level
 
-__global__ void init_refs_kernel(const float* __restrict__ tv, int64_t n, Ref* __restrict__ refs,
-                                 int32_t* __restrict__ ref_node) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float* t = tv + 9 * i;
-  Ref r;
-  r.prim = (int32_t)i;
-  for (int a = 0; a < 3; ++a) {
-    r.lo[a] = smin(smin(t[a], t[3 + a]), t[6 + a]);
-    r.hi[a] = smax(smax(t[a], t[3 + a]), t[6 + a]);
+// What the host keeps of the soup: per axis the vertex that gives the root
+// box its minimum and its maximum, as keys (value in unsigned order, vertex
+// index) whose minimum is taken, and whether any coordinate is not finite.
+// The host scans vertices in order and replaces a bound only by a strictly
+// lower (higher) value, so among equal values, +0 and -0 included, the first
+// vertex wins: the key's low word.
+struct SoupBounds {
+  unsigned long long lo[3], hi[3];
+  uint32_t bad;
+};
+
+__device__ __forceinline__ uint32_t ordered(float x) {
+  const uint32_t u = __float_as_uint(x == 0.0f ? 0.0f : x);
+  return (u & 0x80000000u) ? ~u : u | 0x80000000u;
+}
+
+__global__ void clear_bounds_kernel(SoupBounds* __restrict__ b) {
+  if (threadIdx.x < 3) b->lo[threadIdx.x] = b->hi[threadIdx.x] = ~0ull;
+  if (threadIdx.x == 0) b->bad = 0;
+}
+
+// The root's references, and the bounds of the soup on the way (a pass of their
+// own on the host before: a build of 2^18 triangles 5.52 ms, now 5.25).  At
+// most kInitBlocks blocks, so that few blocks add to the bounds.
+constexpr int kInitBlocks = 512;
+
+__global__ void __launch_bounds__(256) init_refs_kernel(const float* __restrict__ tv, int64_t n,
+                                                        Ref* __restrict__ refs, int32_t* __restrict__ ref_node,
+                                                        SoupBounds* __restrict__ bounds) {
+  __shared__ unsigned long long sh[6];
+  __shared__ int any_bad;
+  if (threadIdx.x < 6) sh[threadIdx.x] = ~0ull;
+  if (threadIdx.x == 0) any_bad = 0;
+  __syncthreads();
+  unsigned long long kl[3] = {~0ull, ~0ull, ~0ull}, kh[3] = {~0ull, ~0ull, ~0ull};
+  bool bad = false;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const float* t = tv + 9 * i;
+    Ref r;
+    r.prim = (int32_t)i;
+    for (int a = 0; a < 3; ++a) {
+      const float v[3] = {t[a], t[3 + a], t[6 + a]};
+      r.lo[a] = smin(smin(v[0], v[1]), v[2]);
+      r.hi[a] = smax(smax(v[0], v[1]), v[2]);
+      for (int k = 0; k < 3; ++k) {
+        bad = bad || !isfinite(v[k]);
+        const uint32_t o = ordered(v[k]);
+        const unsigned long long at = (unsigned long long)(3 * i + k);
+        kl[a] = min(kl[a], ((unsigned long long)o << 32) | at);
+        kh[a] = min(kh[a], ((unsigned long long)(~o) << 32) | at);
+      }
+    }
+    refs[i] = r;
+    ref_node[i] = 0;
   }
-  refs[i] = r;
-  ref_node[i] = 0;
+  for (int a = 0; a < 3; ++a) {
+    for (int off = 32; off >= 1; off >>= 1) {
+      kl[a] = min(kl[a], (unsigned long long)__shfl_xor((unsigned long long)kl[a], off));
+      kh[a] = min(kh[a], (unsigned long long)__shfl_xor((unsigned long long)kh[a], off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicMin(&sh[a], kl[a]);
+      atomicMin(&sh[3 + a], kh[a]);
+    }
+  }
+  if (bad) any_bad = 1;
+  __syncthreads();
+  if (threadIdx.x < 3) atomicMin(&bounds->lo[threadIdx.x], sh[threadIdx.x]);
+  else if (threadIdx.x < 6) atomicMin(&bounds->hi[threadIdx.x - 3], sh[threadIdx.x]);
+  if (threadIdx.x == 6 && any_bad) atomicOr(&bounds->bad, 1u);
 }
 
 __device__ __forceinline__ int bin_of(float v, float lo, float hi, float scale, int nb) {
@@ -854,7 +911,9 @@ struct Scanner {
 
 // Builds the tree of n (> 0) triangles; the outputs are host vectors.
 // device_ms gets the device time of the build (events around all of it).
-hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, const float* root_max,
+// root_min and root_max receive the root box; with a coordinate that is not
+// finite, finite is set to false and nothing is built.
+hipError_t build_device(const float* tri_v, int64_t n, float* root_min, float* root_max, bool& finite,
                         const Params& P, Workspace& ws, hipStream_t s, RecVec<NodeEntry>& out_nodes,
                         RecVec<LeafRec>& out_leaves, RecVec<TriRec>& out_tris, int32_t& depth,
                         int32_t& max_leaf, float& device_ms) {
@@ -890,8 +949,21 @@ hipError_t build_device(const float* tri_v, int64_t n, const float* root_min, co
   KDB_TRY(B.alloc(&n_strad, 1));
   KDB_TRY(refs.ensure(B, n, s));
   KDB_TRY(ref_node.ensure(B, n, s));
-  hipLaunchKernelGGL(init_refs_kernel, dim3(blocks(n, 256)), dim3(256), 0, s, tv, n, refs.p, ref_node.p);
+  SoupBounds* bounds = nullptr;
+  KDB_TRY(B.alloc(&bounds, 1));
+  hipLaunchKernelGGL(clear_bounds_kernel, dim3(1), dim3(64), 0, s, bounds);
+  hipLaunchKernelGGL(init_refs_kernel, dim3(std::min(blocks(n, 256), (unsigned)kInitBlocks)), dim3(256), 0, s, tv, n,
+                     refs.p, ref_node.p, bounds);
   KDB_TRY(hipGetLastError());
+  SoupBounds sb;
+  KDB_TRY(hipMemcpyAsync(&sb, bounds, sizeof(sb), hipMemcpyDeviceToHost, s));
+  KDB_TRY(hipStreamSynchronize(s));
+  finite = sb.bad == 0;
+  if (!finite) return hipSuccess;
+  for (int a = 0; a < 3; ++a) {
+    root_min[a] = std::min(kInf, tri_v[3 * (int64_t)(uint32_t)sb.lo[a] + a]);
+    root_max[a] = std::max(-kInf, tri_v[3 * (int64_t)(uint32_t)sb.hi[a] + a]);
+  }
   KDB_TRY(lv.ensure(B, 1, s));
   bool any_big = false;  // the level holds a node that many blocks bin
   max_leaf = 0;

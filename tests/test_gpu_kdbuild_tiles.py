@@ -20,3 +20,19 @@ def _equal(tri, ctx, **kw):
 def test_tile_edges(gpu_ctx, n, leaf, clip):
     # large triangles: most references straddle the first planes
     _equal(re.random_tris(n, n, -2.0, 2.0, 0.5, 3.0), gpu_ctx, max_leaf_tris=leaf, max_depth=16, clip=clip)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 140000])
+def test_root_box_and_refusal(gpu_ctx, n):
+    # bounds over the last partial block and past the grid's first round (512 blocks of 256); zeros of both signs
+    tri = re.random_tris(n, n, -2.0, 2.0, 0.1, 1.0)
+    tri[:, 4] = np.where(np.arange(n) % 3 == 0, np.float32(-0.0), np.float32(0.0))
+    tri[:, 1], tri[:, 7] = np.abs(tri[:, 1]), np.abs(tri[:, 7])
+    host, dev = re.KDTree(tri, max_depth=4), re.KDTree(tri, max_depth=4, ctx=gpu_ctx)
+    for k in ("root_min", "root_max"):
+        assert host.info[k].tobytes() == dev.info[k].tobytes(), k
+    for at, bad in ((0, np.nan), (n - 1, np.inf), (n // 2, -np.inf)):
+        worse = tri.copy()
+        worse[at, 5] = bad
+        with pytest.raises(re.ReError):
+            re.KDTree(worse, ctx=gpu_ctx)
