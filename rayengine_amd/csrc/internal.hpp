@@ -167,16 +167,7 @@ struct DevVolume {
   float box_min[3] = {0, 0, 0};
   float box_max[3] = {0, 0, 0};
   int64_t bytes = 0;
-  VolView view() const {
-    VolView v;
-    v.data = data;
-    for (int a = 0; a < 3; ++a) {
-      v.dim[a] = dim[a];
-      v.bdim[a] = bdim[a];
-      v.spacing[a] = spacing[a];
-    }
-    return v;
-  }
+  VolView view() const { return make_view(data, dim, bdim, spacing); }
 };
 
 struct NoiseLaunch {
