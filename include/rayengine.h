@@ -361,8 +361,8 @@ typedef struct re_noise_params {
 } re_noise_params;
 
 RE_API void re_noise_default_params(re_noise_params* p);
-/* Generates a volume on the device (bricked 8^3, Morton order inside a
- * brick).  Replaces generate_noise / cuda_update_chunk_gen
+/* Generates a volume on the device (blocks of 4^3 voxels, padded to
+ * multiples of 8).  Replaces generate_noise / cuda_update_chunk_gen
  * (RayEngine/src/cuda-src/renderer.cu:105-126,812-836,982-1005). */
 RE_API re_status re_noise_generate(re_ctx* ctx, const re_noise_params* params, int32_t* vol_id);
 /* Uploads a linear x-fastest grid (index x + dim.x*(y + dim.y*z)).

@@ -31,7 +31,7 @@ re_status alloc_volume(re_ctx* ctx, const int32_t* dim, const float* spacing, De
   return RE_OK;
 }
 
-// Linear x-fastest <-> bricked (Morton inside 8^3 bricks) copies.
+// Linear x-fastest <-> blocked (vox_index) copies.
 void to_bricked(const DevVolume& v, const float* linear, std::vector<float>& bricked) {
   bricked.assign((size_t)(v.bytes / 4), 0.0f);
   for (int z = 0; z < v.dim[2]; ++z)

@@ -530,6 +530,7 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
 // Reference sphere-trace march (single_ray_sphere_trace,
 // RayEngine/src/cuda-src/sphere_tracing.cuh:182-216) clipped to the volume
 // box: sample, step, then test d <= eps * t on the stepped t.
+template <bool NARROW>
 __device__ __forceinline__ bool plain_march(const VolView& V, const float* bmin, const float* bmax, f3 o, f3 d,
                                             int32_t max_steps, float eps, float step_scale, int32_t step_rule,
                                             float& t_out, int32_t& steps) {
@@ -540,7 +541,7 @@ __device__ __forceinline__ bool plain_march(const VolView& V, const float* bmin,
   float t = t_near;
   while (t < t_far && steps < max_steps) {
     const f3 p = add(o, smul(t, d));
-    const float dist = trilinear(V, p);
+    const float dist = trilinear<NARROW>(V, p);
     const float k = step_rule == 0 ? step_scale : fmaxf(0.45f, fminf(t * 0.6f, 0.8f));
     t += dist * k;
     ++steps;
@@ -555,6 +556,7 @@ __device__ __forceinline__ bool plain_march(const VolView& V, const float* bmin,
 // Exact-field march: from the volume entry, step max(f * k_exact, h_min)
 // while the trilinear field stays positive; bisect the first sign change
 // n_bisect times.  A ray entering at f <= 0 hits at the entry.
+template <bool NARROW>
 __device__ __forceinline__ bool exact_march(const VolView& V, const float* bmin, const float* bmax, f3 o, f3 d,
                                             float k_exact, float h_min, int32_t n_bisect, int32_t max_iters,
                                             float& t_out, int32_t& samples) {
@@ -563,7 +565,7 @@ __device__ __forceinline__ bool exact_march(const VolView& V, const float* bmin,
   t_out = kInf;
   if (!ray_box(bmin, bmax, o, d, tn, tf)) return false;
   float t = tn;
-  float f_prev = trilinear(V, add(o, smul(t, d)));
+  float f_prev = trilinear<NARROW>(V, add(o, smul(t, d)));
   ++samples;
   if (f_prev <= 0.0f) {
     t_out = t;
@@ -572,13 +574,13 @@ __device__ __forceinline__ bool exact_march(const VolView& V, const float* bmin,
   for (int it = 0; it < max_iters; ++it) {
     const float h = fmaxf(f_prev * k_exact, h_min);
     const float t_next = t + h;
-    const float f_next = trilinear(V, add(o, smul(t_next, d)));
+    const float f_next = trilinear<NARROW>(V, add(o, smul(t_next, d)));
     ++samples;
     if (f_next <= 0.0f) {
       float a = t, b = t_next;
       for (int k = 0; k < n_bisect; ++k) {
         const float mid = 0.5f * (a + b);
-        const float fm = trilinear(V, add(o, smul(mid, d)));
+        const float fm = trilinear<NARROW>(V, add(o, smul(mid, d)));
         ++samples;
         if (fm > 0.0f) a = mid; else b = mid;
       }

@@ -157,7 +157,7 @@ struct ScratchArea {
 
 hipError_t launch_trace_occluded(const TraceLaunch& L, hipStream_t s);
 
-// A volume resident in HBM: 8x8x8 Morton-ordered bricks.
+// A volume resident in HBM, in 4x4x4 blocks (vox_index).
 struct DevVolume {
   float* data = nullptr;
   float* mat = nullptr;  // material channel, same layout as data; null until loaded or edited

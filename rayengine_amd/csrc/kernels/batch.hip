@@ -62,6 +62,17 @@ __device__ __forceinline__ int32_t wave_fetch_sub(int32_t* p, int32_t sub, int l
   return __builtin_amdgcn_readfirstlane(v);
 }
 
+template <bool NARROW>
+__device__ __forceinline__ void tile_march(const BatchLaunch& L, const BatchTile& tile, int32_t kind, f3 o, f3 d,
+                                           bool& h, float& t, int32_t& n) {
+  if (kind == kItemExact)
+    h = exact_march<NARROW>(tile.vol, tile.box_min, tile.box_max, o, d, tile.hp.k_exact, tile.hp.h_min,
+                            tile.hp.n_bisect, tile.hp.max_iters, t, n);
+  else
+    h = plain_march<NARROW>(tile.vol, tile.box_min, tile.box_max, o, d, L.sdf.max_steps, L.sdf.eps, L.sdf.step_scale,
+                            L.sdf.step_rule, t, n);
+}
+
 template <bool ONE_SIDED>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) batch_kernel(BatchLaunch L) {
   // one CoopWave per wave of the block (dynamic LDS sized by the launch)
@@ -102,12 +113,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) b
         float t;
         int32_t n;
         bool h;
-        if (item.kind == kItemExact)
-          h = exact_march(tile.vol, tile.box_min, tile.box_max, o, d, tile.hp.k_exact, tile.hp.h_min,
-                          tile.hp.n_bisect, tile.hp.max_iters, t, n);
-        else
-          h = plain_march(tile.vol, tile.box_min, tile.box_max, o, d, L.sdf.max_steps, L.sdf.eps, L.sdf.step_scale,
-                          L.sdf.step_rule, t, n);
+        if (tile.vol.narrow) tile_march<true>(L, tile, item.kind, o, d, h, t, n);
+        else tile_march<false>(L, tile, item.kind, o, d, h, t, n);
         L.prim[i] = h ? 0 : -1;
         L.t[i] = h ? t : kInf;
       }

@@ -618,6 +618,7 @@ __global__ void edt_finish_kernel(VolView V, const float* __restrict__ g, float*
 // 2^k training points: even indices uniform in the volume, odd indices near
 // the surface (|signed distance| < near_band, by bounded rejection).  Each
 // sample is (x, y, z, signed distance).
+template <bool NARROW>
 __global__ void sample_kernel(VolView edt, float lo, float hi, int64_t n, uint64_t seed, float near_band,
                               int32_t max_tries, float4* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -628,7 +629,7 @@ __global__ void sample_kernel(VolView edt, float lo, float hi, int64_t n, uint64
   const bool near = (i & 1) != 0;
   for (int t = 0; t < (near ? max_tries : 1); ++t) {
     p = f3{lo + (hi - lo) * rng.uniform(), lo + (hi - lo) * rng.uniform(), lo + (hi - lo) * rng.uniform()};
-    d = trilinear(edt, p);
+    d = trilinear<NARROW>(edt, p);
     if (!near || fabsf(d) < near_band) break;
   }
   out[i] = float4{p.x, p.y, p.z, d};
@@ -684,7 +685,7 @@ __device__ __forceinline__ float wave_surrogate(const bf16x8* spack, const float
 // travel without a crossing, return to the surrogate.
 constexpr int kDeferTile = 16;
 
-template <bool USE_MLP>
+template <bool USE_MLP, bool NARROW>
 __global__ void __launch_bounds__(512) hybrid_trace_kernel(
     VolView V, float bx1, float by1, float bz1, const bf16x8* __restrict__ gpack, const float* __restrict__ gsmall,
     const float* __restrict__ ray_o, const float* __restrict__ ray_d, int64_t n, HybridParams hp,
@@ -704,7 +705,7 @@ __global__ void __launch_bounds__(512) hybrid_trace_kernel(
     if (i < n) {
       float t;
       int32_t samples;
-      const bool h = exact_march(V, bmin, bmax, o, d, hp.k_exact, hp.h_min, hp.n_bisect, hp.max_iters, t, samples);
+      const bool h = exact_march<NARROW>(V, bmin, bmax, o, d, hp.k_exact, hp.h_min, hp.n_bisect, hp.max_iters, t, samples);
       t_out[i] = t;
       hit_out[i] = h ? 1 : 0;
       if (evals_out) evals_out[i] = 0;
@@ -723,7 +724,7 @@ __global__ void __launch_bounds__(512) hybrid_trace_kernel(
     t_far = tf;
     phase = USE_MLP ? SURR : EXACT;
     if (!USE_MLP) {
-      f_prev = trilinear(V, add(o, smul(t, d)));
+      f_prev = trilinear<NARROW>(V, add(o, smul(t, d)));
       ++samples;
       if (f_prev <= 0.0f) { hit = true; phase = DONE; }
     }
@@ -762,7 +763,7 @@ __global__ void __launch_bounds__(512) hybrid_trace_kernel(
           } else {
             phase = EXACT;
             travel = 0.0f;
-            f_prev = trilinear(V, add(o, smul(t, d)));
+            f_prev = trilinear<NARROW>(V, add(o, smul(t, d)));
             ++samples;
             if (f_prev <= 0.0f) {
               hit = true;  // entered the surface region already inside: accept the current point
@@ -775,13 +776,13 @@ __global__ void __launch_bounds__(512) hybrid_trace_kernel(
     if (phase == EXACT) {
       const float h = fmaxf(f_prev * hp.k_exact, hp.h_min);
       const float t_next = t + h;
-      const float f_next = trilinear(V, add(o, smul(t_next, d)));
+      const float f_next = trilinear<NARROW>(V, add(o, smul(t_next, d)));
       ++samples;
       if (f_next <= 0.0f) {
         float a = t, b = t_next;
         for (int k = 0; k < hp.n_bisect; ++k) {
           const float mid = 0.5f * (a + b);
-          const float fm = trilinear(V, add(o, smul(mid, d)));
+          const float fm = trilinear<NARROW>(V, add(o, smul(mid, d)));
           ++samples;
           if (fm > 0.0f) a = mid; else b = mid;
         }
@@ -815,16 +816,17 @@ hipError_t launch_hybrid_trace(const DevVolume& field, const void* pack, const f
                                uint8_t* hit, int32_t* evals, int32_t* samples, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   const VolView V = field.view();
-  if (use_mlp)
-    hipLaunchKernelGGL(hybrid_trace_kernel<true>, dim3((unsigned)((n + kSurrBlock - 1) / kSurrBlock)),
-                       dim3(kSurrBlock), 0, s, V, field.box_max[0],
-                       field.box_max[1], field.box_max[2], (const bf16x8*)pack, small, ray_o, ray_d, n, hp, t, hit,
-                       evals, samples);
-  else
-    hipLaunchKernelGGL(hybrid_trace_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, V,
-                       field.box_max[0],
-                       field.box_max[1], field.box_max[2], (const bf16x8*)pack, small, ray_o, ray_d, n, hp, t, hit,
-                       evals, samples);
+  const int block = use_mlp ? kSurrBlock : 256;
+#define RE_LAUNCH(MLP, NARROW)                                                                                     \
+  hipLaunchKernelGGL((hybrid_trace_kernel<MLP, NARROW>), dim3((unsigned)((n + block - 1) / block)), dim3(block), 0, s, \
+                     V, field.box_max[0], field.box_max[1], field.box_max[2], (const bf16x8*)pack, small, ray_o,      \
+                     ray_d, n, hp, t, hit, evals, samples)
+  if (V.narrow) {
+    if (use_mlp) RE_LAUNCH(true, true); else RE_LAUNCH(false, true);
+  } else {
+    if (use_mlp) RE_LAUNCH(true, false); else RE_LAUNCH(false, false);
+  }
+#undef RE_LAUNCH
   return hipGetLastError();
 }
 
@@ -889,8 +891,11 @@ hipError_t launch_sample(const DevVolume& edt, int64_t n, uint64_t seed, float n
                          float4* out, hipStream_t s) {
   const VolView V = edt.view();
   const float hi = (float)(V.dim[0] - 1) * V.spacing[0];
-  hipLaunchKernelGGL(sample_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, V, 0.0f, hi, n, seed,
-                     near_band, max_tries, out);
+  const dim3 grid((unsigned)((n + 255) / 256));
+  if (V.narrow)
+    hipLaunchKernelGGL(sample_kernel<true>, grid, dim3(256), 0, s, V, 0.0f, hi, n, seed, near_band, max_tries, out);
+  else
+    hipLaunchKernelGGL(sample_kernel<false>, grid, dim3(256), 0, s, V, 0.0f, hi, n, seed, near_band, max_tries, out);
   return hipGetLastError();
 }
 

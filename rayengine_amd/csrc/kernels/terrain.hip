@@ -2,7 +2,7 @@
 //
 // noise_fill_kernel: one work-group per 8x8x8 brick (256 lanes, 2 voxels
 // each), the 512-entry permutation table staged in LDS, every lane writing
-// its voxel's field value at its Morton slot so a wave's stores are one
+// its voxel's field value at its block slot so a wave's stores are one
 // contiguous 256-byte run.  Replaces generate_noise
 // (RayEngine/src/cuda-src/renderer.cu:105-126), which used 8-thread blocks
 // and a linear float2 grid.
@@ -60,22 +60,24 @@ __global__ void __launch_bounds__(256) noise_fill_kernel(float* __restrict__ out
   for (int i = threadIdx.x; i < 512; i += blockDim.x) P[i] = (uint16_t)perm[i];
   __syncthreads();
   const int64_t brick = blockIdx.x;
+  const int32_t bdim[3] = {bx, by, 0};  // (vox_index needs no z count)
   const int gx = (int)(brick % bx), gy = (int)((brick / bx) % by), gz = (int)(brick / ((int64_t)bx * by));
   LdsTable T{P};
   for (int m = threadIdx.x; m < kBrickVox; m += blockDim.x) {
-    const int x = gx * kBrick + (int)compact3((uint32_t)m);
-    const int y = gy * kBrick + (int)compact3((uint32_t)m >> 1);
-    const int z = gz * kBrick + (int)compact3((uint32_t)m >> 2);
+    int qx, qy, qz, lx, ly, lz;
+    brick_block((uint32_t)m >> 6, qx, qy, qz);
+    block_voxel((uint32_t)m & 63u, lx, ly, lz);
+    const int x = gx * kBrick + qx * kBlock + lx, y = gy * kBrick + qy * kBlock + ly, z = gz * kBrick + qz * kBlock + lz;
     float v = 0.0f;
     if (x < dx && y < dy && z < dz) {
       const f3 p{ox + (float)x * sx, oy + (float)y * sy, oz + (float)z * sz};
       v = fbm_field(fp, p, [&](f3 q) { return noise_eval_wave(T, q); });
     }
-    out[brick * kBrickVox + m] = v;
+    out[vox_index(bdim, x, y, z)] = v;
   }
 }
 
-template <bool NORMALS>
+template <bool NORMALS, bool NARROW>
 __global__ void __launch_bounds__(256) sdf_trace_kernel(VolView V, float bx0, float by0, float bz0, float bx1,
                                                         float by1, float bz1, const float* __restrict__ ray_o,
                                                         const float* __restrict__ ray_d, int64_t n, int32_t max_steps,
@@ -89,7 +91,7 @@ __global__ void __launch_bounds__(256) sdf_trace_kernel(VolView V, float bx0, fl
   const float bmin[3] = {bx0, by0, bz0}, bmax[3] = {bx1, by1, bz1};
   int32_t steps = 0;
   float t = kInf;
-  const bool hit = plain_march(V, bmin, bmax, o, d, max_steps, eps, step_scale, step_rule, t, steps);
+  const bool hit = plain_march<NARROW>(V, bmin, bmax, o, d, max_steps, eps, step_scale, step_rule, t, steps);
   t_out[i] = hit ? t : kInf;
   hit_out[i] = hit ? 1 : 0;
   if (steps_out) steps_out[i] = steps;
@@ -98,10 +100,10 @@ __global__ void __launch_bounds__(256) sdf_trace_kernel(VolView V, float bx0, fl
     if (hit) {
       const float delta = fminf((float)(0.001 * (double)t), 0.002f);
       const f3 p = add(o, smul(t, d));
-      const float c = trilinear(V, p);
-      nrm = normalize(f3{trilinear(V, add(p, f3{delta, 0.0f, 0.0f})) - c,
-                         trilinear(V, add(p, f3{0.0f, delta, 0.0f})) - c,
-                         trilinear(V, add(p, f3{0.0f, 0.0f, delta})) - c});
+      const float c = trilinear<NARROW>(V, p);
+      nrm = normalize(f3{trilinear<NARROW>(V, add(p, f3{delta, 0.0f, 0.0f})) - c,
+                         trilinear<NARROW>(V, add(p, f3{0.0f, delta, 0.0f})) - c,
+                         trilinear<NARROW>(V, add(p, f3{0.0f, 0.0f, delta})) - c});
     }
     nrm_out[3 * i] = nrm.x;
     nrm_out[3 * i + 1] = nrm.y;
@@ -134,11 +136,12 @@ __global__ void __launch_bounds__(256) volume_edit_kernel(EditLaunch L) {
   const int gx = (int)(brick % L.bdim[0]), gy = (int)((brick / L.bdim[0]) % L.bdim[1]);
   const int gz = (int)(brick / ((int64_t)L.bdim[0] * L.bdim[1]));
   for (int m = threadIdx.x; m < kBrickVox; m += blockDim.x) {
-    const int x = gx * kBrick + (int)compact3((uint32_t)m);
-    const int y = gy * kBrick + (int)compact3((uint32_t)m >> 1);
-    const int z = gz * kBrick + (int)compact3((uint32_t)m >> 2);
+    int qx, qy, qz, lx, ly, lz;
+    brick_block((uint32_t)m >> 6, qx, qy, qz);
+    block_voxel((uint32_t)m & 63u, lx, ly, lz);
+    const int x = gx * kBrick + qx * kBlock + lx, y = gy * kBrick + qy * kBlock + ly, z = gz * kBrick + qz * kBlock + lz;
     if (x >= L.dim[0] || y >= L.dim[1] || z >= L.dim[2]) continue;
-    const int64_t i = brick * kBrickVox + m;
+    const int64_t i = vox_index(L.bdim, x, y, z);
     float px = (float)x * L.spacing[0] - L.center[0];
     const float py = (float)y * L.spacing[1] - L.center[1];
     float pz = (float)z * L.spacing[2] - L.center[2];
@@ -198,11 +201,15 @@ hipError_t launch_sdf_trace(const SdfLaunch& L, hipStream_t s) {
   if (L.n <= 0) return hipSuccess;
   const int block = L.block > 0 ? L.block : 256;
   const int64_t grid = (L.n + block - 1) / block;
-#define RE_LAUNCH(NRM)                                                                                        \
-  hipLaunchKernelGGL((sdf_trace_kernel<NRM>), dim3((unsigned)grid), dim3(block), 0, s, L.vol, L.box_min[0],  \
+#define RE_LAUNCH(NRM, NARROW)                                                                                \
+  hipLaunchKernelGGL((sdf_trace_kernel<NRM, NARROW>), dim3((unsigned)grid), dim3(block), 0, s, L.vol, L.box_min[0],  \
                      L.box_min[1], L.box_min[2], L.box_max[0], L.box_max[1], L.box_max[2], L.ray_o, L.ray_d, \
                      L.n, L.max_steps, L.eps, L.step_scale, L.step_rule, L.t, L.hit, L.steps, L.nrm)
-  if (L.nrm) RE_LAUNCH(true); else RE_LAUNCH(false);
+  if (L.vol.narrow) {
+    if (L.nrm) RE_LAUNCH(true, true); else RE_LAUNCH(false, true);
+  } else {
+    if (L.nrm) RE_LAUNCH(true, false); else RE_LAUNCH(false, false);
+  }
 #undef RE_LAUNCH
   return hipGetLastError();
 }

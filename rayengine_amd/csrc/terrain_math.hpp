@@ -13,14 +13,29 @@
 
 namespace re {
 
-// Brick of 8x8x8 voxels, Morton-ordered inside: one 128-byte cache line holds
-// a 4x4x2 block, so the 8 corners of a trilinear cell usually share 1-2 lines
-// and a ray marching through a brick stays in 2 KB.
+// Volumes are stored in blocks of 4x4x4 voxels, x fastest inside a block and
+// blocks x fastest: one 128-byte cache line holds a 4x4x2 block, so the 8
+// corners of a trilinear cell usually share 1-2 lines, and a voxel's address
+// is a sum of one short expression per axis.  (Morton order inside 8x8x8
+// bricks shares its lines alike but takes twice the instructions to address.)
+// The padded dimensions are multiples of kBrick, the unit of the kernels that
+// go over whole volumes.
+constexpr int kBlock = 4;
+constexpr int kBlockVox = kBlock * kBlock * kBlock;
 constexpr int kBrick = 8;
 constexpr int kBrickVox = kBrick * kBrick * kBrick;
 
-RE_HD uint32_t spread3(uint32_t v) { return (v & 1u) | ((v & 2u) << 2) | ((v & 4u) << 4); }
-RE_HD uint32_t compact3(uint32_t m) { return (m & 1u) | ((m >> 2) & 2u) | ((m >> 4) & 4u); }
+// Voxel l (0..63) of a block, and block b (0..7) of a brick: x, y, z.
+RE_HD void block_voxel(uint32_t l, int& x, int& y, int& z) {
+  x = (int)(l & 3u);
+  y = (int)((l >> 2) & 3u);
+  z = (int)(l >> 4);
+}
+RE_HD void brick_block(uint32_t b, int& x, int& y, int& z) {
+  x = (int)(b & 1u);
+  y = (int)((b >> 1) & 1u);
+  z = (int)(b >> 2);
+}
 
 struct VolView {
   const float* data;
@@ -30,7 +45,7 @@ struct VolView {
   // Set by make_view, for trilinear's grid coordinates and addresses.
   float inv[3];      // 1 / spacing, correctly rounded
   int32_t by_inv;    // 2: spacings are powers of two, p * inv is p / spacing; 1: quotients by div_by; 0: divide
-  int32_t narrow;    // voxel offsets fit 30 bits and their brick strides 24: 32-bit addresses
+  int32_t narrow;    // voxel offsets fit 30 bits and the block strides 24: 32-bit addresses
 };
 
 inline VolView make_view(const float* data, const int32_t* dim, const int32_t* bdim, const float* spacing) {
@@ -48,15 +63,14 @@ inline VolView make_view(const float* data, const int32_t* dim, const int32_t* b
     if (!(spacing[a] > 0.0f) || e < -40 || e > 40) v.by_inv = 0;
     else if (m != 0.5f && v.by_inv == 2) v.by_inv = 1;
   }
-  const int64_t slab = (int64_t)bdim[0] * bdim[1] * kBrickVox;
-  v.narrow = slab < (1 << 24) && slab * bdim[2] <= (1 << 30);
+  const int64_t slab = (int64_t)bdim[0] * bdim[1] * (kBrickVox / 2);  // one layer of blocks
+  v.narrow = slab < (1 << 24) && 2 * slab * bdim[2] <= (1 << 30);
   return v;
 }
 
 RE_HD int64_t vox_index(const int32_t* bdim, int x, int y, int z) {
-  int64_t b = ((int64_t)(z >> 3) * bdim[1] + (y >> 3)) * bdim[0] + (x >> 3);
-  uint32_t m = spread3((uint32_t)x & 7u) | (spread3((uint32_t)y & 7u) << 1) | (spread3((uint32_t)z & 7u) << 2);
-  return b * kBrickVox + m;
+  const int64_t b = ((int64_t)(z >> 2) * (2 * bdim[1]) + (y >> 2)) * (2 * bdim[0]) + (x >> 2);
+  return b * kBlockVox + ((z & 3) << 4) + ((y & 3) << 2) + (x & 3);
 }
 
 // 16-case gradient dot product (sdf_functions.cuh:25-48) as s1*A + s2*B with
@@ -210,8 +224,8 @@ RE_HD f3 grid_coord(const VolView& V, f3 p) {
   return f3{p.x / V.spacing[0], p.y / V.spacing[1], p.z / V.spacing[2]};
 }
 
-// spread3 of a 3-bit value by or-ing shifted copies.
-RE_HD uint32_t spread3_or(uint32_t v) { return (v | (v << 2) | (v << 4)) & 0x49u; }
+RE_HD int imin(int a, int b) { return a < b ? a : b; }
+RE_HD int imax(int a, int b) { return a > b ? a : b; }
 
 #if defined(__HIP_DEVICE_COMPILE__)
 RE_HD uint32_t mul24(uint32_t a, uint32_t b) { return __umul24(a, b); }
@@ -237,32 +251,35 @@ struct TriCell {
 };
 
 // Loads the cell of world point p: grid coordinate c = p / spacing, cell
-// index clamped to [0, dim-2].  The marching kernels were bound by the
-// instructions of this routine as much as by its loads: 212 per sample with
-// IEEE divisions and eight 64-bit brick addresses.  A brick address is a sum
-// of one part per axis, so the cell needs two parts per axis (12 instead of
-// 24 index computations), and where the volume's size allows (narrow: up to
-// 4 GiB, which is every volume up to 1024^3) the parts are 32-bit offsets
-// from a scalar base.
+// index clamped to [0, dim-2].  The marching kernels are bound by the vector
+// instructions of this routine more than by its loads: 212 per sample with
+// IEEE divisions and eight 64-bit Morton brick addresses, about 80 now.  An
+// address is a sum of one part per axis, so a cell needs two parts per axis,
+// and with NARROW (V.narrow: up to 4 GiB, which is every volume up to 1024^3)
+// the parts are 32-bit offsets from a scalar base.  NARROW is a template
+// parameter because the compiler merges the loads of a run-time branch's two
+// sides into one set with 64-bit addresses.
+template <bool NARROW>
 RE_HD TriCell tri_load(const VolView& V, f3 p) {
   const f3 g = grid_coord(V, p);
   int ix = (int)g.x, iy = (int)g.y, iz = (int)g.z;
-  ix = ix < 0 ? 0 : (ix > V.dim[0] - 2 ? V.dim[0] - 2 : ix);
-  iy = iy < 0 ? 0 : (iy > V.dim[1] - 2 ? V.dim[1] - 2 : iy);
-  iz = iz < 0 ? 0 : (iz > V.dim[2] - 2 ? V.dim[2] - 2 : iz);
+  ix = imax(imin(ix, V.dim[0] - 2), 0);
+  iy = imax(imin(iy, V.dim[1] - 2), 0);
+  iz = imax(imin(iz, V.dim[2] - 2), 0);
   TriCell t;
   t.tx = g.x - (float)ix;
   t.ty = g.y - (float)iy;
   t.tz = g.z - (float)iz;
-  if (V.narrow) {
-    const uint32_t row = (uint32_t)V.bdim[0] * (uint32_t)kBrickVox, slab = row * (uint32_t)V.bdim[1];
+  if (NARROW) {
+    // (x >> 2) 64 + (x & 3) = x + 15 (x & ~3), and likewise 4 y + (y >> 2) (row - 16), 16 z + (z >> 2) (slab - 64)
+    const uint32_t row = (uint32_t)V.bdim[0] * (2 * kBlockVox), slab = row * 2u * (uint32_t)V.bdim[1];
     uint32_t X[2], Y[2], Z[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const uint32_t x = (uint32_t)(ix + k), y = (uint32_t)(iy + k), z = (uint32_t)(iz + k);
-      X[k] = ((x & ~7u) << 6) + spread3_or(x & 7u);
-      Y[k] = mul24(y >> 3, row) + (spread3_or(y & 7u) << 1);
-      Z[k] = mul24(z >> 3, slab) + (spread3_or(z & 7u) << 2);
+      X[k] = mul24(x & ~3u, 15u) + x;
+      Y[k] = mul24(y >> 2, row - 16u) + (y << 2);
+      Z[k] = mul24(z >> 2, slab - 64u) + (z << 4);
     }
     const char* const D = reinterpret_cast<const char*>(V.data);
 #pragma unroll
@@ -279,8 +296,9 @@ RE_HD TriCell tri_load(const VolView& V, f3 p) {
 
 // Trilinear sample at world point p, lerps in x then y then z
 // (interpolate / bilinear, RayEngine/src/cuda-src/sdf_functions.cuh:209-265).
+template <bool NARROW>
 RE_HD float trilinear(const VolView& V, f3 p) {
-  const TriCell t = tri_load(V, p);
+  const TriCell t = tri_load<NARROW>(V, p);
   return trilerp(t.c, t.tx, t.ty, t.tz);
 }
 
