@@ -199,7 +199,7 @@ hipError_t launch_noise_fill(const NoiseLaunch& L, hipStream_t s) {
 
 hipError_t launch_sdf_trace(const SdfLaunch& L, hipStream_t s) {
   if (L.n <= 0) return hipSuccess;
-  const int block = L.block > 0 ? L.block : 256;
+  const int block = L.block > 0 ? L.block : 64;  // one wave (with normals 74 us against 76 at 256, 2,073,600 rays)
   const int64_t grid = (L.n + block - 1) / block;
 #define RE_LAUNCH(NRM, NARROW)                                                                                \
   hipLaunchKernelGGL((sdf_trace_kernel<NRM, NARROW>), dim3((unsigned)grid), dim3(block), 0, s, L.vol, L.box_min[0],  \
