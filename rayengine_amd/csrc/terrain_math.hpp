@@ -97,6 +97,22 @@ RE_HD float grad_dot(uint32_t h, float x, float y, float z) {
   }
 }
 
+// grad_dot's two coefficients as three, one of them zero: s1 A + s2 B =
+// fma(gx, x, fma(gy, y, gz z)) to the bit for finite x, y, z (the products
+// with 0 and +-1 are exact, so one rounding is left; a zero sum may differ in
+// its sign, which the blend's later sums, all ending in 0 + amp * noise, do
+// not show).
+RE_HD f3 grad_coeffs(uint32_t h) {
+  h &= 15u;
+  const float s0 = (h & 1u) ? -1.0f : 1.0f, s1 = (h & 2u) ? -1.0f : 1.0f;
+  if (h < 4u) return f3{s0, s1, 0.0f};
+  if (h < 8u) return f3{s0, 0.0f, s1};
+  if (h < 12u) return f3{0.0f, s0, s1};
+  if (h == 12u) return f3{1.0f, 1.0f, 0.0f};
+  if (h == 13u) return f3{-1.0f, 1.0f, 0.0f};
+  return f3{0.0f, -1.0f, h == 14u ? 1.0f : -1.0f};
+}
+
 RE_HD float quintic(float t) { return t * t * t * (t * (t * 6 - 15) + 10); }
 
 // One octave of noise_eval split in two: the cell-relative coordinates and
@@ -122,15 +138,9 @@ RE_HD NoiseCell noise_cell(f3 p, int fx, int fy, int fz) {
   return c;
 }
 
-RE_HD float noise_blend(const uint32_t* h, const NoiseCell& c) {
-  float a = grad_dot(h[0], c.x0, c.y0, c.z0);
-  float b = grad_dot(h[1], c.x1, c.y0, c.z0);
-  float cc = grad_dot(h[2], c.x0, c.y1, c.z0);
-  float d = grad_dot(h[3], c.x1, c.y1, c.z0);
-  float e = grad_dot(h[4], c.x0, c.y0, c.z1);
-  float f = grad_dot(h[5], c.x1, c.y0, c.z1);
-  float g = grad_dot(h[6], c.x0, c.y1, c.z1);
-  float hh = grad_dot(h[7], c.x1, c.y1, c.z1);
+// The blend of the corner gradients a, b, cc, d (z0), e, f, g, hh (z1).
+RE_HD float noise_mix(float a, float b, float cc, float d, float e, float f, float g, float hh, float u, float v,
+                      float w) {
   float k0 = a;
   float k1 = (b - a);
   float k2 = (cc - a);
@@ -139,8 +149,14 @@ RE_HD float noise_blend(const uint32_t* h, const NoiseCell& c) {
   float k5 = (a + f - b - e);
   float k6 = (a + g - cc - e);
   float k7 = (b + cc + e + hh - a - d - f - g);
-  const float u = c.u, v = c.v, w = c.w;
   return k0 + k1 * u + k2 * v + k3 * w + k4 * u * v + k5 * u * w + k6 * v * w + k7 * u * v * w;
+}
+
+RE_HD float noise_blend(const uint32_t* h, const NoiseCell& c) {
+  return noise_mix(grad_dot(h[0], c.x0, c.y0, c.z0), grad_dot(h[1], c.x1, c.y0, c.z0),
+                   grad_dot(h[2], c.x0, c.y1, c.z0), grad_dot(h[3], c.x1, c.y1, c.z0),
+                   grad_dot(h[4], c.x0, c.y0, c.z1), grad_dot(h[5], c.x1, c.y0, c.z1),
+                   grad_dot(h[6], c.x0, c.y1, c.z1), grad_dot(h[7], c.x1, c.y1, c.z1), c.u, c.v, c.w);
 }
 
 // The corners' hashes of lattice cell (fx, fy, fz).
