@@ -51,7 +51,16 @@ __device__ bool ray_sphere(V3 o, V3 d, float radius, float& t0, float& t1) {
   return true;
 }
 
-__device__ V3 incident_light(const FrameLaunch& L, V3 orig, V3 dir) {
+// UP: the sun at (0, 1, 0), the default direction.  A light sample's x and z
+// are then its view sample's, so their squares leave the light loop (the
+// products with 0 and 1 are exact, so every sum keeps its bits): 28 of the
+// loop's 35 issue slots per sample remain, four of them per square root and
+// exponential.  The loop is bound by vector issue; a 1920x1080 frame with
+// 542,677 sky pixels takes 136 us against 154 in the general form.  (All
+// eight light samples unrolled without the branch: 144 us, though 640x360,
+// which is bound by latency, went from 36 to 31.)
+template <bool UP>
+__device__ __forceinline__ V3 incident_light(const FrameLaunch& L, V3 orig, V3 dir) {
   const V3 sun{L.sun[0], L.sun[1], L.sun[2]};
   const V3 betaR{3.8e-6f, 13.5e-6f, 33.1e-6f};
   const float betaM = 21e-6f;
@@ -84,10 +93,16 @@ __device__ V3 incident_light(const FrameLaunch& L, V3 orig, V3 dir) {
     const float seg_l = t1l / (float)num_samples_light;
     float t_cur_l = 0;
     float od_lr = 0, od_lm = 0;
+    const float sxx = sp.x * sp.x, szz = sp.z * sp.z;
     int j;
     for (j = 0; j < num_samples_light; ++j) {
-      const V3 spl = sp + (t_cur_l + seg_l * 0.5f) * sun;
-      const float hl = hlen(spl) - L.er;
+      float hl;
+      if (UP) {
+        const float y = sp.y + (t_cur_l + seg_l * 0.5f);
+        hl = hsqrt(sxx + y * y + szz) - L.er;
+      } else {
+        hl = hlen(sp + (t_cur_l + seg_l * 0.5f) * sun) - L.er;
+      }
       if (hl < 0) break;
       od_lr += hexp(-hl * inv_hr) * seg_l;
       od_lm += hexp(-hl * inv_hm) * seg_l;
@@ -111,6 +126,7 @@ __device__ __forceinline__ float sky_tone(float c) {
   return c < 1.413f ? powf(c * 0.38317f, 1.0f / 2.2f) : 1.0f - expf(-c);
 }
 
+template <bool UP>
 __global__ void __launch_bounds__(256) frame_kernel(FrameLaunch L) {
   const int64_t n = (int64_t)L.width * L.height;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -125,7 +141,7 @@ __global__ void __launch_bounds__(256) frame_kernel(FrameLaunch L) {
     const float f = fmaxf(0.f, dot(nrm, V3{-d.x, -d.y, -d.z}) / 2);
     c = {saturate(L.base[0] + 0.5f * f), saturate(L.base[1] + 0.5f * f), saturate(L.base[2] + 0.5f * f)};
   } else {
-    const V3 sky = incident_light(L, V3{L.origin[0], L.origin[1], L.origin[2]}, d);
+    const V3 sky = incident_light<UP>(L, V3{L.origin[0], L.origin[1], L.origin[2]}, d);
     c = {sky_tone(sky.x), sky_tone(sky.y), sky_tone(sky.z)};
   }
   if (L.gamma) c = {powf(c.x, 1.0f / 2.2f), powf(c.y, 1.0f / 2.2f), powf(c.z, 1.0f / 2.2f)};
@@ -142,7 +158,13 @@ __global__ void __launch_bounds__(256) frame_kernel(FrameLaunch L) {
 hipError_t launch_frame(const FrameLaunch& L, hipStream_t s) {
   const int64_t n = (int64_t)L.width * L.height;
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(frame_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, L);
+  // far from overflow, where 0 * t would not be 0
+  const bool up = L.sun[0] == 0.0f && L.sun[1] == 1.0f && L.sun[2] == 0.0f && L.ar < 1e15f && L.ar > -1e15f;
+  bool near = true;
+  for (float o : L.origin) near = near && o < 1e15f && o > -1e15f;
+  const dim3 grid((unsigned)((n + 255) / 256));
+  if (up && near) hipLaunchKernelGGL(frame_kernel<true>, grid, dim3(256), 0, s, L);
+  else hipLaunchKernelGGL(frame_kernel<false>, grid, dim3(256), 0, s, L);
   return hipGetLastError();
 }
 
