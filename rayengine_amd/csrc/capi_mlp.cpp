@@ -192,10 +192,11 @@ RE_API re_status re_mlp_batch_step(re_ctx* ctx, int32_t mlp_id, const float* sam
   st = ensure_stage(ctx, stage_size({(size_t)n * 16}));
   if (st) return st;
   HIP_TRY(ctx, hipMemcpyAsync(ctx->stage, samples, (size_t)n * 16, hipMemcpyHostToDevice, ctx->stream), "copy samples");
+  const int32_t blocks = mlp_train_grid(m->partial_blocks, n);
   HIP_TRY(ctx, launch_mlp_train(m->pack, m->small, (const float4*)ctx->stage, n, 0, (int32_t)n, over_weight,
-                                m->partial, m->partial_blocks, ctx->stream), "mlp train");
+                                m->partial, blocks, ctx->stream), "mlp train");
   if (adam) ++m->step;
-  HIP_TRY(ctx, launch_mlp_update(m->params, m->m1, m->m2, m->partial, m->partial_blocks, m->step, lr, 0.9f, 0.999f,
+  HIP_TRY(ctx, launch_mlp_update(m->params, m->m1, m->m2, m->partial, blocks, m->step, lr, 0.9f, 0.999f,
                                  1e-8f, adam ? 1 : 0, m->grad, m->pack, m->small, m->loss, ctx->stream), "mlp update");
   if (grad) HIP_TRY(ctx, hipMemcpyAsync(grad, m->grad, (size_t)kParams * 4, hipMemcpyDeviceToHost, ctx->stream), "copy grad");
   if (loss) HIP_TRY(ctx, hipMemcpyAsync(loss, m->loss, 4, hipMemcpyDeviceToHost, ctx->stream), "copy loss");
@@ -380,16 +381,17 @@ RE_API re_status re_mlp_train(re_ctx* ctx, int32_t mlp_id, int32_t dist_vol_id, 
     m->cursor = 0;
   }
   const int64_t first = m->cursor;
+  const int32_t blocks = mlp_train_grid(m->partial_blocks, p.batch);
   float4* samples = nullptr;
   HIP_TRY(ctx, hipMalloc((void**)&samples, (size_t)p.n_samples * 16), "sample pool");
   hipError_t e = launch_sample(dv, p.n_samples, p.seed, p.near_band_voxels * dv.spacing[0], 256, samples, ctx->stream);
   for (int32_t s = 0; e == hipSuccess && s < p.steps; ++s) {
     const int64_t start = (int64_t)(((unsigned __int128)(first + s) * (uint64_t)p.batch) % (uint64_t)p.n_samples);
     e = launch_mlp_train(m->pack, m->small, samples, p.n_samples, start, p.batch, p.over_weight, m->partial,
-                         m->partial_blocks, ctx->stream);
+                         blocks, ctx->stream);
     if (e == hipSuccess) {
       ++m->step;
-      e = launch_mlp_update(m->params, m->m1, m->m2, m->partial, m->partial_blocks, m->step, p.lr, p.beta1, p.beta2,
+      e = launch_mlp_update(m->params, m->m1, m->m2, m->partial, blocks, m->step, p.lr, p.beta1, p.beta2,
                             p.eps, 1, nullptr, m->pack, m->small, m->loss + s, ctx->stream);
     }
   }

@@ -253,6 +253,12 @@ struct DevMlp {
 };
 
 size_t mlp_train_lds_bytes();
+// Blocks of a training launch over `batch` points, of at most `most`: none
+// without a 64-point chunk (their partial gradients would be written, and read
+// again by the update, as zeros).
+inline int32_t mlp_train_grid(int32_t most, int64_t batch) {
+  return batch / 64 < most ? (int32_t)(batch / 64) : most;
+}
 
 // The inference operands (mlp_layout.hpp: pre-activations carried as
 // -log2(e) z) stored after the training ones in the same buffers.

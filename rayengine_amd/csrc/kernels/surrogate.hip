@@ -36,16 +36,12 @@ __device__ __forceinline__ float cos_rev(float x) { return __builtin_amdgcn_cosf
 __device__ __forceinline__ float sigmoid_fast(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504089f));
 }
-__device__ __forceinline__ float silu(float z) { return z * sigmoid_fast(z); }
 // The same unit on the scaled pre-activation u = -log2(e) z of the inference
 // operands: u / (1 + 2^u) = -log2(e) SiLU(z).
 __device__ __forceinline__ float silu_scaled(float u) { return u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(u)); }
 
-// Its derivative: s (1 + z (1 - s)) with s = sigmoid(z).
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = sigmoid_fast(z);
-  return s * (1.0f + z * (1.0f - s));
-}
+// Its derivative s (1 + z (1 - s)) from z and s = sigmoid(z).
+__device__ __forceinline__ float dsilu(float z, float s) { return s * (1.0f + z * (1.0f - s)); }
 
 // Device PCG32 (same generator as the host scene generators).
 struct DevPcg {
@@ -98,10 +94,19 @@ __device__ __forceinline__ void features(f3 p, int g, bf16x8 xb[4]) {
 // ----------------------------------------------------------------- forward
 
 struct TileAct {
-  f32x4 z[4][4];    // pre-activations [layer][M-tile], lane holds neurons 16m+4g+r
+  f32x4 ds[4][4];   // dSiLU/dz [layer][M-tile], lane holds neurons 16m+4g+r (KEEP): kept instead of z, so that
+                    // the backward pass takes no exponential and reciprocal of its own
   bf16x8 hb[4][2];  // bf16 B operands of h0..h3 (hb[3] feeds nothing but the staging)
   float h3[4][4];   // FP32 h3 for the output layer
 };
+
+template <bool KEEP, bool SCALED>
+__device__ __forceinline__ float activate(float z, f32x4& ds, int r) {
+  if (SCALED) return silu_scaled(z);
+  const float s = sigmoid_fast(z);
+  if (KEEP) ds[r] = dsilu(z, s);
+  return z * s;
+}
 
 // SCALED: the inference operands (pre-activations carried as -log2(e) z).
 template <bool KEEP, bool SCALED = false>
@@ -123,8 +128,7 @@ __device__ __forceinline__ float forward_tile(const bf16x8* __restrict__ packF, 
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float z = acc[m][r];
-        if (KEEP) T.z[0][m][r] = z;
-        T.hb[0][m >> 1][(m & 1) * 4 + r] = (__bf16)(SCALED ? silu_scaled(z) : silu(z));
+        T.hb[0][m >> 1][(m & 1) * 4 + r] = (__bf16)activate<KEEP, SCALED>(z, T.ds[0][m], r);
       }
   }
   // layers 1..3: 2 K-steps of 32 neurons, chained in registers
@@ -145,8 +149,7 @@ __device__ __forceinline__ float forward_tile(const bf16x8* __restrict__ packF, 
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float z = acc[m][r];
-        if (KEEP) T.z[L][m][r] = z;
-        const float h = SCALED ? silu_scaled(z) : silu(z);
+        const float h = activate<KEEP, SCALED>(z, T.ds[L][m], r);
         T.hb[L][m >> 1][(m & 1) * 4 + r] = (__bf16)h;
         if (L == 3) T.h3[m][r] = h;
       }
@@ -199,32 +202,47 @@ __global__ void __launch_bounds__(512) mlp_infer_kernel(const bf16x8* __restrict
 
 // ----------------------------------------------------------------- training
 
-// Per 64-point chunk (16 per wave) every wave runs forward and backward on its
-// tile and stages, transposed as [neuron][point] in LDS, the bf16 dZ of every
-// layer and the input activations of layers 0..3.  Wave w then accumulates the
-// weight gradient of layer w over the chunk's 64 points with K = points, and
-// its bias gradient as the product with a column of ones.  The output layer's
-// gradient is summed in registers, per lane over its own points, and reduced
-// over lanes and waves once at the end.
+// A block's eight waves take two 64-point chunks at a time, waves 0-3 the first
+// and waves 4-7 the second, 16 points each.  Every wave runs forward and
+// backward on its tile; the weight gradients are products over the points, so
+// layer by layer the waves stage the bf16 dZ of the layer and its input
+// activations, transposed as [neuron][point], in LDS, and after a barrier each
+// wave accumulates its own two of the layer's 16 result tiles (three or four of
+// layer 0's 28) with K = points, and the bias gradients of two of the layers as
+// the product with a column of ones.  The output layer's gradient is summed in
+// registers, per lane over its own points, and reduced over lanes and waves
+// once at the end.  Staging one layer at a time (two buffers, one barrier per
+// layer) is what leaves the LDS room for eight waves beside the 64 KB of
+// operands; with four waves and every layer staged at once a SIMD ran one wave
+// and stood still through its chains of LDS reads, MFMAs and exponentials:
+// 38.5 us per launch of 65,536 points, now 31.9.
+//
+// Additions keep the order of one chunk after the other: K runs over the first
+// chunk's points, then the second's, and the output layer's per-lane sums of
+// both chunks are kept by one half (neurons m = 0, 1 by the first, 2, 3 by the
+// second), which the other hands its products through LDS (exchange).
 constexpr int kChunkPts = 64;
-// Staged rows are padded by 16 bytes (72 bf16): the 16 rows of one MFMA operand
+constexpr int kPairPts = 2 * kChunkPts;
+// Staged rows are padded by 16 bytes (136 bf16): the 16 rows of one MFMA operand
 // read then cover all 64 LDS banks once, and the four neuron groups of a
 // staging write fall in different banks.
-constexpr int kRow = kChunkPts + 8;
+constexpr int kRow = kPairPts + 8;
 // Layer-0 inputs staged: the 99 used, padded to 7 column tiles of 16.
 constexpr int kInStage = 112;
-constexpr int kTrainBlock = 256;
+constexpr int kTrainBlock = 512;
+constexpr int kHalfThreads = kTrainBlock / 2;
+constexpr int kExchange = 18;  // per lane of a half: 8 + 8 products of the output layer, dout, loss
 
 struct TrainLds {
   bf16x8 pack[kPack >> 3];            // 64 KB: forward and backward operands
   float small[kSmall + 3];
-  __bf16 dzT[4][kH][kRow];            // 36 KB
-  __bf16 xT[kInStage][kRow];          // 15.75 KB
-  __bf16 hT[3][kH][kRow];             // 27 KB (h0..h2, the inputs of layers 1..3)
+  __bf16 dz1[kH][kRow], in1[kH][kRow];        // staging of layers 3 and 1
+  __bf16 dz0[kH][kRow], in0[kInStage][kRow];  // staging of layers 2 and 0
+  unsigned char tail[kExchange * kHalfThreads * 4 - (kInStage - kH) * kRow * 2];  // the exchange's end
 };
 static_assert(sizeof(TrainLds) <= 160 * 1024, "one training block must fit the LDS of a CU");
-static_assert(sizeof(__bf16) * 4 * kH * kRow >= sizeof(float) * (4 * kH + 8),
-              "the final reduction reuses the dZ staging area");
+static_assert(sizeof(__bf16) * kH * kRow >= sizeof(float) * (4 * kH + 8),
+              "the final reduction reuses a staging buffer");
 static_assert((kPack >> 3) % kTrainBlock == 0, "the operand pack is copied in whole rounds");
 
 __device__ __forceinline__ int64_t train_sample_index(int64_t batch_start, int ch, int p_local, int64_t n_samples) {
@@ -239,17 +257,25 @@ __global__ void __launch_bounds__(kTrainBlock) mlp_train_kernel(const bf16x8* __
   extern __shared__ __align__(16) unsigned char lds_raw[];
   TrainLds& S = *reinterpret_cast<TrainLds*>(lds_raw);
   const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int half = wv >> 2;           // which chunk of the pair
   const int g = lane >> 4, j = lane & 15;
-  const int p_local = 16 * w + j;
+  const int p_local = 16 * (wv & 3) + j;
+  const int p_row = kChunkPts * half + p_local;
+  const int mi = wv >> 1, odd = wv & 1;  // result tiles: rows 16 mi, and the even or odd wave's columns
   const float inv_b = 1.0f / (float)batch;
   const int n_chunks = batch / kChunkPts;
+  // Rows of lane values; they overlap rows of in0 that only layer 0 stages, two
+  // barriers after they are read.
+  float* const exchange = reinterpret_cast<float*>(&S.in0[kH][0]);
+  const int xl = threadIdx.x & (kHalfThreads - 1);
 
   // The first chunk's sample is requested before the operand copy, and the
   // copy issues all of a thread's loads before its first LDS store.
   float4 smp_next = make_float4(0.f, 0.f, 0.f, 0.f);
-  if ((int)blockIdx.x < n_chunks) smp_next = samples[train_sample_index(batch_start, blockIdx.x, p_local, n_samples)];
   {
+    const int c0 = (int)blockIdx.x + half * (int)gridDim.x;
+    if (c0 < n_chunks) smp_next = samples[train_sample_index(batch_start, c0, p_local, n_samples)];
     constexpr int kPer = (kPack >> 3) / kTrainBlock;
     bf16x8 r[kPer];
 #pragma unroll
@@ -260,155 +286,202 @@ __global__ void __launch_bounds__(kTrainBlock) mlp_train_kernel(const bf16x8* __
   }
   __syncthreads();
 
-  f32x4 acc[4][7], accb[4];
+  // [layer][tile], layers 1-3 use two tiles; biases of layers 0 and 1 (even
+  // waves) or 2 and 3 (odd waves)
+  f32x4 acc[4][4], accb[2];
 #pragma unroll
   for (int a = 0; a < 4; ++a) {
-    accb[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (a < 2) accb[a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int b = 0; b < 7; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // B operand of the bias product: column 0 all ones, the other columns zero
   bf16x8 ones;
 #pragma unroll
   for (int s = 0; s < 8; ++s) ones[s] = (__bf16)(j == 0 ? 1.0f : 0.0f);
-  // per lane, over its points: dout * h3 for neurons 16 m + 4 g + r (index
-  // 4 m + r), and dout (g == 0 lanes)
-  float dw4r[16];
+  // per lane, over its points and those of the other half's same lane: dout * h3
+  // for neurons 16 m + 4 g + r, m = 2 half, 2 half + 1; dout and the loss (first
+  // half, g == 0 lanes)
+  float dw4r[8];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) dw4r[q] = 0.0f;
+  for (int q = 0; q < 8; ++q) dw4r[q] = 0.0f;
   float db4r = 0.0f, loss = 0.0f;
 
-  for (int ch = blockIdx.x; ch < n_chunks; ch += gridDim.x) {
+  for (int ch = blockIdx.x; ch < n_chunks; ch += 2 * gridDim.x) {
+    const bool have = ch + half * (int)gridDim.x < n_chunks;    // this half's chunk exists
+    const bool two = ch + (int)gridDim.x < n_chunks;            // both do
+    const int k_steps = two ? kPairPts / 32 : kChunkPts / 32;
     const float4 smp = smp_next;
-    if (ch + (int)gridDim.x < n_chunks)
-      smp_next = samples[train_sample_index(batch_start, ch + gridDim.x, p_local, n_samples)];
-    const f3 p{smp.x, smp.y, smp.z};
-    bf16x8 xb[4];
-    features(p, g, xb);
-    TileAct T;
-    const float o = forward_tile<true>(S.pack, S.small, xb, lane, T);
-    const float r = o - smp.w;
-    const float wgt = r > 0.0f ? over_weight : 1.0f;
-    const float dout = 2.0f * wgt * r * inv_b;
-    if (g == 0) {
-      loss += wgt * r * r * inv_b;
-      db4r += dout;
+    {
+      const int next = ch + (2 + half) * (int)gridDim.x;
+      if (next < n_chunks) smp_next = samples[train_sample_index(batch_start, next, p_local, n_samples)];
     }
+    TileAct T;
+    float dz[4][4], own[8];
+    if (have) {
+      bf16x8 xb[4];
+      features(f3{smp.x, smp.y, smp.z}, g, xb);
+      const float o = forward_tile<true>(S.pack, S.small, xb, lane, T);
+      const float r = o - smp.w;
+      const float wgt = r > 0.0f ? over_weight : 1.0f;
+      const float dout = 2.0f * wgt * r * inv_b;
+      const float l = wgt * r * r * inv_b;
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+      for (int q = 0; q < 8; ++q) {
+        const float lo = dout * T.h3[q >> 2][q & 3], hi = dout * T.h3[2 + (q >> 2)][q & 3];
+        own[q] = half ? hi : lo;
+        exchange[(8 * half + q) * kHalfThreads + xl] = half ? lo : hi;
+      }
+      if (half == 1) {
+        exchange[16 * kHalfThreads + xl] = dout;
+        exchange[17 * kHalfThreads + xl] = l;
+      } else if (g == 0) {
+        loss += l;
+        db4r += dout;
+      }
 #pragma unroll
-      for (int r2 = 0; r2 < 4; ++r2) dw4r[4 * m + r2] += dout * T.h3[m][r2];
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r2 = 0; r2 < 4; ++r2) dz[m][r2] = dout * S.small[256 + 16 * m + 4 * g + r2] * T.ds[3][m][r2];
+    }
 
     // backward through the hidden layers, chaining dZ in registers
-    float dz[4][4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-#pragma unroll
-      for (int r2 = 0; r2 < 4; ++r2) dz[m][r2] = dout * S.small[256 + 16 * m + 4 * g + r2] * dsilu(T.z[3][m][r2]);
 #pragma unroll
     for (int L = 3; L >= 0; --L) {
-      // stage dZ_L
+      __bf16(*const dzT)[kRow] = (L & 1) ? S.dz1 : S.dz0;
+      __bf16(*const inT)[kRow] = (L & 1) ? S.in1 : S.in0;
+      if (have) {
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
+        for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) S.dzT[L][16 * m + 4 * g + r2][p_local] = (__bf16)dz[m][r2];
-      if (L == 0) break;
-      bf16x8 dzb[2];
+          for (int r2 = 0; r2 < 4; ++r2) dzT[16 * m + 4 * g + r2][p_row] = (__bf16)dz[m][r2];
+        if (L > 0) {
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
+          for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) dzb[m >> 1][(m & 1) * 4 + r2] = (__bf16)dz[m][r2];
-      const int off = (oPackB1 + (L - 1) * kPackL) >> 3;
-      f32x4 dh[4];
+            for (int r2 = 0; r2 < 4; ++r2)
+              inT[16 * m + 4 * g + r2][p_row] = T.hb[L - 1][m >> 1][(m & 1) * 4 + r2];
+        } else {
+          // taken again (12 of the chunk's transcendentals): kept since the
+          // forward pass they are 16 registers that the others then spill
+          float px = smp.x, py = smp.y, pz = smp.z;
+          asm volatile("" : "+v"(px), "+v"(py), "+v"(pz));
+          bf16x8 xb[4];
+          features(f3{px, py, pz}, g, xb);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        dh[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+          for (int c = 0; c < 4; ++c) {
+            if (c == 3 && g >= 2) break;  // rows 112..127 are zero padding, never read
 #pragma unroll
-        for (int c = 0; c < 2; ++c) dh[m] = mfma16(S.pack[off + (m * 2 + c) * 64 + lane], dzb[c], dh[m]);
-      }
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) dz[m][r2] = dh[m][r2] * dsilu(T.z[L - 1][m][r2]);
-    }
-    // stage the inputs of layers 0..3: features (rows 0..111), h0..h2
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      if (c == 3 && g >= 2) break;  // rows 112..127 are zero padding, never read
-#pragma unroll
-      for (int s = 0; s < 8; ++s) S.xT[32 * c + 8 * g + s][p_local] = xb[c][s];
-    }
-#pragma unroll
-    for (int L = 0; L < 3; ++L)
-#pragma unroll
-      for (int m = 0; m < 4; ++m)
-#pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) S.hT[L][16 * m + 4 * g + r2][p_local] = T.hb[L][m >> 1][(m & 1) * 4 + r2];
-    __syncthreads();
-
-    // weight gradient of layer w: dW = dZ^T (64 x pts) . H (pts x in), K = points
-    const int n_tiles = (w == 0) ? 7 : 4;
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&S.dzT[w][16 * mi + j][32 * kc + 8 * g]);
-        accb[mi] = mfma16(a, ones, accb[mi]);
-#pragma unroll
-        for (int nj = 0; nj < 7; ++nj) {
-          if (nj >= n_tiles) break;
-          const __bf16* brow = (w == 0) ? &S.xT[16 * nj + j][32 * kc + 8 * g] : &S.hT[w - 1][16 * nj + j][32 * kc + 8 * g];
-          acc[mi][nj] = mfma16(a, *reinterpret_cast<const bf16x8*>(brow), acc[mi][nj]);
+            for (int s = 0; s < 8; ++s) inT[32 * c + 8 * g + s][p_row] = xb[c][s];
+          }
         }
       }
+      // The layer is staged; the other buffer's readers are done with it once
+      // every wave has passed here, so it may be written after.
+      __syncthreads();
+      if (L == 3) {
+        // the first chunk's products, then the second's
+        if (half == 0) {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) dw4r[q] += own[q];
+          if (two) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) dw4r[q] += exchange[(8 + q) * kHalfThreads + xl];
+            if (g == 0) {
+              db4r += exchange[16 * kHalfThreads + xl];
+              loss += exchange[17 * kHalfThreads + xl];
+            }
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) dw4r[q] += exchange[q * kHalfThreads + xl];
+          if (two) {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) dw4r[q] += own[q];
+          }
+        }
+      }
+      // this wave's tiles of dW = dZ^T (64 x points) . H (points x in)
+      const int n0 = L > 0 ? 2 * odd : 4 * odd;  // first column tile
+      const int n_tiles = L > 0 ? 2 : (odd ? 3 : 4);
+#pragma unroll
+      for (int kc = 0; kc < kPairPts / 32; ++kc) {
+        if (kc >= k_steps) break;
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(&dzT[16 * mi + j][32 * kc + 8 * g]);
+        if (odd == (L >> 1)) accb[L & 1] = mfma16(a, ones, accb[L & 1]);
+#pragma unroll
+        for (int t = 0; t < (L > 0 ? 2 : 4); ++t) {
+          if (t >= n_tiles) break;
+          acc[L][t] = mfma16(a, *reinterpret_cast<const bf16x8*>(&inT[16 * (n0 + t) + j][32 * kc + 8 * g]), acc[L][t]);
+        }
+      }
+      if (have && L > 0) {
+        bf16x8 dzb[2];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int r2 = 0; r2 < 4; ++r2) dzb[m >> 1][(m & 1) * 4 + r2] = (__bf16)dz[m][r2];
+        const int off = (oPackB1 + (L - 1) * kPackL) >> 3;
+        f32x4 dh[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          dh[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int c = 0; c < 2; ++c) dh[m] = mfma16(S.pack[off + (m * 2 + c) * 64 + lane], dzb[c], dh[m]);
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+          for (int r2 = 0; r2 < 4; ++r2) dz[m][r2] = dh[m][r2] * T.ds[L - 1][m][r2];
+      }
     }
-    __syncthreads();
   }
 
   // write this block's partial gradient (flat parameter layout) and loss
   float* P = partial + (int64_t)blockIdx.x * (kParams + 1);
-  {
-    const int nin = (w == 0) ? kIn : kH;
-    const int oW = (w == 0) ? oW0 : (w == 1 ? oW1 : (w == 2 ? oW2 : oW3));
-    const int ob = (w == 0) ? ob0 : (w == 1 ? ob1 : (w == 2 ? ob2 : ob3));
-    const int n_tiles = (w == 0) ? 7 : 4;
-    if (j == 0)
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
+  for (int L = 0; L < 4; ++L) {
+    const int nin = L == 0 ? kIn : kH;
+    const int oW = L == 0 ? oW0 : (L == 1 ? oW1 : (L == 2 ? oW2 : oW3));
+    const int ob = L == 0 ? ob0 : (L == 1 ? ob1 : (L == 2 ? ob2 : ob3));
+    const int n0 = L > 0 ? 2 * odd : 4 * odd;
+    const int n_tiles = L > 0 ? 2 : (odd ? 3 : 4);
+    if (odd == (L >> 1) && j == 0)
 #pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) P[ob + 16 * mi + 4 * g + r2] = accb[mi][r2];
+      for (int r2 = 0; r2 < 4; ++r2) P[ob + 16 * mi + 4 * g + r2] = accb[L & 1][r2];
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
+    for (int t = 0; t < (L > 0 ? 2 : 4); ++t) {
+      if (t >= n_tiles) break;
 #pragma unroll
-      for (int nj = 0; nj < 7; ++nj) {
-        if (nj >= n_tiles) break;
-#pragma unroll
-        for (int r2 = 0; r2 < 4; ++r2) {
-          const int i = 16 * mi + 4 * g + r2, k = 16 * nj + j;
-          if (k < nin) P[oW + i * nin + k] = acc[mi][nj][r2];
-        }
+      for (int r2 = 0; r2 < 4; ++r2) {
+        const int i = 16 * mi + 4 * g + r2, k = 16 * (n0 + t) + j;
+        if (k < nin) P[oW + i * nin + k] = acc[L][t][r2];
       }
+    }
   }
   // the output layer: over the 16 points of a lane group, then over the four
-  // waves (the loop ended on a barrier: the staging area is free)
-  float* red = reinterpret_cast<float*>(&S.dzT[0][0][0]);  // [wave][64], then [wave][2]
+  // waves of a half (the buffer of layers 3 and 1 has no readers left: every
+  // wave has passed layer 0's barrier since)
+  float* red = reinterpret_cast<float*>(&S.dz1[0][0]);  // [wave][64], then [wave][2]
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
+  for (int q = 0; q < 8; ++q) {
     float v = dw4r[q];
     v += __shfl_xor(v, 1);
     v += __shfl_xor(v, 2);
     v += __shfl_xor(v, 4);
     v += __shfl_xor(v, 8);
-    if (j == 0) red[w * 64 + 16 * (q >> 2) + 4 * g + (q & 3)] = v;
+    if (j == 0) red[(wv & 3) * 64 + 16 * (2 * half + (q >> 2)) + 4 * g + (q & 3)] = v;
   }
-  float d4 = db4r, l = loss;
-  for (int off = 32; off > 0; off >>= 1) {
-    d4 += __shfl_xor(d4, off);
-    l += __shfl_xor(l, off);
-  }
-  if (lane == 0) {
-    red[4 * 64 + 2 * w] = d4;
-    red[4 * 64 + 2 * w + 1] = l;
+  if (half == 0) {
+    float d4 = db4r, l = loss;
+    for (int off = 32; off > 0; off >>= 1) {
+      d4 += __shfl_xor(d4, off);
+      l += __shfl_xor(l, off);
+    }
+    if (lane == 0) {
+      red[4 * 64 + 2 * wv] = d4;
+      red[4 * 64 + 2 * wv + 1] = l;
+    }
   }
   __syncthreads();
   if (threadIdx.x < 64) {
@@ -501,15 +574,18 @@ __global__ void mlp_update_kernel(float* __restrict__ params, float* __restrict_
   pack_param(p, wv, pack, small);
 }
 
-// The two stages above in one launch: a block covers 64 parameters with four
-// quarters of threads; quarter q sums the kFold-row groups q, q + 4, ... in
-// row order, then one thread per parameter adds the group sums in group order
-// and takes the Adam step.  The additions are the ones the two stages make,
+// The two stages above in one launch: a block covers 64 parameters with
+// kReduceRows rows of threads; row q sums the kFold-row groups q, q +
+// kReduceRows, ... in row order, then one thread per parameter adds the group
+// sums in group order and takes the Adam step.  Bound by the partials' 19.4 MB
+// (256 blocks): with a row of threads per group every load is in flight at
+// once, 7.6 us against 8.6 with four rows.  The additions are the ones the two stages make,
 // in the same order, so the result is the same to the bit.
 constexpr int kReduceParams = 64;
+constexpr int kReduceRows = 16;
 constexpr int kMaxFoldGroups = 64;
 
-__global__ void __launch_bounds__(256) grad_reduce_update_kernel(
+__global__ void __launch_bounds__(kReduceParams * kReduceRows) grad_reduce_update_kernel(
     float* __restrict__ params, float* __restrict__ m1, float* __restrict__ m2, const float* __restrict__ partial,
     int32_t n_blocks, int32_t step, float lr, float b1, float b2, float eps, int32_t do_adam,
     float* __restrict__ grad_out, __bf16* __restrict__ pack, float* __restrict__ small, float* __restrict__ loss_out) {
@@ -518,7 +594,7 @@ __global__ void __launch_bounds__(256) grad_reduce_update_kernel(
   const int p = blockIdx.x * kReduceParams + pl;
   const int n_groups = (n_blocks + kFold - 1) / kFold;
   if (p <= kParams) {
-    for (int sg = q; sg < n_groups; sg += 256 / kReduceParams) {
+    for (int sg = q; sg < n_groups; sg += kReduceRows) {
       const int r0 = sg * kFold;
       const int r1 = r0 + kFold < n_blocks ? r0 + kFold : n_blocks;
       float v[kFold];
@@ -860,7 +936,8 @@ hipError_t launch_mlp_update(float* params, float* m1, float* m2, float* partial
   const int threads = 256;
   const int blocks = (kParams + 1 + threads - 1) / threads;
   if (partial && n_blocks > 0 && (n_blocks + kFold - 1) / kFold <= kMaxFoldGroups) {
-    hipLaunchKernelGGL(grad_reduce_update_kernel, dim3((kParams + kReduceParams) / kReduceParams), dim3(256), 0, s,
+    hipLaunchKernelGGL(grad_reduce_update_kernel, dim3((kParams + kReduceParams) / kReduceParams),
+                       dim3(kReduceParams * kReduceRows), 0, s,
                        params, m1, m2, partial, n_blocks, step, lr, b1, b2, eps, do_adam, grad_out, (__bf16*)pack,
                        small, loss_out);
     return hipGetLastError();
