@@ -171,7 +171,7 @@ __device__ __forceinline__ void trace_ray(const NodeEntry* __restrict__ nodes, c
     f3 ro, rd;
     xform_ray(ob, o, d, secondary, ro, rd);
     // the slab reciprocals once per object, not per leaf (bit-identical)
-    const f3 fr{1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z};
+    const f3 fr{recip(rd.x), recip(rd.y), recip(rd.z)};
     float t_entry, t_exit;
     if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) continue;
     int32_t cur = ob.root;
@@ -440,7 +440,7 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
       ++k_obj;
       const ObjXform ob = objs[k_obj];
       xform_ray(ob, o, d, secondary, ro, rd);
-      fr = f3{1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z};
+      fr = f3{recip(rd.x), recip(rd.y), recip(rd.z)};
       if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) continue;
       cur = ob.root;
       if (HINT != 0) cur = hinted_start(leaves, n_leaves, hint, k_obj, add(ro, smul(t_entry, rd)), cur);

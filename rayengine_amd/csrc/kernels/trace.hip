@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(256) trace_persistent_kernel(
       ++k_obj;
       const ObjXform ob = objs[k_obj];
       xform_ray(ob, o, d, secondary != 0, ro, rd);
-      fr = f3{1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z};
+      fr = f3{recip(rd.x), recip(rd.y), recip(rd.z)};
       if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) continue;
       cur = ob.root;
       visits = 0;
@@ -338,7 +338,7 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
   // the walk of object k from the ray (o, d): its first visit, or none
   auto start_walk = [&](const ObjXform& ob, int32_t k, f3 oo, f3 dd) {
     xform_ray(ob, oo, dd, secondary != 0, ro, rd);
-    fr = f3{1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z};
+    fr = f3{recip(rd.x), recip(rd.y), recip(rd.z)};
     if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) return;
     cur = ob.root;
     if (HINT != 0) cur = hinted_start(leaves, n_leaves, hint, k, add(ro, smul(t_entry, rd)), cur);
@@ -526,7 +526,7 @@ __global__ void __launch_bounds__(256) trace_status_kernel(const NodeEntry* __re
     const ObjXform ob = objs[k];
     f3 ro, rd;
     xform_ray(ob, o, d, secondary != 0, ro, rd);
-    const f3 fr{1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z};
+    const f3 fr{recip(rd.x), recip(rd.y), recip(rd.z)};
     float t_entry, t_exit;
     if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) {
       reason = 5;
