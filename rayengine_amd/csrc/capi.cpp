@@ -339,6 +339,7 @@ re_status trace_common(re_ctx* ctx, int32_t scene_id, const float* ray_o, const 
     if (g <= 0) g = p.variant == 5 ? trace_coop_refill_grid(blk) : trace_persistent_grid(blk);
     L.grid_blocks = g;
   }
+  const bool queue = p.variant == 1 || trace_refills(p.variant, n, it->second.n_trirecs);
   const bool dev = (flags & RE_DEVICE_PTRS) != 0;
   const size_t ray_bytes = (size_t)n * 12;
   char* base = nullptr;
@@ -386,7 +387,7 @@ re_status trace_common(re_ctx* ctx, int32_t scene_id, const float* ray_o, const 
     // capture the call in a graph
     if (counts) HIP_TRY(ctx, launch_zero_words((uint32_t*)d_counts, (int32_t)(sizeof(TraceCounts) / 4), ctx->stream),
                         "counts clear");
-    if (L.variant == 1 || L.variant == 5)
+    if (queue)
       HIP_TRY(ctx, launch_zero_words((uint32_t*)L.queue, kQueueWords, ctx->stream), "queue clear");
   }
   HIP_TRY(ctx, ctx->launch_begin(), "event");

@@ -129,6 +129,12 @@ __device__ __forceinline__ uint32_t descend(const NodeEntry* __restrict__ nodes,
   }
 }
 
+__device__ __forceinline__ void load_ray(const float* __restrict__ ray_o, const float* __restrict__ ray_d, int64_t i,
+                                         f3& o, f3& d) {
+  o = f3{ray_o[3 * i], ray_o[3 * i + 1], ray_o[3 * i + 2]};
+  d = f3{ray_d[3 * i], ray_d[3 * i + 1], ray_d[3 * i + 2]};
+}
+
 // The state that decides a walk's next visit is (cur, t_entry, t_exit).
 // When it equals the state of one of the last two visits, no hit was
 // accepted in between (an accepted hit lowers t_exit), so from here the walk
@@ -279,10 +285,10 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
   return x;
 }
 
-template <bool ONE_SIDED>
+template <bool ONE_SIDED, bool ANY = false>
 __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, bool at_leaf, uint32_t first,
                                                uint32_t cnt, f3 ro, f3 rd, float& t_exit, bool& found, float& hit_t,
-                                               int32_t& hit_prim, CoopWave& W) {
+                                               uint32_t& hit_rec, CoopWave& W) {
   const int lane = threadIdx.x & 63;
   const unsigned long long at_mask = __ballot(at_leaf);
   const int lead = __ffsll((long long)at_mask) - 1;  // wave-uniform
@@ -304,7 +310,7 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       if (at_leaf) {
-        for (uint32_t j = 0; j < m; ++j) {
+        for (uint32_t j = 0; j < m && !(ANY && found); ++j) {
           const float* f = stage[j].v0;
           float t;
           const f3 v0{f[0], f[1], f[2]}, e1{f[3], f[4], f[5]}, e2{f[6], f[7], f[8]};
@@ -312,7 +318,7 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
           if (h && t < t_exit) {
             found = true;
             hit_t = t;
-            hit_prim = stage[j].prim;
+            hit_rec = lead_first + base + j;
             t_exit = t;
           }
         }
@@ -329,7 +335,9 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
   // in a scalar register, so the loops below exit on scalar branches taken by
   // the whole wave (their bodies hold wave barriers)
   const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-  W.slot[lane] = ~0ull;
+  uint32_t* const any = reinterpret_cast<uint32_t*>(W.slot);  // ANY: a record that is hit, whichever
+  if (ANY) any[lane] = ~0u;
+  else W.slot[lane] = ~0ull;
   if (at_leaf) {
     W.ray[lane][0] = make_float4(ro.x, ro.y, ro.z, t_exit);
     W.ray[lane][1] = make_float4(rd.x, rd.y, rd.z, __uint_as_float(first - excl));
@@ -359,7 +367,9 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
         float t;
         const bool h =
             ONE_SIDED ? ray_tri(oro, ord, g.v0, g.e1, g.e2, t) : ray_tri_2s(oro, ord, g.v0, g.e1, g.e2, t);
-        if (h && t < a.w)
+        if (ANY) {
+          if (h && t < a.w) any[L] = rec;
+        } else if (h && t < a.w)
           atomicMin(&W.slot[L], ((unsigned long long)__float_as_uint(t) << 32) | (unsigned long long)rec);
       }
     }
@@ -367,12 +377,18 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  if (at_leaf) {
+  if (ANY) {
+    const uint32_t rec = any[lane];
+    if (at_leaf && rec != ~0u) {
+      found = true;
+      hit_rec = rec;
+    }
+  } else if (at_leaf) {
     const unsigned long long sv = W.slot[lane];
     if (sv != ~0ull) {
       found = true;
       hit_t = __uint_as_float((uint32_t)(sv >> 32));
-      hit_prim = tris[(uint32_t)sv].prim;
+      hit_rec = (uint32_t)sv;
       t_exit = hit_t;
     }
   }
@@ -411,11 +427,14 @@ __device__ __forceinline__ int32_t hinted_start(const DevLeaf* __restrict__ leav
 // part in the wave's work without a ray of their own.  Results are
 // bit-identical to trace_ray's.  Every lane of the wave must call it (it
 // holds wave-wide operations); the loop ends on a wave-uniform branch.
-template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0>
+// With ANY (as in trace_ray) a lane is done at its first accepted hit.
+// ray(o, d) reads the lane's ray: once per object, so that with several
+// objects the untransformed ray holds no registers during a walk.
+template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0, bool ANY = false, class Ray>
 __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ nodes,
                                                 const DevLeaf* __restrict__ leaves, const TriRec* __restrict__ tris,
                                                 const ObjXform* __restrict__ objs, int32_t k0, int32_t k1,
-                                                bool has_ray, f3 o, f3 d, int32_t cap, bool secondary, float& best_t,
+                                                bool has_ray, const Ray& ray, int32_t cap, bool secondary, float& best_t,
                                                 int32_t& best_prim, int32_t& best_obj, RayCounts& rc, CoopWave& W,
                                                 int32_t hint = -1, int64_t n_leaves = 0,
                                                 int32_t* best_leaf = nullptr) {
@@ -429,7 +448,8 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
   bool live = false, open = false, done = !has_ray;
   f3 ro{0, 0, 0}, rd{0, 0, 0}, fr{0, 0, 0};
   float t_entry = 0.0f, t_exit = 0.0f, hit_t = kInf;
-  int32_t hit_prim = -1, cur = 0, visits = 0;
+  uint32_t hit_rec = 0;  // record of the walk's hit, valid when found
+  int32_t cur = 0, visits = 0;
   bool found = false, have_window = false;
   uint4 w = make_uint4(0u, 0u, 0u, 0u);
   WalkMemo memo;
@@ -439,6 +459,8 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
     while (!live && k_obj + 1 < k_end) {
       ++k_obj;
       const ObjXform ob = objs[k_obj];
+      f3 o, d;
+      ray(o, d);
       xform_ray(ob, o, d, secondary, ro, rd);
       fr = f3{recip(rd.x), recip(rd.y), recip(rd.z)};
       if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) continue;
@@ -446,7 +468,6 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
       if (HINT != 0) cur = hinted_start(leaves, n_leaves, hint, k_obj, add(ro, smul(t_entry, rd)), cur);
       found = false;
       hit_t = kInf;
-      hit_prim = -1;
       visits = 0;
       have_window = false;
       memo = WalkMemo{};
@@ -461,15 +482,15 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
     // a lane between walks closes the last one and, with more objects,
     // starts the next
     if (!live && !done) {
-      if (open && found && hit_t < best_t) {
+      if (open && found && (ANY || hit_t < best_t)) {
         best_t = hit_t;
-        best_prim = hit_prim;
+        best_prim = tris[hit_rec].prim;
         best_obj = k_obj;
         if (HINT == 2) *best_leaf = last_leaf;
       }
+      if (ONE_OBJ || (ANY && open && found)) done = true;
       open = false;
-      if (ONE_OBJ) done = true;
-      else start_next();
+      if (!done) start_next();
     }
     if (__ballot(!done) == 0ull) break;
     bool at_leaf = false, box_ok = false;
@@ -508,11 +529,11 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
       }
     }
     if (__ballot(at_leaf) != 0ull) {
-      coop_leaf_test<ONE_SIDED>(tris, at_leaf, first, cnt, ro, rd, t_exit, found, hit_t, hit_prim, W);
+      coop_leaf_test<ONE_SIDED, ANY>(tris, at_leaf, first, cnt, ro, rd, t_exit, found, hit_t, hit_rec, W);
       if (COUNT && at_leaf) rc.tri += cnt;
     }
     if (at_leaf) {
-      if (!box_ok) {
+      if (!box_ok || (ANY && found)) {
         live = false;
       } else {
         t_entry = tf;

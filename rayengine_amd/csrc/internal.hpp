@@ -131,6 +131,21 @@ int64_t trace_coop_refill_grid(int block);
 // default (256 for the persistent per-lane variant 1, one wave otherwise).
 inline int trace_launch_block(int block, int variant) { return block > 0 ? block : (variant == 1 ? 256 : 64); }
 
+// Whether variant 5 refills its waves, or is the plain cooperative kernel (the
+// same walks, one set of rays a wave).  Refill keeps lanes busy where walks are
+// long and uneven, and pays for it with a counter per 64 rays, a setup of 32
+// rays at a time and waves whose halves are apart.  It is ahead once a launch
+// has two rounds of resident waves (256 CUs x 24) and the scene 10^5 triangle
+// records.  us, refill / plain, diffuse bounces: 2,919,928 records, 207,360
+// rays 245 / 224, 507,206 398 / 368, 829,440 463 / 485, 1,866,240 768 / 899;
+// 157,048 records, 829,440 rays 391 / 366, 3,317,760 1054 / 1093; 68,589
+// records, 207,360 rays 165 / 131, 829,440 322 / 270, 3,317,760 852 / 785;
+// 17,832 records, 1,866,240 rays 354 / 283.
+constexpr int64_t kRefillRays = 2 * 6144 * 64, kRefillRecs = 100000;
+inline bool trace_refills(int variant, int64_t n, int64_t n_trirecs) {
+  return variant == 5 && n > kRefillRays && n_trirecs > kRefillRecs;
+}
+
 hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s);
 // Zeroes n 32-bit words with a kernel (no memset node when a caller captures).
 hipError_t launch_zero_words(uint32_t* p, int32_t n, hipStream_t s);

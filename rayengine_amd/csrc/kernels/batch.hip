@@ -91,13 +91,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) b
         const int r = r0 + lane;
         const bool has = r < item.count;
         const int64_t i = item.begin + (has ? r : 0);
-        const f3 o{L.ray_o[3 * i], L.ray_o[3 * i + 1], L.ray_o[3 * i + 2]};
-        const f3 d{L.ray_d[3 * i], L.ray_d[3 * i + 1], L.ray_d[3 * i + 2]};
+        const auto ray = [&](f3& o, f3& d) { load_ray(L.ray_o, L.ray_d, i, o, d); };
         float bt;
         int32_t bp, bo;
         RayCounts rc;
         coop_trace_wave<false, ONE_SIDED, true>(L.nodes, L.leaves, L.tris, L.objs, item.target, item.target + 1, has,
-                                                o, d, L.cap, L.secondary != 0, bt, bp, bo, rc, wv);
+                                                ray, L.cap, L.secondary != 0, bt, bp, bo, rc, wv);
         if (has) {
           L.prim[i] = bp;
           L.t[i] = bt;

@@ -75,28 +75,6 @@ trace_closest_o6_kernel(RE_CLOSEST_PARAMS) {
   closest_body<COUNT, ONE_SIDED, true, ONE_OBJ>(RE_CLOSEST_ARGS);
 }
 
-// Any-hit query (trace_shadow, RayEngine/src/cuda-src/ray_functions.cuh:365-374):
-// one ray per lane, last block first, 6-wave budget; each ray stops at its
-// first accepted hit.
-template <bool ONE_SIDED>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
-trace_occluded_kernel(const NodeEntry* __restrict__ nodes, const DevLeaf* __restrict__ leaves,
-                      const TriRec* __restrict__ tris, const ObjXform* __restrict__ objs, int32_t n_obj,
-                      const float* __restrict__ ray_o, const float* __restrict__ ray_d, int64_t n, int32_t cap,
-                      int32_t secondary, uint8_t* __restrict__ occluded) {
-  const int64_t n_blk = (n + blockDim.x - 1) / blockDim.x;
-  const int64_t i = (n_blk - 1 - (int64_t)blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const f3 o{ray_o[3 * i], ray_o[3 * i + 1], ray_o[3 * i + 2]};
-  const f3 d{ray_d[3 * i], ray_d[3 * i + 1], ray_d[3 * i + 2]};
-  float best_t;
-  int32_t best_prim, best_obj;
-  RayCounts rc;
-  trace_ray<false, ONE_SIDED, true>(nodes, leaves, tris, objs, 0, n_obj, o, d, cap, secondary != 0, best_t,
-                                    best_prim, best_obj, rc);
-  occluded[i] = best_prim >= 0 ? 1 : 0;
-}
-
 // ---------------------------------------------------------------------------
 // Persistent variant.  A wave keeps 64 rays in flight and refills each lane
 // as soon as its ray finishes, from a wave-private chunk of CHUNK
@@ -250,22 +228,22 @@ __global__ void __launch_bounds__(256) trace_persistent_kernel(
 template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int32_t* __restrict__ hit_leaf,
-                  int64_t n_leaves) {
+                  int64_t n_leaves, int32_t lanes) {
   // one CoopWave per wave of the block (dynamic LDS sized by the launch)
   extern __shared__ CoopWave waves[];
   CoopWave& wv = waves[threadIdx.x >> 6];
-  const int64_t blk = (int64_t)(gridDim.x - 1 - blockIdx.x);  // last block of rays first
-  const int64_t i = blk * blockDim.x + threadIdx.x;
-  const bool has_ray = i < n;
-  const int64_t ic = has_ray ? i : 0;
-  const f3 o{ray_o[3 * ic], ray_o[3 * ic + 1], ray_o[3 * ic + 2]};
-  const f3 d{ray_d[3 * ic], ray_d[3 * ic + 1], ray_d[3 * ic + 2]};
+  const int lane = (int)(threadIdx.x & 63);
+  // `lanes` rays a wave, the last block of rays first
+  const int64_t blk = (int64_t)(gridDim.x - 1 - blockIdx.x);
+  const int64_t i = (blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * lanes + lane;
+  const bool has_ray = lane < lanes && i < n;
+  const auto ray = [&](f3& o, f3& d) { load_ray(ray_o, ray_d, i, o, d); };
   float best_t;
   int32_t best_prim, best_obj;
   RayCounts rc;
   const int32_t hint = (HINT != 0 && start_leaf && has_ray) ? start_leaf[i] : -1;
   int32_t best_leaf = -1;
-  coop_trace_wave<COUNT, ONE_SIDED, ONE_OBJ, HINT>(nodes, leaves, tris, objs, 0, ONE_OBJ ? 1 : n_obj, has_ray, o, d,
+  coop_trace_wave<COUNT, ONE_SIDED, ONE_OBJ, HINT>(nodes, leaves, tris, objs, 0, ONE_OBJ ? 1 : n_obj, has_ray, ray,
                                                    cap, secondary != 0, best_t, best_prim, best_obj, rc, wv, hint,
                                                    n_leaves, &best_leaf);
   if (has_ray) {
@@ -282,6 +260,34 @@ trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int
   }
 }
 
+// Any-hit query (trace_shadow, RayEngine/src/cuda-src/ray_functions.cuh:365-374):
+// the cooperative walk, each ray done at its first accepted hit.  us against
+// one ray per lane with its own leaf tests: 507,206 shadow rays on 2^20
+// clustered triangles 199 / 254, on 50,021 137 / 140, on 6,144 124 / 127;
+// 16,000 on 50,021 77 / 94.  (126,450 to 262,440 on 6,144 triangles, whose
+// waves stay together: 4 % slower, 83 / 81 and 103 / 100.)
+template <bool ONE_SIDED, bool ONE_OBJ>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
+trace_occluded_kernel(const NodeEntry* __restrict__ nodes, const DevLeaf* __restrict__ leaves,
+                      const TriRec* __restrict__ tris, const ObjXform* __restrict__ objs, int32_t n_obj,
+                      const float* __restrict__ ray_o, const float* __restrict__ ray_d, int64_t n, int32_t cap,
+                      int32_t secondary, uint8_t* __restrict__ occluded, int32_t lanes) {
+  extern __shared__ CoopWave waves[];
+  CoopWave& wv = waves[threadIdx.x >> 6];
+  const int lane = (int)(threadIdx.x & 63);
+  // the wave's first ray is a scalar, which leaves the kernel 72 registers
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t i = ((int64_t)(gridDim.x - 1 - blockIdx.x) * (blockDim.x >> 6) + w) * lanes + lane;
+  const bool has_ray = lane < lanes && i < n;
+  const auto ray = [&](f3& o, f3& d) { load_ray(ray_o, ray_d, i, o, d); };
+  float best_t;
+  int32_t best_prim, best_obj;
+  RayCounts rc;
+  coop_trace_wave<false, ONE_SIDED, ONE_OBJ, 0, true>(nodes, leaves, tris, objs, 0, ONE_OBJ ? 1 : n_obj, has_ray,
+                                                      ray, cap, secondary != 0, best_t, best_prim, best_obj, rc, wv);
+  if (has_ray) occluded[i] = best_prim >= 0 ? 1 : 0;
+}
+
 // Cooperative variant with refill (variant 5): persistent waves; once at
 // least half of a wave's lanes have finished their rays, those lanes take the
 // next rays at the start of the following visit round, from a wave-private
@@ -295,6 +301,13 @@ trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int
 // from the end of the array, so appended bounce rays start first.  Per-ray
 // results equal the other variants' (each ray's walk is the same sequence of
 // visits).
+// A 64-bit value that is the same in every lane, or lane 0's, as a scalar.
+__device__ __forceinline__ int64_t uniform64(unsigned long long v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  return (int64_t)(((unsigned long long)hi << 32) | lo);
+}
+
 constexpr int kRefillLanes = 32;  // refill threshold: half a wave
 
 // HINT: 0 none; 1 each ray's walk may start at its start_leaf entry (may be
@@ -325,10 +338,10 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
   int tried = 0;  // wave-uniform: parts found taken
   const int64_t part = ((n + kQueueSlots - 1) / kQueueSlots + 63) / 64 * 64;
   int64_t ray = -1;
-  f3 o{0, 0, 0}, d{0, 0, 0};  // kept only with several objects (the next object's transform)
   f3 ro{0, 0, 0}, rd{0, 0, 0}, fr{0, 0, 0};
   float t_entry = 0.0f, t_exit = 0.0f, hit_t = kInf, best_t = kInf;
-  int32_t k_obj = -1, cur = 0, visits = 0, hit_prim = -1, best_prim = -1, best_obj = -1;
+  uint32_t hit_rec = 0;  // record of the walk's hit, valid when found
+  int32_t k_obj = -1, cur = 0, visits = 0, best_prim = -1, best_obj = -1;
   int32_t hint = -1, walk_leaf = -1, best_leaf = -1;  // HINT only
   bool live = false, open = false, found = false, have_window = false;
   uint4 w = make_uint4(0u, 0u, 0u, 0u);
@@ -336,15 +349,16 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
   RayCounts rc;
   unsigned c_hit = 0;
   // the walk of object k from the ray (o, d): its first visit, or none
-  auto start_walk = [&](const ObjXform& ob, int32_t k, f3 oo, f3 dd) {
-    xform_ray(ob, oo, dd, secondary != 0, ro, rd);
+  auto start_walk = [&](const ObjXform& ob, int32_t k) {
+    f3 o, d;  // read again for each object: no registers held during a walk
+    load_ray(ray_o, ray_d, ray, o, d);
+    xform_ray(ob, o, d, secondary != 0, ro, rd);
     fr = f3{recip(rd.x), recip(rd.y), recip(rd.z)};
     if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) return;
     cur = ob.root;
     if (HINT != 0) cur = hinted_start(leaves, n_leaves, hint, k, add(ro, smul(t_entry, rd)), cur);
     found = false;
     hit_t = kInf;
-    hit_prim = -1;
     visits = 0;
     have_window = false;
     memo = WalkMemo{};
@@ -355,7 +369,7 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
   auto start_next = [&]() {
     while (!live && k_obj + 1 < k_end) {
       ++k_obj;
-      start_walk(objs[k_obj], k_obj, o, d);
+      start_walk(objs[k_obj], k_obj);
     }
   };
   auto finish = [&]() {
@@ -372,7 +386,7 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
     if (ray >= 0 && !live) {
       if (open && found && hit_t < best_t) {
         best_t = hit_t;
-        best_prim = hit_prim;
+        best_prim = tris[hit_rec].prim;
         best_obj = ONE_OBJ ? 0 : k_obj;
         if (HINT == 2) best_leaf = walk_leaf;
       }
@@ -390,14 +404,17 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
       if (pool_next >= pool_end) {
         // at most one chunk request per round: a part found taken moves the
         // wave on to the next part at the next round (every wave tries all
-        // parts before it stops, so every chunk is taken once)
+        // parts before it stops, so every chunk is taken once).  The parts
+        // after its own are read first and asked only while they have chunks
+        // left (a counter only grows): as additions, the last tries of 6144
+        // waves are 50 us of contention on eight lines
         const int x = (xcd + tried) & (kQueueSlots - 1);
         const int64_t lo_x = part * x < n ? part * x : n;
         const int64_t hi_x = part * (x + 1) < n ? part * (x + 1) : n;
-        const unsigned long long v = atomicAdd(queue + kQueueStride * x, lane == 0 ? 64ull : 0ull);
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-        const int64_t b = lo_x + (int64_t)(((unsigned long long)hi << 32) | lo);
+        unsigned long long* const q = queue + kQueueStride * x;
+        int64_t b = 0;
+        if (tried != 0) b = lo_x + uniform64(__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (b < hi_x) b = lo_x + uniform64(atomicAdd(q, lane == 0 ? 64ull : 0ull));
         if (b < hi_x) {
           pool_next = b;
           pool_end = b + 64 < hi_x ? b + 64 : hi_x;
@@ -410,8 +427,6 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
         const int rank = __popcll(need & below);
         if (ray < 0 && rank < avail) {
           ray = n - 1 - (pool_next + rank);
-          const f3 no{ray_o[3 * ray], ray_o[3 * ray + 1], ray_o[3 * ray + 2]};
-          const f3 nd{ray_d[3 * ray], ray_d[3 * ray + 1], ray_d[3 * ray + 2]};
           best_t = kInf;
           best_prim = -1;
           best_obj = -1;
@@ -420,10 +435,8 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
           live = false;
           open = false;
           if (ONE_OBJ) {
-            start_walk(objs[0], 0, no, nd);
+            start_walk(objs[0], 0);
           } else {
-            o = no;
-            d = nd;
             k_obj = -1;
             start_next();
           }
@@ -474,7 +487,7 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
       }
     }
     if (__ballot(at_leaf) != 0ull) {
-      coop_leaf_test<ONE_SIDED>(tris, at_leaf, first, cnt, ro, rd, t_exit, found, hit_t, hit_prim, W);
+      coop_leaf_test<ONE_SIDED>(tris, at_leaf, first, cnt, ro, rd, t_exit, found, hit_t, hit_rec, W);
       if (COUNT && at_leaf) rc.tri += cnt;
     }
     if (at_leaf) {
@@ -753,6 +766,25 @@ hipError_t debug_bounds_take(uint32_t* mask) {
 #endif
 }
 
+// Rays per wave of the cooperative kernels: 64, or fewer when the waves would
+// not fill the chip.  A launch of few rays lasts as long as its slowest wave,
+// which walks until its longest ray is done and tests the triangles of all
+// its lanes, 64 at a time: fewer rays a wave shorten both, as long as the
+// waves stay resident.  The limit is three quarters of the 6144 waves that
+// 256 CUs hold at 6 per SIMD.
+// us for 64 / 32 / 16 / 8 rays a wave, camera rays on 2^20 clustered triangles:
+// 4,096 rays 182 / 146 / 131 / 123; 72,720 rays 242 / 181 / 170 / 192;
+// 140,500 rays 255 / 199 / 182 / 239.  Incoherent rays on 20,000 triangles:
+// 4,096 rays 124 / 108 / 103 / 99; 72,720 rays 173 / 162 / 162 / 200;
+// 140,500 rays 190 / 173 / 223 / 289; 200,000 rays 196 / 223 / 277 / 364.
+// (4 rays a wave: within 3 % of 8 up to 17,600 rays, slower above.)
+constexpr int64_t kCoopFillWaves = 4608;
+static int coop_lanes(int64_t n) {
+  int lanes = 8;
+  while (lanes < 64 && n > lanes * kCoopFillWaves) lanes *= 2;
+  return lanes;
+}
+
 hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
   if (L.n <= 0) return hipSuccess;
   {
@@ -763,7 +795,9 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
   // the one-ray-per-thread kernels (finer dispatch granularity at the tail;
   // 64 and 128 measured alike and ahead of 256 on the cluster workload).
   const int block = trace_launch_block(L.block, L.variant);
-  if (L.variant == 5) {
+  const bool refill = trace_refills(L.variant, L.n, L.scene->n_trirecs);
+  const bool coop = L.variant == 4 || (L.variant == 5 && !refill);
+  if (refill) {
     // Persistent cooperative waves: enough blocks to fill every CU at the
     // kernel's occupancy, never more than the rays need.
     const int64_t want = (L.n + block - 1) / block;
@@ -818,7 +852,9 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
 #undef RE_LAUNCH
     return hipGetLastError();
   }
-  const int64_t grid = (L.n + block - 1) / block;
+  const int lanes = coop ? coop_lanes(L.n) : 64;
+  const int64_t per_block = (int64_t)(block / 64) * lanes;
+  const int64_t grid = (L.n + per_block - 1) / per_block;
 #define RE_LAUNCH(K, ...)                                                                                       \
   hipLaunchKernelGGL((K<__VA_ARGS__>), dim3((unsigned)grid), dim3(block), 0, s, S.nodes, S.leaves, S.tris, S.objs, \
                      S.n_obj, L.ray_o, L.ray_d, L.n, cap, L.secondary, L.prim, L.t, L.obj, L.counts)
@@ -832,13 +868,13 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
       else RE_LAUNCH(K, false, false __VA_ARGS__);                        \
     }                                                                     \
   } while (0)
-  if (L.variant == 4) {
+  if (coop) {
     const int hint = L.hit_leaf ? 2 : (L.start_leaf ? 1 : 0);
 #define RE_LAUNCH_COOP_H(C, O, ONE, H)                                                                        \
   hipLaunchKernelGGL((trace_coop_kernel<C, O, ONE, H>), dim3((unsigned)grid), dim3(block),                    \
                      (block / 64) * sizeof(CoopWave), s, S.nodes, S.leaves,                                      \
                      S.tris, S.objs, S.n_obj, L.ray_o, L.ray_d, L.n, cap, L.secondary, L.prim, L.t, L.obj,        \
-                     L.counts, L.start_leaf, L.hit_leaf, S.n_leaves)
+                     L.counts, L.start_leaf, L.hit_leaf, S.n_leaves, lanes)
 #define RE_LAUNCH_COOP(C, O, ONE)                                         \
   do {                                                                    \
     if (hint == 2) RE_LAUNCH_COOP_H(C, O, ONE, 2);                        \
@@ -873,13 +909,17 @@ hipError_t launch_trace_occluded(const TraceLaunch& L, hipStream_t s) {
   const int block = L.block > 0 ? L.block : 64;
   const DevScene& S = *L.scene;
   const int32_t cap = (L.cap > 0 && L.cap < kMaxLeafVisits) ? L.cap : kMaxLeafVisits;
-  const int64_t grid = (L.n + block - 1) / block;
-  if (L.one_sided)
-    hipLaunchKernelGGL(trace_occluded_kernel<true>, dim3((unsigned)grid), dim3(block), 0, s, S.nodes, S.leaves,
-                       S.tris, S.objs, S.n_obj, L.ray_o, L.ray_d, L.n, cap, L.secondary, L.occluded);
-  else
-    hipLaunchKernelGGL(trace_occluded_kernel<false>, dim3((unsigned)grid), dim3(block), 0, s, S.nodes, S.leaves,
-                       S.tris, S.objs, S.n_obj, L.ray_o, L.ray_d, L.n, cap, L.secondary, L.occluded);
+  const int lanes = coop_lanes(L.n);
+  const int64_t per_block = (int64_t)(block / 64) * lanes;
+  const int64_t grid = (L.n + per_block - 1) / per_block;
+#define RE_LAUNCH_OCCLUDED(O, ONE)                                                                            \
+  hipLaunchKernelGGL((trace_occluded_kernel<O, ONE>), dim3((unsigned)grid), dim3(block),                      \
+                     (block / 64) * sizeof(CoopWave), s, S.nodes, S.leaves, S.tris, S.objs, S.n_obj, L.ray_o, \
+                     L.ray_d, L.n, cap, L.secondary, L.occluded, lanes)
+  const bool one = S.n_obj == 1;
+  if (L.one_sided) { if (one) RE_LAUNCH_OCCLUDED(true, true); else RE_LAUNCH_OCCLUDED(true, false); }
+  else { if (one) RE_LAUNCH_OCCLUDED(false, true); else RE_LAUNCH_OCCLUDED(false, false); }
+#undef RE_LAUNCH_OCCLUDED
   return hipGetLastError();
 }
 
