@@ -615,7 +615,8 @@ typedef struct re_batch_tile {
 } re_batch_tile;
 
 typedef struct re_batch_config {
-  int32_t item_rays; /* rays per work item, default 256 */
+  int32_t item_rays; /* rays per work item of the plan, default 256; the device's items are shorter where
+                        the launch has few */
   int32_t block;     /* threads per block (64, 128, 256), default 256 */
   int32_t mlp_id;    /* network of surrogate tiles, -1 none */
   re_trace_params trace;

@@ -766,25 +766,6 @@ hipError_t debug_bounds_take(uint32_t* mask) {
 #endif
 }
 
-// Rays per wave of the cooperative kernels: 64, or fewer when the waves would
-// not fill the chip.  A launch of few rays lasts as long as its slowest wave,
-// which walks until its longest ray is done and tests the triangles of all
-// its lanes, 64 at a time: fewer rays a wave shorten both, as long as the
-// waves stay resident.  The limit is three quarters of the 6144 waves that
-// 256 CUs hold at 6 per SIMD.
-// us for 64 / 32 / 16 / 8 rays a wave, camera rays on 2^20 clustered triangles:
-// 4,096 rays 182 / 146 / 131 / 123; 72,720 rays 242 / 181 / 170 / 192;
-// 140,500 rays 255 / 199 / 182 / 239.  Incoherent rays on 20,000 triangles:
-// 4,096 rays 124 / 108 / 103 / 99; 72,720 rays 173 / 162 / 162 / 200;
-// 140,500 rays 190 / 173 / 223 / 289; 200,000 rays 196 / 223 / 277 / 364.
-// (4 rays a wave: within 3 % of 8 up to 17,600 rays, slower above.)
-constexpr int64_t kCoopFillWaves = 4608;
-static int coop_lanes(int64_t n) {
-  int lanes = 8;
-  while (lanes < 64 && n > lanes * kCoopFillWaves) lanes *= 2;
-  return lanes;
-}
-
 hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
   if (L.n <= 0) return hipSuccess;
   {
