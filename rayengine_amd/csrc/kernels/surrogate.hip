@@ -753,6 +753,8 @@ __device__ __forceinline__ float wave_surrogate(const bf16x8* spack, const float
   return need ? wout[slot] : 0.0f;
 }
 
+// The march through the learned distance, one ray per lane; a wave takes new
+// rays for its idle lanes once half of its lanes are idle.
 // Exact-phase march: h = max(f * k_exact, h_min) from a point with f > 0;
 // on the first sample with f <= 0 the crossing is bisected (n_bisect steps)
 // between the last positive and the first non-positive sample.
@@ -760,25 +762,41 @@ __device__ __forceinline__ float wave_surrogate(const bf16x8* spack, const float
 // exceeds tau, then hand over to the exact phase; after rejoin of exact
 // travel without a crossing, return to the surrogate.
 constexpr int kDeferTile = 16;
+// Blocks of the network's march: two per CU (84 VGPRs, 50 KB of LDS), each
+// wave taking rays until the block's are gone.  With a block per 512 rays a
+// block stayed until its longest march was done and whole blocks of the image
+// cost many times others: 921,600 rays on 192^3 1,042 us, now 964 (their 7.7 M
+// network points alone take 610 at the inference kernel's rate).
+constexpr int64_t kHybridBlocks = 512;
+// Rays a wave holds: 64, or fewer while 12,288 runs (three per wave) are not
+// reached, as a wave lasts as long as its longest march and the network's
+// tile is 16 points.  us for 16 / 32 / 64 (and a block per 512 rays): 14,400
+// rays 93 / 127 / 160 (198); 90,000 203 / 291 / 331 (323); 140,500 252 / 278 /
+// 303 (334); 230,400 422 / 418 / 528 (487); 360,000 595 / 515 / 663 (596);
+// 518,400 783 / 719 / 729 (763); 921,600 1,355 / 1,122 / 964 (1,042).
+constexpr int64_t kHybridRuns = 12288;
 
 template <bool USE_MLP, bool NARROW>
 __global__ void __launch_bounds__(512) hybrid_trace_kernel(
     VolView V, float bx1, float by1, float bz1, const bf16x8* __restrict__ gpack, const float* __restrict__ gsmall,
     const float* __restrict__ ray_o, const float* __restrict__ ray_d, int64_t n, HybridParams hp,
     float* __restrict__ t_out, uint8_t* __restrict__ hit_out, int32_t* __restrict__ evals_out,
-    int32_t* __restrict__ samples_out) {
+    int32_t* __restrict__ samples_out, int32_t log_lanes) {
   __shared__ bf16x8 spack[USE_MLP ? (oPackB1 >> 3) : 1];
   __shared__ __align__(16) float ssmall[kSmall];
   __shared__ float slots[USE_MLP ? kSurrBlock / 64 : 1][4 * 64];  // per wave: x, y, z, result
-  if (USE_MLP) load_weights(gpack, gsmall, spack, ssmall, oPackB1 >> 3);
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t ic = i < n ? i : n - 1;
-  const f3 o{ray_o[3 * ic], ray_o[3 * ic + 1], ray_o[3 * ic + 2]};
-  const f3 d{ray_d[3 * ic], ray_d[3 * ic + 1], ray_d[3 * ic + 2]};
+  __shared__ uint32_t queue;  // the block's rays taken so far
+  if (USE_MLP) {
+    if (threadIdx.x == 0) queue = 0u;
+    load_weights(gpack, gsmall, spack, ssmall, oPackB1 >> 3);
+  }
   const float bmin[3] = {0.0f, 0.0f, 0.0f}, bmax[3] = {bx1, by1, bz1};
   if (!USE_MLP) {
     // Without the network: the exact-field march from the volume entry.
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
+      const f3 o{ray_o[3 * i], ray_o[3 * i + 1], ray_o[3 * i + 2]};
+      const f3 d{ray_d[3 * i], ray_d[3 * i + 1], ray_d[3 * i + 2]};
       float t;
       int32_t samples;
       const bool h = exact_march<NARROW>(V, bmin, bmax, o, d, hp.k_exact, hp.h_min, hp.n_bisect, hp.max_iters, t, samples);
@@ -789,62 +807,85 @@ __global__ void __launch_bounds__(512) hybrid_trace_kernel(
     }
     return;
   }
+  // The block's rays: every gridDim.x-th run of `lanes` from its own on.
+  const int lanes = 1 << log_lanes;
+  const int64_t runs = (n + lanes - 1) >> log_lanes;
+  const uint32_t total = (uint32_t)((runs - blockIdx.x + gridDim.x - 1) / gridDim.x) << log_lanes;
   enum { SURR = 0, EXACT = 1, DONE = 2 };
+  const int lane = threadIdx.x & 63;
   int phase = DONE;
-  bool hit = false;
+  bool hit = false, drained = false;  // drained: wave-uniform
+  int64_t ray = -1;
+  f3 o{0, 0, 0}, d{0, 0, 0};
   float t = 0.0f, t_far = 0.0f, f_prev = 0.0f, travel = 0.0f;
-  int32_t evals = 0, samples = 0;
-  float tn, tf;
-  if (i < n && ray_box(bmin, bmax, o, d, tn, tf)) {
-    t = tn;
-    t_far = tf;
-    phase = USE_MLP ? SURR : EXACT;
-    if (!USE_MLP) {
-      f_prev = trilinear<NARROW>(V, add(o, smul(t, d)));
-      ++samples;
-      if (f_prev <= 0.0f) { hit = true; phase = DONE; }
-    }
-  }
-  // A lane is advanced at most max_iters times (one network evaluation and/or
+  int32_t evals = 0, samples = 0, advances = 0;
+  // A ray is advanced at most max_iters times (one network evaluation and/or
   // one exact step per advance).  While some lane can take an exact step, the
   // network only runs full 16-point tiles of the waiting lanes (which ones is
   // rotated from iteration to iteration); when none can, it runs for all of
   // them.  A waiting lane keeps its state, so every ray takes the same steps
   // as when the network runs for every waiting lane at once, in fewer
-  // part-filled tiles.  Each wave iteration advances at least one lane, which
-  // bounds the loop.
-  int32_t advances = 0;
-  const int64_t wave_iters = 64ll * hp.max_iters;
+  // part-filled tiles.  Each wave iteration takes a ray, finds the queue empty
+  // or advances at least one lane, which bounds the loop.
 #pragma unroll 1
-  for (int64_t it = 0; it < wave_iters; ++it) {
+  for (uint32_t it = 0;; ++it) {
     if (phase != DONE && advances >= hp.max_iters) phase = DONE;
-    if (!__any(phase != DONE)) break;
+    const bool idle = phase == DONE;
+    const unsigned long long imask = __ballot(idle && lane < lanes);
+    const uint32_t want = (uint32_t)__popcll(imask);
+    if (!drained && 2 * want >= (uint32_t)lanes) {
+      if (idle && ray >= 0) {
+        t_out[ray] = hit ? t : kInf;
+        hit_out[ray] = hit ? 1 : 0;
+        if (evals_out) evals_out[ray] = evals;
+        if (samples_out) samples_out[ray] = samples;
+        ray = -1;
+      }
+      const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)atomicAdd(&queue, lane == 0 ? want : 0u));
+      drained = at + want >= total;
+      const uint32_t s = at + (uint32_t)__popcll(imask & ((1ull << lane) - 1ull));
+      const int64_t i = (((int64_t)blockIdx.x + (int64_t)(s >> log_lanes) * gridDim.x) << log_lanes) + (s & (uint32_t)(lanes - 1));
+      if (idle && lane < lanes && s < total && i < n) {
+        ray = i;
+        o = f3{ray_o[3 * i], ray_o[3 * i + 1], ray_o[3 * i + 2]};
+        d = f3{ray_d[3 * i], ray_d[3 * i + 1], ray_d[3 * i + 2]};
+        hit = false;
+        t = 0.0f;
+        evals = samples = advances = 0;
+        float tn, tf;
+        if (ray_box(bmin, bmax, o, d, tn, tf)) {
+          t = tn;
+          t_far = tf;
+          phase = SURR;
+        }
+      }
+      continue;
+    }
+    if (want == (uint32_t)lanes) break;  // and drained: an idle wave takes rays as long as there are some
     bool advanced = phase == EXACT;
-    if (USE_MLP) {
-      const bool wait = phase == SURR;
-      const unsigned long long wmask = __ballot(wait);
-      const int n_wait = __popcll(wmask);
-      const int n_run = __any(phase == EXACT) ? (n_wait & ~(kDeferTile - 1)) : n_wait;
-      if (n_run > 0) {
-        const int rank = __popcll(wmask & ((1ull << (threadIdx.x & 63)) - 1ull));
-        const bool need = wait && (rank + (int)((uint32_t)it % (uint32_t)n_wait)) % n_wait < n_run;
-        float* ws = slots[threadIdx.x >> 6];
-        const float s = wave_surrogate(spack, ssmall, add(o, smul(t, d)), need, ws, ws + 192);
-        if (need) {
-          advanced = true;
-          ++evals;
-          if (s > hp.tau) {
-            t += s - hp.margin;
-            if (t >= t_far) phase = DONE;
-          } else {
-            phase = EXACT;
-            travel = 0.0f;
-            f_prev = trilinear<NARROW>(V, add(o, smul(t, d)));
-            ++samples;
-            if (f_prev <= 0.0f) {
-              hit = true;  // entered the surface region already inside: accept the current point
-              phase = DONE;
-            }
+    const bool wait = phase == SURR;
+    const unsigned long long wmask = __ballot(wait);
+    const int n_wait = __popcll(wmask);
+    const int n_run = __any(phase == EXACT) ? (n_wait & ~(kDeferTile - 1)) : n_wait;
+    if (n_run > 0) {
+      const int rank = __popcll(wmask & ((1ull << lane) - 1ull));
+      const bool need = wait && (rank + (int)(it % (uint32_t)n_wait)) % n_wait < n_run;
+      float* ws = slots[threadIdx.x >> 6];
+      const float s = wave_surrogate(spack, ssmall, add(o, smul(t, d)), need, ws, ws + 192);
+      if (need) {
+        advanced = true;
+        ++evals;
+        if (s > hp.tau) {
+          t += s - hp.margin;
+          if (t >= t_far) phase = DONE;
+        } else {
+          phase = EXACT;
+          travel = 0.0f;
+          f_prev = trilinear<NARROW>(V, add(o, smul(t, d)));
+          ++samples;
+          if (f_prev <= 0.0f) {
+            hit = true;  // entered the surface region already inside: accept the current point
+            phase = DONE;
           }
         }
       }
@@ -870,16 +911,16 @@ __global__ void __launch_bounds__(512) hybrid_trace_kernel(
         f_prev = f_next;
         travel += h;
         if (t >= t_far) phase = DONE;
-        else if (USE_MLP && travel > hp.rejoin) phase = SURR;
+        else if (travel > hp.rejoin) phase = SURR;
       }
     }
     if (advanced) ++advances;
   }
-  if (i < n) {
-    t_out[i] = hit ? t : kInf;
-    hit_out[i] = hit ? 1 : 0;
-    if (evals_out) evals_out[i] = evals;
-    if (samples_out) samples_out[i] = samples;
+  if (ray >= 0) {
+    t_out[ray] = hit ? t : kInf;
+    hit_out[ray] = hit ? 1 : 0;
+    if (evals_out) evals_out[ray] = evals;
+    if (samples_out) samples_out[ray] = samples;
   }
 }
 
@@ -896,10 +937,17 @@ hipError_t launch_hybrid_trace(const DevVolume& field, const void* pack, const f
   // the scheduler's accounts, and marches differ many times in length (137 us
   // against 147 with blocks of 256 on 921,600 rays).
   const int block = use_mlp ? kSurrBlock : 64;
+  int64_t blocks = (n + block - 1) / block;
+  int32_t log_lanes = 6;
+  if (use_mlp) {
+    log_lanes = n <= 16 * kHybridRuns ? 4 : n <= 32 * kHybridRuns ? 5 : 6;
+    const int64_t runs = (n + (1 << log_lanes) - 1) >> log_lanes;
+    blocks = runs < kHybridBlocks ? runs : kHybridBlocks;
+  }
 #define RE_LAUNCH(MLP, NARROW)                                                                                     \
-  hipLaunchKernelGGL((hybrid_trace_kernel<MLP, NARROW>), dim3((unsigned)((n + block - 1) / block)), dim3(block), 0, s, \
+  hipLaunchKernelGGL((hybrid_trace_kernel<MLP, NARROW>), dim3((unsigned)blocks), dim3(block), 0, s,                \
                      V, field.box_max[0], field.box_max[1], field.box_max[2], (const bf16x8*)pack, small, ray_o,      \
-                     ray_d, n, hp, t, hit, evals, samples)
+                     ray_d, n, hp, t, hit, evals, samples, log_lanes)
   if (V.narrow) {
     if (use_mlp) RE_LAUNCH(true, true); else RE_LAUNCH(false, true);
   } else {
