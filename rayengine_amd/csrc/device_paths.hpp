@@ -145,15 +145,16 @@ __device__ __forceinline__ void load_ray(const float* __restrict__ ray_o, const 
 // the reference walks on to the cap.
 struct WalkMemo {
   int32_t c1 = kNoRope, c2 = kNoRope;  // cur is never kNoRope inside a walk
-  float e1 = 0.0f, e2 = 0.0f, x1 = 0.0f, x2 = 0.0f;
-  __device__ __forceinline__ bool repeats(int32_t cur, float te, float tx) {
-    if ((cur == c1 && te == e1 && tx == x1) || (cur == c2 && te == e2 && tx == x2)) return true;
+  float e1 = 0.0f, e2 = 0.0f;
+  // t_exit changes only when a hit is accepted (a hit has t < t_exit), which
+  // ends every earlier state's chance to come back: no t_exit is kept
+  __device__ __forceinline__ void hit() { c1 = c2 = kNoRope; }
+  __device__ __forceinline__ bool repeats(int32_t cur, float te) {
+    if ((cur == c1 && te == e1) || (cur == c2 && te == e2)) return true;
     c2 = c1;
     e2 = e1;
-    x2 = x1;
     c1 = cur;
     e1 = te;
-    x1 = tx;
     return false;
   }
 };
@@ -189,7 +190,7 @@ __device__ __forceinline__ void trace_ray(const NodeEntry* __restrict__ nodes, c
     bool have_window = false;
     WalkMemo memo;
     while (t_entry < t_exit && visits < cap) {
-      if (memo.repeats(cur, t_entry, t_exit)) break;
+      if (memo.repeats(cur, t_entry)) break;
       ++visits;
       const f3 pe = add(ro, smul(t_entry, rd));
       uint32_t leaf_id;
@@ -218,7 +219,9 @@ __device__ __forceinline__ void trace_ray(const NodeEntry* __restrict__ nodes, c
       const int32_t r = face >= 0 ? lp->rope[face] : kNoRope;
       have_window = r >= 0;
       if (have_window) w = load_window(nodes, r);
+      const float t_exit0 = t_exit;
       test_leaf<ONE_SIDED, COUNT, ANY>(tris + first, count, ro, rd, t_exit, found, hit_t, hit_prim, rc.tri);
+      if (t_exit != t_exit0) memo.hit();
       if (ANY && found) break;
       if (!box_ok) break;
       t_entry = tf;
@@ -293,7 +296,7 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
 template <bool ONE_SIDED, bool ANY = false>
 __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, bool at_leaf, uint32_t first,
                                                uint32_t cnt, f3 ro, f3 rd, float& t_exit, bool& found, float& hit_t,
-                                               uint32_t& hit_rec, CoopWave& W) {
+                                               uint32_t& hit_rec, WalkMemo& memo, CoopWave& W) {
   const int lane = threadIdx.x & 63;
   const unsigned long long at_mask = __ballot(at_leaf);
   const int lead = __ffsll((long long)at_mask) - 1;  // wave-uniform
@@ -325,6 +328,7 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
             hit_t = t;
             hit_rec = lead_first + base + j;
             t_exit = t;
+            memo.hit();
           }
         }
       }
@@ -405,6 +409,7 @@ __device__ __forceinline__ void coop_leaf_test(const TriRec* __restrict__ tris, 
       hit_t = __uint_as_float((uint32_t)(sv >> 32));
       hit_rec = (uint32_t)sv;
       t_exit = hit_t;
+      memo.hit();
     }
   }
 }
@@ -513,7 +518,7 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
     float tf = 0.0f;
     int32_t r = kNoRope;
     if (live) {
-      if (memo.repeats(cur, t_entry, t_exit)) {
+      if (memo.repeats(cur, t_entry)) {
         live = false;
       } else {
         ++visits;
@@ -544,7 +549,7 @@ __device__ __forceinline__ void coop_trace_wave(const NodeEntry* __restrict__ no
       }
     }
     if (__ballot(at_leaf) != 0ull) {
-      coop_leaf_test<ONE_SIDED, ANY>(tris, at_leaf, first, cnt, ro, rd, t_exit, found, hit_t, hit_rec, W);
+      coop_leaf_test<ONE_SIDED, ANY>(tris, at_leaf, first, cnt, ro, rd, t_exit, found, hit_t, hit_rec, memo, W);
       if (COUNT && at_leaf) rc.tri += cnt;
     }
     if (at_leaf) {
