@@ -191,13 +191,14 @@ enum Face { LEFT = 0, FRONT = 1, RIGHT = 2, BACK = 3, TOP = 4, BOTTOM = 5 };
 // plane lies within kEps of the exit point.
 // RayEngine/src/cuda-src/kd_tree_functions.cuh:31-62.  Returns -1 for none.
 RE_HD int exit_face(const float* bmin, const float* bmax, f3 p) {
-  if (fabsf(p.x - bmin[0]) < kEps) return LEFT;
-  if (fabsf(p.z - bmax[2]) < kEps) return FRONT;
-  if (fabsf(p.x - bmax[0]) < kEps) return RIGHT;
-  if (fabsf(p.z - bmin[2]) < kEps) return BACK;
-  if (fabsf(p.y - bmax[1]) < kEps) return TOP;
-  if (fabsf(p.y - bmin[1]) < kEps) return BOTTOM;
-  return -1;
+  int f = -1;  // the last test that holds wins: selects, no branches
+  if (fabsf(p.y - bmin[1]) < kEps) f = BOTTOM;
+  if (fabsf(p.y - bmax[1]) < kEps) f = TOP;
+  if (fabsf(p.z - bmin[2]) < kEps) f = BACK;
+  if (fabsf(p.x - bmax[0]) < kEps) f = RIGHT;
+  if (fabsf(p.z - bmax[2]) < kEps) f = FRONT;
+  if (fabsf(p.x - bmin[0]) < kEps) f = LEFT;
+  return f;
 }
 
 // ---------------------------------------------------------------------------
