@@ -150,6 +150,25 @@ inline int coop_lanes(int64_t n) {
   return lanes;
 }
 
+// Whether a ray's walks of the scene's objects get a lane each: they are then
+// side by side instead of one after another and their kernel is the one-object
+// one, without spills; but a lane whose object the ray misses stays empty, and
+// an any-hit ray walks all its objects.  Limits: three rounds of resident waves
+// (one for any-hit).  us, one after another / side by side, incoherent rays:
+// 3 objects of 6,670 triangles, 1,000 rays 170 / 90, 100,003 326 / 171, 300,000
+// 480 / 379; 8 apart, 40,000 253 / 125, 200,000 393 / 372, 300,000 442 / 525;
+// 30 apart, 10,000 242 / 63, 100,003 424 / 310, 200,000 532 / 575.  Any-hit:
+// 100,003 rays on 3 256 / 167, 300,000 330 / 366; 2 objects, 200,000 216 / 198,
+// 300,000 215 / 248.
+constexpr int64_t kSpreadWalks = 3 * 6144 * 64, kSpreadAnyWalks = 6144 * 64;
+inline bool trace_spreads(int64_t n, int32_t n_obj, int64_t most) {
+  return n_obj > 1 && n_obj <= 64 && n <= most / n_obj;
+}
+inline int spread_rays(int64_t n, int32_t n_obj) {
+  const int r = coop_lanes(n * n_obj) / n_obj;
+  return r > 1 ? r : 1;
+}
+
 // Whether variant 5 refills its waves, or is the plain cooperative kernel (the
 // same walks, one set of rays a wave).  Refill keeps lanes busy where walks are
 // long and uneven, and pays for it with a counter per 64 rays, a setup of 32

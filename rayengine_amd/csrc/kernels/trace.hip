@@ -223,40 +223,74 @@ __global__ void __launch_bounds__(256) trace_persistent_kernel(
   }
 }
 
+// The lanes of a wave over `rays` rays and, with SPREAD, their objects: lane
+// obj * rays + r walks object obj of the wave's ray r, so that a ray's walks
+// run side by side (they are independent of each other: each starts from its
+// object's box).
+template <bool SPREAD>
+__device__ __forceinline__ void coop_lane(int rays, int& r, int& obj) {
+  const int lane = (int)(threadIdx.x & 63);
+  obj = SPREAD ? lane / rays : 0;
+  r = lane - obj * rays;
+}
+
+// Lane r's value, taken from the walk of object k of its ray.
+template <typename T>
+__device__ __forceinline__ T of_walk(T v, int k, int rays) {
+  return __shfl(v, (int)(threadIdx.x & 63) + k * rays);
+}
+
 // Cooperative variant (see coop_trace_wave): one ray per lane, last block of
 // rays first, 6-wave register budget.
 // HINT (as in the refill kernel below): 1 takes each ray's walk-start leaf
 // from start_leaf (may be null), 2 also writes each ray's hit leaf.
-template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0>
+template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0, bool SPREAD = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int32_t* __restrict__ hit_leaf,
                   int64_t n_leaves, int32_t lanes) {
   // one CoopWave per wave of the block (dynamic LDS sized by the launch)
   extern __shared__ CoopWave waves[];
   CoopWave& wv = waves[threadIdx.x >> 6];
-  const int lane = (int)(threadIdx.x & 63);
+  int r, obj;
+  coop_lane<SPREAD>(lanes, r, obj);
   // `lanes` rays a wave, the last block of rays first
   const int64_t blk = (int64_t)(gridDim.x - 1 - blockIdx.x);
-  const int64_t i = (blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * lanes + lane;
-  const bool has_ray = lane < lanes && i < n;
+  const int64_t i = (blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * lanes + r;
+  const bool has_ray = (SPREAD ? obj < n_obj : r < lanes) && i < n;
   const auto ray = [&](f3& o, f3& d) { load_ray(ray_o, ray_d, i, o, d); };
   float best_t;
   int32_t best_prim, best_obj;
   RayCounts rc;
   const int32_t hint = (HINT != 0 && start_leaf && has_ray) ? start_leaf[i] : -1;
   int32_t best_leaf = -1;
-  coop_trace_wave<COUNT, ONE_SIDED, ONE_OBJ, HINT>(nodes, leaves, tris, objs, 0, ONE_OBJ ? 1 : n_obj, has_ray, ray,
+  coop_trace_wave<COUNT, ONE_SIDED, ONE_OBJ, HINT>(nodes, leaves, tris, objs, obj, ONE_OBJ ? 1 : n_obj, has_ray, ray,
                                                    cap, secondary != 0, best_t, best_prim, best_obj, rc, wv, hint,
                                                    n_leaves, &best_leaf);
-  if (has_ray) {
+  if (COUNT && has_ray) {
+    atomicAdd(&counts->entries, (unsigned long long)rc.ent);
+    atomicAdd(&counts->leaves, (unsigned long long)rc.leaf);
+    atomicAdd(&counts->tris, (unsigned long long)rc.tri);
+  }
+  if (SPREAD) {
+    // the objects in order, each taken only when strictly closer
+    for (int k = 1; k < n_obj; ++k) {
+      const float t = of_walk(best_t, k, lanes);
+      const int32_t p = of_walk(best_prim, k, lanes), o = of_walk(best_obj, k, lanes);
+      const int32_t lf = HINT == 2 ? of_walk(best_leaf, k, lanes) : 0;
+      if (obj == 0 && t < best_t) {
+        best_t = t;
+        best_prim = p;
+        best_obj = o;
+        best_leaf = lf;
+      }
+    }
+  }
+  if (has_ray && obj == 0) {
     prim_out[i] = best_prim;
     t_out[i] = best_t;
     if (obj_out) obj_out[i] = best_obj;
     if (HINT == 2) hit_leaf[i] = best_leaf;
     if (COUNT) {
-      atomicAdd(&counts->entries, (unsigned long long)rc.ent);
-      atomicAdd(&counts->leaves, (unsigned long long)rc.leaf);
-      atomicAdd(&counts->tris, (unsigned long long)rc.tri);
       if (best_prim >= 0) atomicAdd(&counts->rays_hit, 1ull);
     }
   }
@@ -268,7 +302,7 @@ trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int
 // clustered triangles 199 / 254, on 50,021 137 / 140, on 6,144 124 / 127;
 // 16,000 on 50,021 77 / 94.  (126,450 to 262,440 on 6,144 triangles, whose
 // waves stay together: 4 % slower, 83 / 81 and 103 / 100.)
-template <bool ONE_SIDED, bool ONE_OBJ>
+template <bool ONE_SIDED, bool ONE_OBJ, bool SPREAD = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 trace_occluded_kernel(const NodeEntry* __restrict__ nodes, const DevLeaf* __restrict__ leaves,
                       const TriRec* __restrict__ tris, const ObjXform* __restrict__ objs, int32_t n_obj,
@@ -276,18 +310,29 @@ trace_occluded_kernel(const NodeEntry* __restrict__ nodes, const DevLeaf* __rest
                       int32_t secondary, uint8_t* __restrict__ occluded, int32_t lanes) {
   extern __shared__ CoopWave waves[];
   CoopWave& wv = waves[threadIdx.x >> 6];
-  const int lane = (int)(threadIdx.x & 63);
+  int r, obj;
+  coop_lane<SPREAD>(lanes, r, obj);
   // the wave's first ray is a scalar, which leaves the kernel 72 registers
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t i = ((int64_t)(gridDim.x - 1 - blockIdx.x) * (blockDim.x >> 6) + w) * lanes + lane;
-  const bool has_ray = lane < lanes && i < n;
+  const int64_t i = ((int64_t)(gridDim.x - 1 - blockIdx.x) * (blockDim.x >> 6) + w) * lanes + r;
+  const bool has_ray = (SPREAD ? obj < n_obj : r < lanes) && i < n;
   const auto ray = [&](f3& o, f3& d) { load_ray(ray_o, ray_d, i, o, d); };
   float best_t;
   int32_t best_prim, best_obj;
   RayCounts rc;
-  coop_trace_wave<false, ONE_SIDED, ONE_OBJ, 0, true>(nodes, leaves, tris, objs, 0, ONE_OBJ ? 1 : n_obj, has_ray,
+  coop_trace_wave<false, ONE_SIDED, ONE_OBJ, 0, true>(nodes, leaves, tris, objs, obj, ONE_OBJ ? 1 : n_obj, has_ray,
                                                       ray, cap, secondary != 0, best_t, best_prim, best_obj, rc, wv);
-  if (has_ray) occluded[i] = best_prim >= 0 ? 1 : 0;
+  if (SPREAD) {
+    // the first object that detects a hit
+    for (int k = 1; k < n_obj; ++k) {
+      const int32_t p = of_walk(best_prim, k, lanes), o = of_walk(best_obj, k, lanes);
+      if (obj == 0 && best_obj < 0 && o >= 0) {
+        best_prim = p;
+        best_obj = o;
+      }
+    }
+  }
+  if (has_ray && obj == 0) occluded[i] = best_prim >= 0 ? 1 : 0;
 }
 
 // Cooperative variant with refill (variant 5): persistent waves; once at
@@ -840,7 +885,8 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
 #undef RE_LAUNCH
     return hipGetLastError();
   }
-  const int lanes = coop ? coop_lanes(L.n) : 64;
+  const bool spread = coop && trace_spreads(L.n, S.n_obj, kSpreadWalks);
+  const int lanes = spread ? spread_rays(L.n, S.n_obj) : coop ? coop_lanes(L.n) : 64;
   const int64_t per_block = (int64_t)(block / 64) * lanes;
   const int64_t grid = (L.n + per_block - 1) / per_block;
 #define RE_LAUNCH(K, ...)                                                                                       \
@@ -859,7 +905,12 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
   if (coop) {
     const int hint = L.hit_leaf ? 2 : (L.start_leaf ? 1 : 0);
 #define RE_LAUNCH_COOP_H(C, O, ONE, H)                                                                        \
-  hipLaunchKernelGGL((trace_coop_kernel<C, O, ONE, H>), dim3((unsigned)grid), dim3(block),                    \
+  do {                                                                                                        \
+    if (spread) RE_LAUNCH_COOP_S(C, O, true, H, !ONE);                                                        \
+    else RE_LAUNCH_COOP_S(C, O, ONE, H, false);                                                               \
+  } while (0)
+#define RE_LAUNCH_COOP_S(C, O, ONE, H, S_)                                                                    \
+  hipLaunchKernelGGL((trace_coop_kernel<C, O, ONE, H, S_>), dim3((unsigned)grid), dim3(block),                    \
                      (block / 64) * sizeof(CoopWave), s, S.nodes, S.leaves,                                      \
                      S.tris, S.objs, S.n_obj, L.ray_o, L.ray_d, L.n, cap, L.secondary, L.prim, L.t, L.obj,        \
                      L.counts, L.start_leaf, L.hit_leaf, S.n_leaves, lanes)
@@ -879,6 +930,7 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
     }
 #undef RE_LAUNCH_COOP
 #undef RE_LAUNCH_COOP_H
+#undef RE_LAUNCH_COOP_S
   } else if (L.variant == 2) RE_LAUNCH_ALL(trace_closest_kernel, , true);
   else if (L.variant == 3 && S.n_obj == 1) RE_LAUNCH_ALL(trace_closest_o6_kernel, , true);
   else if (L.variant == 3) RE_LAUNCH_ALL(trace_closest_o6_kernel, , false);
@@ -897,17 +949,24 @@ hipError_t launch_trace_occluded(const TraceLaunch& L, hipStream_t s) {
   const int block = L.block > 0 ? L.block : 64;
   const DevScene& S = *L.scene;
   const int32_t cap = (L.cap > 0 && L.cap < kMaxLeafVisits) ? L.cap : kMaxLeafVisits;
-  const int lanes = coop_lanes(L.n);
+  const bool spread = trace_spreads(L.n, S.n_obj, kSpreadAnyWalks);
+  const int lanes = spread ? spread_rays(L.n, S.n_obj) : coop_lanes(L.n);
   const int64_t per_block = (int64_t)(block / 64) * lanes;
   const int64_t grid = (L.n + per_block - 1) / per_block;
 #define RE_LAUNCH_OCCLUDED(O, ONE)                                                                            \
-  hipLaunchKernelGGL((trace_occluded_kernel<O, ONE>), dim3((unsigned)grid), dim3(block),                      \
+  do {                                                                                                        \
+    if (spread) RE_LAUNCH_OCCLUDED_S(O, true, !ONE);                                                          \
+    else RE_LAUNCH_OCCLUDED_S(O, ONE, false);                                                                 \
+  } while (0)
+#define RE_LAUNCH_OCCLUDED_S(O, ONE, S_)                                                                      \
+  hipLaunchKernelGGL((trace_occluded_kernel<O, ONE, S_>), dim3((unsigned)grid), dim3(block),                      \
                      (block / 64) * sizeof(CoopWave), s, S.nodes, S.leaves, S.tris, S.objs, S.n_obj, L.ray_o, \
                      L.ray_d, L.n, cap, L.secondary, L.occluded, lanes)
   const bool one = S.n_obj == 1;
   if (L.one_sided) { if (one) RE_LAUNCH_OCCLUDED(true, true); else RE_LAUNCH_OCCLUDED(true, false); }
   else { if (one) RE_LAUNCH_OCCLUDED(false, true); else RE_LAUNCH_OCCLUDED(false, false); }
 #undef RE_LAUNCH_OCCLUDED
+#undef RE_LAUNCH_OCCLUDED_S
   return hipGetLastError();
 }
 
