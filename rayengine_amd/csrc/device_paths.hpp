@@ -54,16 +54,13 @@ __device__ __forceinline__ TriGeom load_geom(const TriRec* __restrict__ tp, uint
 // before any of them is tested, so a lane has four independent loads in
 // flight instead of one; the prim id is read only for an accepted hit.
 //
-// ANY: stop at the first accepted hit (any-hit query; the reference's
-// intersection_detected becomes true there and never reverts).
 // BATCH records are loaded per round (4 by default; fewer where registers
 // are short).
-template <bool ONE_SIDED, bool COUNT, bool ANY = false, int BATCH = 4>
+template <bool ONE_SIDED, bool COUNT, int BATCH = 4>
 __device__ __forceinline__ void test_leaf(const TriRec* __restrict__ tp, uint32_t count, f3 ro, f3 rd,
                                           float& t_exit, bool& found, float& hit_t, int32_t& hit_prim,
                                           unsigned& c_tri) {
   for (uint32_t j = 0; j < count; j += BATCH) {
-    if (ANY && found) return;
     TriGeom g[BATCH];
 #pragma unroll
     for (int q = 0; q < BATCH; ++q)
@@ -80,7 +77,6 @@ __device__ __forceinline__ void test_leaf(const TriRec* __restrict__ tp, uint32_
         hit_t = t;
         hit_prim = tp[j + q].prim;
         t_exit = t;
-        if (ANY) break;
       }
     }
   }
@@ -160,12 +156,8 @@ struct WalkMemo {
 };
 
 // Closest hit of one ray over objects [k0, k1): stackless_kdtree_traversal and
-// trace_scene, RayEngine/src/cuda-src/ray_functions.cuh:230-396.  With ANY the
-// walk of an object stops at its first accepted hit and the objects after the
-// first that reports one are skipped: best_prim >= 0 then says whether any
-// object detects an intersection, which is all trace_shadow
-// (ray_functions.cuh:365-374) delivers to its callers.
-template <bool COUNT, bool ONE_SIDED, bool ANY = false>
+// trace_scene, RayEngine/src/cuda-src/ray_functions.cuh:230-396.
+template <bool COUNT, bool ONE_SIDED>
 __device__ __forceinline__ void trace_ray(const NodeEntry* __restrict__ nodes, const DevLeaf* __restrict__ leaves,
                                           const TriRec* __restrict__ tris, const ObjXform* __restrict__ objs,
                                           int32_t k0, int32_t k1, f3 o, f3 d, int32_t cap, bool secondary,
@@ -220,9 +212,8 @@ __device__ __forceinline__ void trace_ray(const NodeEntry* __restrict__ nodes, c
       have_window = r >= 0;
       if (have_window) w = load_window(nodes, r);
       const float t_exit0 = t_exit;
-      test_leaf<ONE_SIDED, COUNT, ANY>(tris + first, count, ro, rd, t_exit, found, hit_t, hit_prim, rc.tri);
+      test_leaf<ONE_SIDED, COUNT>(tris + first, count, ro, rd, t_exit, found, hit_t, hit_prim, rc.tri);
       if (t_exit != t_exit0) memo.hit();
-      if (ANY && found) break;
       if (!box_ok) break;
       t_entry = tf;
       if (r == kNoRope) break;
@@ -233,7 +224,6 @@ __device__ __forceinline__ void trace_ray(const NodeEntry* __restrict__ nodes, c
       best_prim = hit_prim;
       best_obj = k;
     }
-    if (ANY && found) return;
   }
 }
 
@@ -447,7 +437,10 @@ __device__ __forceinline__ int32_t hinted_start(const DevLeaf* __restrict__ leav
 // part in the wave's work without a ray of their own.  Results are
 // bit-identical to trace_ray's.  Every lane of the wave must call it (it
 // holds wave-wide operations); the loop ends on a wave-uniform branch.
-// With ANY (as in trace_ray) a lane is done at its first accepted hit.
+// With ANY a walk stops at its first accepted hit and the objects after the
+// first that reports one are skipped: best_prim >= 0 then says whether any object
+// detects an intersection, which is all trace_shadow
+// (RayEngine/src/cuda-src/ray_functions.cuh:365-374) delivers to its callers.
 // ray(o, d) reads the lane's ray: once per object, so that with several
 // objects the untransformed ray holds no registers during a walk.
 template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0, bool ANY = false, class Ray>
