@@ -138,11 +138,11 @@ inline int trace_launch_block(int block, int variant) { return block > 0 ? block
 // waves stay resident.  The limit is three quarters of the 6144 waves that
 // 256 CUs hold at 6 per SIMD.
 // us for 64 / 32 / 16 / 8 rays a wave, camera rays on 2^20 clustered triangles:
-// 4,096 rays 182 / 146 / 131 / 123; 72,720 rays 242 / 181 / 170 / 192;
-// 140,500 rays 255 / 199 / 182 / 239.  Incoherent rays on 20,000 triangles:
-// 4,096 rays 124 / 108 / 103 / 99; 72,720 rays 173 / 162 / 162 / 200;
-// 140,500 rays 190 / 173 / 223 / 289; 200,000 rays 196 / 223 / 277 / 364.
-// (4 rays a wave: within 3 % of 8 up to 17,600 rays, slower above.)
+// 4,096 rays 162 / 134 / 119 / 116; 72,720 rays 220 / 174 / 173 / 205;
+// 140,500 rays 231 / 181 / 173 / 232.  Incoherent rays on 20,000 triangles:
+// 4,096 rays 144 / 132 / 129 / 119; 72,720 rays 165 / 153 / 152 / 186;
+// 140,500 rays 174 / 164 / 204 / 265; 200,000 rays 187 / 216 / 261 / 352.
+// (4 rays a wave: within 5 % of 8 at 4,096 rays, slower above.)
 constexpr int64_t kCoopFillWaves = 4608;
 inline int coop_lanes(int64_t n) {
   int lanes = 8;
@@ -155,11 +155,11 @@ inline int coop_lanes(int64_t n) {
 // one, without spills; but a lane whose object the ray misses stays empty, and
 // an any-hit ray walks all its objects.  Limits: three rounds of resident waves
 // (one for any-hit).  us, one after another / side by side, incoherent rays:
-// 3 objects of 6,670 triangles, 1,000 rays 170 / 90, 100,003 326 / 171, 300,000
-// 480 / 379; 8 apart, 40,000 253 / 125, 200,000 393 / 372, 300,000 442 / 525;
-// 30 apart, 10,000 242 / 63, 100,003 424 / 310, 200,000 532 / 575.  Any-hit:
-// 100,003 rays on 3 256 / 167, 300,000 330 / 366; 2 objects, 200,000 216 / 198,
-// 300,000 215 / 248.
+// 3 objects of 6,670 triangles, 1,000 rays 176 / 89, 100,003 328 / 170, 300,000
+// 472 / 380; 8 apart, 40,000 249 / 125, 200,000 391 / 374, 300,000 441 / 528;
+// 30 apart, 10,000 245 / 63, 100,003 421 / 309, 200,000 531 / 573.  Any-hit:
+// 100,003 rays on 3 259 / 165, 300,000 327 / 366; 2 objects, 200,000 215 / 195,
+// 300,000 214 / 248.
 constexpr int64_t kSpreadWalks = 3 * 6144 * 64, kSpreadAnyWalks = 6144 * 64;
 inline bool trace_spreads(int64_t n, int32_t n_obj, int64_t most) {
   return n_obj > 1 && n_obj <= 64 && n <= most / n_obj;
@@ -175,10 +175,10 @@ inline int spread_rays(int64_t n, int32_t n_obj) {
 // rays at a time and waves whose halves are apart.  It is ahead once a launch
 // has two rounds of resident waves (256 CUs x 24) and the scene 10^5 triangle
 // records.  us, refill / plain, diffuse bounces: 2,919,928 records, 207,360
-// rays 245 / 224, 507,206 398 / 368, 829,440 463 / 485, 1,866,240 768 / 899;
-// 157,048 records, 829,440 rays 391 / 366, 3,317,760 1054 / 1093; 68,589
-// records, 207,360 rays 165 / 131, 829,440 322 / 270, 3,317,760 852 / 785;
-// 17,832 records, 1,866,240 rays 354 / 283.
+// rays 231 / 205, 507,206 358 / 342, 829,440 437 / 457, 1,866,240 722 / 846;
+// 157,048 records, 829,440 rays 369 / 345, 3,317,760 943 / 1035; 68,589
+// records, 207,360 rays 158 / 126, 829,440 305 / 258, 3,317,760 773 / 748;
+// 17,832 records, 1,866,240 rays 343 / 269.
 constexpr int64_t kRefillRays = 2 * 6144 * 64, kRefillRecs = 100000;
 inline bool trace_refills(int variant, int64_t n, int64_t n_trirecs) {
   return variant == 5 && n > kRefillRays && n_trirecs > kRefillRecs;

@@ -299,9 +299,9 @@ trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int
 // Any-hit query (trace_shadow, RayEngine/src/cuda-src/ray_functions.cuh:365-374):
 // the cooperative walk, each ray done at its first accepted hit.  us against
 // one ray per lane with its own leaf tests: 507,206 shadow rays on 2^20
-// clustered triangles 199 / 254, on 50,021 137 / 140, on 6,144 124 / 127;
-// 16,000 on 50,021 77 / 94.  (126,450 to 262,440 on 6,144 triangles, whose
-// waves stay together: 4 % slower, 83 / 81 and 103 / 100.)
+// clustered triangles 186 / 254, on 50,021 128 / 140, on 6,144 113 / 127;
+// 15,840 on 50,021 68 / 94; 126,450 on 6,144, whose waves stay together, 80 /
+// 81.
 template <bool ONE_SIDED, bool ONE_OBJ, bool SPREAD = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 trace_occluded_kernel(const NodeEntry* __restrict__ nodes, const DevLeaf* __restrict__ leaves,
