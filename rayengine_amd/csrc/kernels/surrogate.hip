@@ -215,12 +215,24 @@ __global__ void __launch_bounds__(512) mlp_infer_kernel(const bf16x8* __restrict
 // layer) is what leaves the LDS room for eight waves beside the 64 KB of
 // operands; with four waves and every layer staged at once a SIMD ran one wave
 // and stood still through its chains of LDS reads, MFMAs and exponentials:
-// 38.5 us per launch of 65,536 points, now 31.9.
+// 38.5 us per launch of 65,536 points, now 30.8.
 //
 // Additions keep the order of one chunk after the other: K runs over the first
 // chunk's points, then the second's, and the output layer's per-lane sums of
 // both chunks are kept by one half (neurons m = 0, 1 by the first, 2, 3 by the
 // second), which the other hands its products through LDS (exchange).
+//
+// A round of the loop has four barriers, B3 to B0, one per layer.  What lies
+// between the last access of one use of an LDS area and the first of the next:
+//   dz1, in1          staged for layer 3 before B3, read after it     B2
+//                     staged for layer 1 before B1, read after it     B0
+//   dz0, in0[0..63]   staged for layer 2 before B2, read after it     B1
+//                     staged for layer 0 before B0, read after it     B3 of the next round
+//   in0[64..], tail   exchange written after B3, read after B2        B1
+//                     staged for layer 0 before B0, read after it     B3 of the next round
+// (A wave in the next round passes B3 only when every wave has left layer 0 of
+// this one, so the exchange must not be written before B3.)  After the loop the
+// final sums are written to dz1, whose last readers are behind B0.
 constexpr int kChunkPts = 64;
 constexpr int kPairPts = 2 * kChunkPts;
 // Staged rows are padded by 16 bytes (136 bf16): the 16 rows of one MFMA operand
@@ -265,8 +277,7 @@ __global__ void __launch_bounds__(kTrainBlock) mlp_train_kernel(const bf16x8* __
   const int mi = wv >> 1, odd = wv & 1;  // result tiles: rows 16 mi, and the even or odd wave's columns
   const float inv_b = 1.0f / (float)batch;
   const int n_chunks = batch / kChunkPts;
-  // Rows of lane values; they overlap rows of in0 that only layer 0 stages, two
-  // barriers after they are read.
+  // Rows of lane values, over rows of in0 that only layer 0 stages
   float* const exchange = reinterpret_cast<float*>(&S.in0[kH][0]);
   const int xl = threadIdx.x & (kHalfThreads - 1);
 
@@ -317,25 +328,22 @@ __global__ void __launch_bounds__(kTrainBlock) mlp_train_kernel(const bf16x8* __
       if (next < n_chunks) smp_next = samples[train_sample_index(batch_start, next, p_local, n_samples)];
     }
     TileAct T;
-    float dz[4][4], own[8];
+    float dz[4][4], own[8], give[8], dout = 0.0f, l = 0.0f;
     if (have) {
       bf16x8 xb[4];
       features(f3{smp.x, smp.y, smp.z}, g, xb);
       const float o = forward_tile<true>(S.pack, S.small, xb, lane, T);
       const float r = o - smp.w;
       const float wgt = r > 0.0f ? over_weight : 1.0f;
-      const float dout = 2.0f * wgt * r * inv_b;
-      const float l = wgt * r * r * inv_b;
+      dout = 2.0f * wgt * r * inv_b;
+      l = wgt * r * r * inv_b;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const float lo = dout * T.h3[q >> 2][q & 3], hi = dout * T.h3[2 + (q >> 2)][q & 3];
         own[q] = half ? hi : lo;
-        exchange[(8 * half + q) * kHalfThreads + xl] = half ? lo : hi;
+        give[q] = half ? lo : hi;
       }
-      if (half == 1) {
-        exchange[16 * kHalfThreads + xl] = dout;
-        exchange[17 * kHalfThreads + xl] = l;
-      } else if (g == 0) {
+      if (half == 0 && g == 0) {
         loss += l;
         db4r += dout;
       }
@@ -376,10 +384,16 @@ __global__ void __launch_bounds__(kTrainBlock) mlp_train_kernel(const bf16x8* __
           }
         }
       }
-      // The layer is staged; the other buffer's readers are done with it once
-      // every wave has passed here, so it may be written after.
-      __syncthreads();
-      if (L == 3) {
+      __syncthreads();  // barrier L of the table above
+      if (L == 3 && have) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) exchange[(8 * half + q) * kHalfThreads + xl] = give[q];
+        if (half == 1) {
+          exchange[16 * kHalfThreads + xl] = dout;
+          exchange[17 * kHalfThreads + xl] = l;
+        }
+      }
+      if (L == 2) {
         // the first chunk's products, then the second's
         if (half == 0) {
 #pragma unroll
