@@ -64,21 +64,53 @@ constexpr int kMaxBins = 64;
 constexpr int kBinChunk = 1024;
 constexpr int kWaveBinMax = kBinChunk;
 
-// Device and pinned host memory that a context keeps between its device
-// builds: one chunk of what the last build took, at most kKeepBytes, and the
-// words a level's totals are written to.  A build that needs more takes and
-// frees the rest itself.
-constexpr size_t kKeepBytes = (size_t)256 << 20;
-struct Workspace {
-  char* chunk = nullptr;
-  size_t bytes = 0;
-  int64_t* totals = nullptr;  // pinned, 4 words
-};
-
 RE_HD int32_t mode_of(int32_t n, int32_t depth, const Params& P) {
   if (n <= P.max_leaf || depth >= P.max_depth) return kModeLeaf;
   return n <= kExactMax ? kModeExact : (n <= kWaveBinMax ? kModeBinned : kModeBig);
 }
+
+// What a node adds to the next level and to the leaf pool, scanned together:
+// next-level references, leaf-pool references, next-level nodes; and, in
+// `last`, the largest leaf in the low 31 bits, with bit 31 set when a
+// next-level node is to be binned by bin_count_kernel (their maximum and or).
+// The references are summed in 64 bits: a reference that straddles a plane
+// counts twice, so a level of 2^31 - 1 may ask for twice as many.
+struct Adds {
+  int64_t refs, leaf;
+  int32_t kids;
+  uint32_t last;
+};
+constexpr uint32_t kBigBit = 0x80000000u;
+struct AddsSum {
+  RE_HD Adds operator()(const Adds& a, const Adds& b) const {
+    const uint32_t m = a.last & ~kBigBit, n = b.last & ~kBigBit;
+    return Adds{a.refs + b.refs, a.leaf + b.leaf, a.kids + b.kids, ((a.last | b.last) & kBigBit) | (m > n ? m : n)};
+  }
+};
+// Of a node whose split is decided.
+RE_HD Adds node_adds(const LNode& nd, const Params& P) {
+  if (!nd.split) return Adds{0, nd.n, 0, (uint32_t)nd.n};
+  const bool big = mode_of(nd.cl, nd.depth + 1, P) == kModeBig || mode_of(nd.cr, nd.depth + 1, P) == kModeBig;
+  return Adds{(int64_t)nd.cl + nd.cr, 0, 2, big ? kBigBit : 0u};
+}
+
+// Whether the level after one with `nodes` tree nodes up to its end and
+// `records` leaf-pool references up to its end can be built: node indices have
+// 30 bits, references and triangle records are indexed with 31.
+inline bool level_fits(int64_t nodes, int64_t records, const Adds& total) {
+  return nodes + total.kids <= (int64_t)0x3fffffff && total.refs <= (int64_t)0x7fffffff &&
+         records + total.leaf <= (int64_t)0x7fffffff;
+}
+
+// Device and pinned host memory that a context keeps between its device
+// builds: one chunk of what the last build took, at most kKeepBytes, and the
+// totals of a level.  A build that needs more takes and frees the rest itself.
+constexpr size_t kKeepBytes = (size_t)256 << 20;
+struct Workspace {
+  char* chunk = nullptr;
+  size_t bytes = 0;
+  Adds* totals = nullptr;  // pinned
+};
 
 }  // namespace kdb
 }  // namespace re

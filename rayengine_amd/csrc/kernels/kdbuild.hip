@@ -537,22 +537,6 @@ __global__ void __launch_bounds__(64) part_clip_kernel(const float* __restrict__
   }
 }
 
-// What a node adds to the next level and to the leaf pool, scanned together:
-// next-level nodes, next-level references, leaf-pool references; and, in
-// `last`, the largest leaf in the low 31 bits, with bit 31 set when a
-// next-level node is to be binned by bin_count_kernel (their maximum and or).
-struct Adds {
-  int32_t kids, refs, leaf;
-  uint32_t last;
-};
-constexpr uint32_t kBigBit = 0x80000000u;
-struct AddsSum {
-  __host__ __device__ Adds operator()(const Adds& a, const Adds& b) const {
-    return Adds{a.kids + b.kids, a.refs + b.refs, a.leaf + b.leaf,
-                ((a.last | b.last) & kBigBit) | max(a.last & ~kBigBit, b.last & ~kBigBit)};
-  }
-};
-
 // The split decision of every node, its below and above counts taken from
 // the scan of its references' flags (flags_x exclusive; a node's references
 // are contiguous).
@@ -568,24 +552,15 @@ __global__ void decide_kernel(LNode* __restrict__ nodes, int32_t nn, const uint6
     nd.cr = (int32_t)(c >> 32);
   }
   nd.split = (will_try(nd) && !(nd.cl == nd.n && nd.cr == nd.n)) ? 1 : 0;
-  Adds a{0, 0, nd.n, (uint32_t)nd.n};
-  if (nd.split) {
-    const bool big = mode_of(nd.cl, nd.depth + 1, P) == kModeBig || mode_of(nd.cr, nd.depth + 1, P) == kModeBig;
-    a = Adds{2, nd.cl + nd.cr, 0, big ? kBigBit : 0u};
-  }
-  adds[i] = a;
+  adds[i] = node_adds(nd, P);
 }
 
 // Totals of the scan over a level's nodes, to pinned host memory (read after
 // the stream's synchronisation); the straddler list starts empty again for
 // the next level.
-__global__ void totals_kernel(const Adds* adds, const Adds* adds_x, int64_t nn, int64_t* out, int32_t* n_strad) {
+__global__ void totals_kernel(const Adds* adds, const Adds* adds_x, int64_t nn, Adds* out, int32_t* n_strad) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
-    const Adds a = AddsSum{}(adds_x[nn - 1], adds[nn - 1]);
-    out[0] = a.kids;
-    out[1] = a.refs;
-    out[2] = a.leaf;
-    out[3] = a.last;
+    *out = AddsSum{}(adds_x[nn - 1], adds[nn - 1]);
     *n_strad = 0;
   }
 }
@@ -711,9 +686,9 @@ __global__ void preorder_kernel(const GNode* __restrict__ gn, int32_t g0, int32_
   else if (n.axis == 1) { sl = 5; sr = 4; }
   else { sl = 3; sr = 1; }
   for (int f = 0; f < 6; ++f) {
-    const int r = ropes[6 * g + f];
-    ropes[6 * c0 + f] = f == sr ? c1 : r;
-    ropes[6 * c1 + f] = f == sl ? c0 : r;
+    const int r = ropes[6 * (int64_t)g + f];
+    ropes[6 * (int64_t)c0 + f] = f == sr ? c1 : r;
+    ropes[6 * (int64_t)c1 + f] = f == sl ? c0 : r;
   }
 }
 
@@ -938,7 +913,7 @@ hipError_t build_device(const float* tri_v, int64_t n, float* root_min, float* r
                         const Params& P, Workspace& ws, hipStream_t s, RecVec<NodeEntry>& out_nodes,
                         RecVec<LeafRec>& out_leaves, RecVec<TriRec>& out_tris, int32_t& depth,
                         int32_t& max_leaf, float& device_ms) {
-  if (!ws.totals) KDB_TRY(hipHostMalloc((void**)&ws.totals, 4 * sizeof(int64_t), hipHostMallocDefault));
+  if (!ws.totals) KDB_TRY(hipHostMalloc((void**)&ws.totals, sizeof(Adds), hipHostMallocDefault));
   Bufs B(ws, s);
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   KDB_TRY(hipEventCreate(&ev0));
@@ -1039,15 +1014,15 @@ hipError_t build_device(const float* tri_v, int64_t n, float* root_min, float* r
     hipLaunchKernelGGL(decide_kernel, dim3(blocks(nn, 256)), dim3(256), 0, s, lv.p, (int32_t)nn, flags.p, flags_x.p,
                        P, adds.p);
     KDB_TRY(hipGetLastError());
-    KDB_TRY(scan.run(B, adds.p, adds_x.p, nn, s, AddsSum{}, Adds{0, 0, 0, 0}));
+    KDB_TRY(scan.run(B, adds.p, adds_x.p, nn, s, AddsSum{}, Adds{0, 0, 0, 0u}));
     hipLaunchKernelGGL(totals_kernel, dim3(1), dim3(64), 0, s, adds.p, adds_x.p, nn, ws.totals, n_strad);
     KDB_TRY(hipGetLastError());
     KDB_TRY(hipStreamSynchronize(s));
-    const int64_t* t4 = ws.totals;
-    const int64_t n_next = t4[0], r_next = t4[1], l_now = t4[2];
-    any_big = (t4[3] & kBigBit) != 0;
-    max_leaf = std::max(max_leaf, (int32_t)(t4[3] & ~(int64_t)kBigBit));
-    if (gbase + nn + n_next > (int64_t)0x3fffffff || r_next > (int64_t)0x7fffffff) return hipErrorInvalidValue;
+    const Adds sum = *ws.totals;
+    const int64_t n_next = sum.kids, r_next = sum.refs, l_now = sum.leaf;
+    any_big = (sum.last & kBigBit) != 0;
+    max_leaf = std::max(max_leaf, (int32_t)(sum.last & ~kBigBit));
+    if (!level_fits(gbase + nn, pused, sum)) return hipErrorInvalidValue;
 
     KDB_TRY(gn.ensure(B, gused + n_next, s, gused));
     KDB_TRY(pool.ensure(B, pused + l_now, s, pused));
@@ -1080,7 +1055,7 @@ hipError_t build_device(const float* tri_v, int64_t n, float* root_min, float* r
   KDB_TRY(B.alloc(&nleaf, (size_t)total));
   KDB_TRY(B.alloc(&entry, (size_t)total));
   KDB_TRY(B.alloc(&lbase, (size_t)total));
-  KDB_TRY(B.alloc(&ropes, (size_t)(6 * total)));
+  KDB_TRY(B.alloc(&ropes, 6 * (size_t)total));
   for (auto it = levels.rbegin(); it != levels.rend(); ++it)
     hipLaunchKernelGGL(sizes_kernel, dim3(blocks(it->second, 256)), dim3(256), 0, s, gn.p, it->first, it->second,
                        size, nleaf);
