@@ -43,16 +43,16 @@ struct DevScene {
 
 // One object's tree records inside a scene's arrays, copied as the builder
 // left them, and their place: the bases are the counts of the records before
-// them (kernels/scene.hip).
+// them, first_block the blocks of the placing kernel before its own
+// (kernels/scene.hip).
 struct ScenePlace {
-  NodeEntry* nodes;
-  DevLeaf* leaves;  // LeafRec records until placed
-  TriRec* tris;
-  int64_t n_nodes, n_leaves, n_tris;
+  int64_t n_nodes, n_leaves, n_tris, first_block;
   uint32_t node_base, leaf_base, tri_base;
-  int32_t prim_offset, object;
+  int32_t prim_offset;
 };
-hipError_t launch_scene_place(const ScenePlace& P, hipStream_t s);
+int64_t scene_place_blocks(const ScenePlace& p);
+// Places all objects; place: n_obj records in device memory.
+hipError_t launch_scene_place(const DevScene& s, const ScenePlace* place, int32_t n_obj, int64_t blocks, hipStream_t st);
 
 struct AttrLaunch {
   const DevScene* scene;
