@@ -21,7 +21,10 @@ inline re_status set_err(re_ctx* ctx, re_status st, const char* msg) {
 
 inline re_status set_err(re_ctx* ctx, re_status st, const std::string& msg) { return set_err(ctx, st, msg.c_str()); }
 
+// An error is the failing call's alone: left as the thread's last error, the
+// check after the next launch would report it again.
 inline re_status hip_err(re_ctx* ctx, hipError_t e, const char* where) {
+  (void)hipGetLastError();
   char buf[400];
   snprintf(buf, sizeof(buf), "%s: %s", where, hipGetErrorString(e));
   return set_err(ctx, e == hipErrorOutOfMemory ? RE_ERR_OOM : RE_ERR_HIP, buf);
