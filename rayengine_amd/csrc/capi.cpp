@@ -193,7 +193,7 @@ RE_API re_status re_scene_upload(re_ctx* ctx, const re_object* objs, int32_t n_o
   hipError_t e = hipSuccess;
   auto alloc = [&](void** dst, size_t bytes, size_t more = 0) {
     if (bytes == 0) bytes = 64;  // keep every pointer valid
-    if (e == hipSuccess) e = hipMalloc(dst, bytes + more);  // (`more` is not counted as the scene's)
+    if (e == hipSuccess) e = device_malloc(ctx, dst, bytes + more);  // (`more` is not counted as the scene's)
     s.bytes += (int64_t)bytes;
   };
   auto copy = [&](void* dst, const void* src, size_t bytes) {
@@ -579,9 +579,9 @@ RE_API re_status re_scene_set_attributes(re_ctx* ctx, int32_t scene_id, const fl
       seen[(size_t)r.prim] = 1;
     }
     float *g = nullptr, *nr = nullptr, *uv = nullptr;
-    hipError_t e = hipMalloc((void**)&g, geom.size() * 4);
-    if (e == hipSuccess) e = hipMalloc((void**)&nr, (size_t)n_prims * 36);
-    if (e == hipSuccess && uvs) e = hipMalloc((void**)&uv, (size_t)n_prims * 24);
+    hipError_t e = device_malloc(ctx, (void**)&g, geom.size() * 4);
+    if (e == hipSuccess) e = device_malloc(ctx, (void**)&nr, (size_t)n_prims * 36);
+    if (e == hipSuccess && uvs) e = device_malloc(ctx, (void**)&uv, (size_t)n_prims * 24);
     if (e == hipSuccess) e = hipMemcpyAsync(g, geom.data(), geom.size() * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(nr, normals, (size_t)n_prims * 36, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess && uvs) e = hipMemcpyAsync(uv, uvs, (size_t)n_prims * 24, hipMemcpyHostToDevice, ctx->stream);

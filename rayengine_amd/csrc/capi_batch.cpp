@@ -175,7 +175,7 @@ RE_API re_status re_batch_create(re_ctx* ctx, const re_batch_scene* scenes, int3
   b.n_items = (int64_t)plan.items.size();
   hipError_t e = hipSuccess;
   auto alloc = [&](void** p, size_t bytes) {
-    if (e == hipSuccess) e = hipMalloc(p, bytes > 0 ? bytes : 64);
+    if (e == hipSuccess) e = device_malloc(ctx, p, bytes > 0 ? bytes : 64);
   };
   alloc((void**)&b.tiles, htiles.size() * sizeof(BatchTile));
   alloc((void**)&b.ray_o, rb);

@@ -62,14 +62,14 @@ RE_API re_status re_mlp_create(re_ctx* ctx, uint64_t seed, int32_t* mlp_id) {
   m.partial_blocks = train_blocks(ctx);
   const size_t pb = (size_t)kParams * 4;
   hipError_t e = hipSuccess;
-  if (e == hipSuccess) e = hipMalloc((void**)&m.params, pb);
-  if (e == hipSuccess) e = hipMalloc((void**)&m.m1, pb);
-  if (e == hipSuccess) e = hipMalloc((void**)&m.m2, pb);
-  if (e == hipSuccess) e = hipMalloc(&m.pack, (size_t)kPackAlloc * 2);
-  if (e == hipSuccess) e = hipMalloc((void**)&m.small, (size_t)kSmallAlloc * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&m.partial, (size_t)m.partial_blocks * (kParams + 1) * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&m.grad, pb);
-  if (e == hipSuccess) e = hipMalloc((void**)&m.loss, 4 * 1024);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.params, pb);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.m1, pb);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.m2, pb);
+  if (e == hipSuccess) e = device_malloc(ctx, &m.pack, (size_t)kPackAlloc * 2);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.small, (size_t)kSmallAlloc * 4);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.partial, (size_t)m.partial_blocks * (kParams + 1) * 4);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.grad, pb);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&m.loss, 4 * 1024);
   if (e != hipSuccess) {
     free_mlp(m);
     return hip_err(ctx, e, "re_mlp_create");
@@ -215,9 +215,9 @@ RE_API re_status re_sdf_distance_volume(re_ctx* ctx, int32_t vol_id, int32_t* di
   d.data = nullptr;
   const size_t nvox = (size_t)f.dim[0] * f.dim[1] * f.dim[2];
   float *a = nullptr, *b = nullptr;
-  hipError_t e = hipMalloc((void**)&d.data, (size_t)f.bytes);
-  if (e == hipSuccess) e = hipMalloc((void**)&a, nvox * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&b, nvox * 4);
+  hipError_t e = device_malloc(ctx, (void**)&d.data, (size_t)f.bytes);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&a, nvox * 4);
+  if (e == hipSuccess) e = device_malloc(ctx, (void**)&b, nvox * 4);
   if (e == hipSuccess) e = hipMemsetAsync(d.data, 0, (size_t)f.bytes, ctx->stream);
   if (e == hipSuccess) e = ctx->launch_begin();
   if (e == hipSuccess) e = launch_edt(f, a, b, d.data, ctx->stream);
@@ -364,7 +364,7 @@ RE_API re_status re_mlp_train(re_ctx* ctx, int32_t mlp_id, int32_t dist_vol_id, 
   if (m->loss_cap < p.steps) {
     if (m->loss) (void)hipFree(m->loss);
     m->loss = nullptr;
-    HIP_TRY(ctx, hipMalloc((void**)&m->loss, (size_t)(p.steps > 0 ? p.steps : 1) * 4), "loss history");
+    HIP_TRY(ctx, device_malloc(ctx, (void**)&m->loss, (size_t)(p.steps > 0 ? p.steps : 1) * 4), "loss history");
     m->loss_cap = p.steps;
   }
   // The pool is a pure function of (volume, seed, n_samples, band): a call
@@ -383,7 +383,7 @@ RE_API re_status re_mlp_train(re_ctx* ctx, int32_t mlp_id, int32_t dist_vol_id, 
   const int64_t first = m->cursor;
   const int32_t blocks = mlp_train_grid(m->partial_blocks, p.batch);
   float4* samples = nullptr;
-  HIP_TRY(ctx, hipMalloc((void**)&samples, (size_t)p.n_samples * 16), "sample pool");
+  HIP_TRY(ctx, device_malloc(ctx, (void**)&samples, (size_t)p.n_samples * 16), "sample pool");
   hipError_t e = launch_sample(dv, p.n_samples, p.seed, p.near_band_voxels * dv.spacing[0], 256, samples, ctx->stream);
   for (int32_t s = 0; e == hipSuccess && s < p.steps; ++s) {
     const int64_t start = (int64_t)(((unsigned __int128)(first + s) * (uint64_t)p.batch) % (uint64_t)p.n_samples);

@@ -27,7 +27,7 @@ re_status alloc_volume(re_ctx* ctx, const int32_t* dim, const float* spacing, De
     v.box_max[a] = (float)dim[a] * spacing[a];
   }
   v.bytes = (int64_t)v.bdim[0] * v.bdim[1] * v.bdim[2] * kBrickVox * (int64_t)sizeof(float);
-  HIP_TRY(ctx, hipMalloc((void**)&v.data, (size_t)v.bytes), "volume hipMalloc");
+  HIP_TRY(ctx, device_malloc(ctx, (void**)&v.data, (size_t)v.bytes), "volume hipMalloc");
   return RE_OK;
 }
 
@@ -64,7 +64,7 @@ re_status read_channel(re_ctx* ctx, const DevVolume& v, const float* src, float*
 // Gives a volume a zero material channel if it has none.
 re_status ensure_material(re_ctx* ctx, DevVolume& v) {
   if (v.mat) return RE_OK;
-  HIP_TRY(ctx, hipMalloc((void**)&v.mat, (size_t)v.bytes), "material hipMalloc");
+  HIP_TRY(ctx, device_malloc(ctx, (void**)&v.mat, (size_t)v.bytes), "material hipMalloc");
   HIP_TRY(ctx, hipMemsetAsync(v.mat, 0, (size_t)v.bytes, ctx->stream), "material clear");
   return RE_OK;
 }
@@ -252,7 +252,7 @@ re_status upload_pairs(re_ctx* ctx, const int32_t* dim, const float* spacing, co
   std::vector<float> bd, bm;
   to_bricked(v, dist.data(), bd);
   to_bricked(v, mat.data(), bm);
-  hipError_t e = hipMalloc((void**)&v.mat, (size_t)v.bytes);
+  hipError_t e = device_malloc(ctx, (void**)&v.mat, (size_t)v.bytes);
   if (e == hipSuccess) e = hipMemcpyAsync(v.data, bd.data(), (size_t)v.bytes, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(v.mat, bm.data(), (size_t)v.bytes, hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);

@@ -86,14 +86,14 @@ RE_API re_status re_autotune_trace(re_ctx* ctx, const float* tri_v, int64_t n_tr
     const float* d_o = ray_o;
     const float* d_d = ray_d;
     if (!(flags & RE_DEVICE_PTRS)) {
-      HIP_TRY(ctx, hipMalloc(&S.rays, 2 * ray_bytes), "re_autotune_trace: ray buffer");
+      HIP_TRY(ctx, device_malloc(ctx, &S.rays, 2 * ray_bytes), "re_autotune_trace: ray buffer");
       HIP_TRY(ctx, hipMemcpyAsync(S.rays, ray_o, ray_bytes, hipMemcpyHostToDevice, ctx->stream), "copy ray_o");
       HIP_TRY(ctx, hipMemcpyAsync((char*)S.rays + ray_bytes, ray_d, ray_bytes, hipMemcpyHostToDevice, ctx->stream),
               "copy ray_d");
       d_o = (const float*)S.rays;
       d_d = (const float*)((char*)S.rays + ray_bytes);
     }
-    HIP_TRY(ctx, hipMalloc(&S.out, (size_t)n * 8), "re_autotune_trace: result buffer");
+    HIP_TRY(ctx, device_malloc(ctx, &S.out, (size_t)n * 8), "re_autotune_trace: result buffer");
     int32_t* d_prim = (int32_t*)S.out;
     float* d_t = (float*)((char*)S.out + (size_t)n * 4);
 

@@ -50,6 +50,19 @@ re_status guarded(re_ctx* ctx, const char* what, F&& body) {
   }
 }
 
+// hipMalloc.  When the device has no room, what the context keeps between its
+// kd builds is given back first: no call fails for want of memory that only
+// waits for the next build.
+inline hipError_t device_malloc(re_ctx* ctx, void** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || !ctx->kd_build.chunk) return e;
+  (void)hipGetLastError();  // else the next launch's check finds it
+  (void)hipFree(ctx->kd_build.chunk);
+  ctx->kd_build.chunk = nullptr;
+  ctx->kd_build.bytes = 0;
+  return hipMalloc(p, bytes);
+}
+
 // Grows the context's staging buffer to at least `bytes`.
 inline re_status ensure_stage(re_ctx* ctx, size_t bytes) {
   if (ctx->stage_bytes >= bytes) return RE_OK;
@@ -58,7 +71,7 @@ inline re_status ensure_stage(re_ctx* ctx, size_t bytes) {
   ctx->stage = nullptr;
   ctx->stage_bytes = 0;
   size_t want = bytes + bytes / 4;
-  HIP_TRY(ctx, hipMalloc(&ctx->stage, want), "stage hipMalloc");
+  HIP_TRY(ctx, device_malloc(ctx, &ctx->stage, want), "stage hipMalloc");
   ctx->stage_bytes = want;
   return RE_OK;
 }

@@ -104,7 +104,8 @@ inline bool level_fits(int64_t nodes, int64_t records, const Adds& total) {
 
 // Device and pinned host memory that a context keeps between its device
 // builds: one chunk of what the last build took, at most kKeepBytes, and the
-// totals of a level.  A build that needs more takes and frees the rest itself.
+// totals of a level.  A build that needs more takes and frees the rest itself;
+// an allocation of the context that finds the device full frees the chunk.
 constexpr size_t kKeepBytes = (size_t)256 << 20;
 struct Workspace {
   char* chunk = nullptr;
