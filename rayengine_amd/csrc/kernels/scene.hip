@@ -7,6 +7,8 @@ namespace re {
 namespace {
 
 constexpr int kPlaceBlock = 256;
+static_assert(sizeof(LeafRec) == sizeof(DevLeaf) && alignof(LeafRec) == alignof(DevLeaf),
+              "a leaf record is rewritten in place");
 
 // The blocks of object k follow those of the objects before it (first_block,
 // found by bisection, the same in every thread).  Thread i of an object takes
@@ -41,7 +43,8 @@ __global__ void __launch_bounds__(kPlaceBlock) scene_place_kernel(NodeEntry* __r
     nodes[i].meta = meta;
   }
   if (i < P.n_leaves) {
-    LeafRec l = reinterpret_cast<const LeafRec*>(leaves)[i];
+    LeafRec l;
+    __builtin_memcpy(&l, leaves + i, sizeof(l));  // not a DevLeaf yet
     for (int f = 0; f < 6; ++f) {
       const int32_t r = l.rope[f];
       if (r != kNoRope) l.rope[f] = ref_is_leaf(r) ? leaf_ref(ref_leaf_id(r) + P.leaf_base) : r + (int32_t)P.node_base;
