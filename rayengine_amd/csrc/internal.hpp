@@ -151,15 +151,17 @@ inline int coop_lanes(int64_t n) {
 }
 
 // Whether a ray's walks of the scene's objects get a lane each: they are then
-// side by side instead of one after another and their kernel is the one-object
-// one, without spills; but a lane whose object the ray misses stays empty, and
-// an any-hit ray walks all its objects.  Limits: three rounds of resident waves
-// (one for any-hit).  us, one after another / side by side, incoherent rays:
-// 3 objects of 6,670 triangles, 1,000 rays 176 / 89, 100,003 328 / 170, 300,000
-// 472 / 380; 8 apart, 40,000 249 / 125, 200,000 391 / 374, 300,000 441 / 528;
-// 30 apart, 10,000 245 / 63, 100,003 421 / 309, 200,000 531 / 573.  Any-hit:
-// 100,003 rays on 3 259 / 165, 300,000 327 / 366; 2 objects, 200,000 215 / 195,
-// 300,000 214 / 248.
+// side by side instead of one after another; but a lane whose object the ray
+// misses stays empty, and an any-hit ray walks all its objects.  Limits: three
+// rounds of resident waves (one for any-hit), below the first sizes at which
+// side by side is behind.  us, one after another / side by side, incoherent
+// rays: 3 objects of 6,670 triangles, 1,000 rays 227 / 87, 100,000 366 / 197,
+// 300,000 511 / 440; 8 of 3,750 30,000 600 / 146, 150,000 889 / 472; 30 of
+// 1,000 12,000 1,100 / 118, 60,000 1,498 / 433; 30 of them apart, camera rays,
+// 40,000 150 / 94, 100,000 167 / 200.  Any-hit: 3 objects 100,000 304 / 195,
+// 200,000 368 / 311, 300,000 367 / 400; 2 of 6,000 200,000 257 / 199, 300,000
+// 305 / 308; 3 apart, two-sided, 100,000 126 / 90, 200,000 104 / 112; 8, two-
+// sided, 60,000 225 / 207, 150,000 332 / 359.
 constexpr int64_t kSpreadWalks = 3 * 6144 * 64, kSpreadAnyWalks = 6144 * 64;
 inline bool trace_spreads(int64_t n, int32_t n_obj, int64_t most) {
   return n_obj > 1 && n_obj <= 64 && n <= most / n_obj;

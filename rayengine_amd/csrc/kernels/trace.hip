@@ -257,7 +257,11 @@ trace_coop_kernel(RE_CLOSEST_PARAMS, const int32_t* __restrict__ start_leaf, int
   const int64_t blk = (int64_t)(gridDim.x - 1 - blockIdx.x);
   const int64_t i = (blk * (blockDim.x >> 6) + (threadIdx.x >> 6)) * lanes + r;
   const bool has_ray = (SPREAD ? obj < n_obj : r < lanes) && i < n;
-  const auto ray = [&](f3& o, f3& d) { load_ray(ray_o, ray_d, i, o, d); };
+  const auto ray = [&](f3& o, f3& d) {
+    int64_t j = i;
+    if (!ONE_OBJ) asm volatile("" : "+v"(j));  // read anew for every object: not held in registers during a walk
+    load_ray(ray_o, ray_d, j, o, d);
+  };
   float best_t;
   int32_t best_prim, best_obj;
   RayCounts rc;
@@ -316,7 +320,11 @@ trace_occluded_kernel(const NodeEntry* __restrict__ nodes, const DevLeaf* __rest
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t i = ((int64_t)(gridDim.x - 1 - blockIdx.x) * (blockDim.x >> 6) + w) * lanes + r;
   const bool has_ray = (SPREAD ? obj < n_obj : r < lanes) && i < n;
-  const auto ray = [&](f3& o, f3& d) { load_ray(ray_o, ray_d, i, o, d); };
+  const auto ray = [&](f3& o, f3& d) {
+    int64_t j = i;
+    if (!ONE_OBJ) asm volatile("" : "+v"(j));  // read anew for every object: not held in registers during a walk
+    load_ray(ray_o, ray_d, j, o, d);
+  };
   float best_t;
   int32_t best_prim, best_obj;
   RayCounts rc;
