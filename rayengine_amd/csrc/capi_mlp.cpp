@@ -212,12 +212,15 @@ RE_API re_status re_sdf_distance_volume(re_ctx* ctx, int32_t vol_id, int32_t* di
   if (f.dim[0] > 4096 || f.dim[1] > 4096 || f.dim[2] > 4096)
     return set_err(ctx, RE_ERR_INVALID, "re_sdf_distance_volume: dims above 4096");
   DevVolume d = f;
-  d.data = nullptr;
+  d.data = d.mat = nullptr;  // its own: either volume may be released first
   const size_t nvox = (size_t)f.dim[0] * f.dim[1] * f.dim[2];
   float *a = nullptr, *b = nullptr;
   hipError_t e = device_malloc(ctx, (void**)&d.data, (size_t)f.bytes);
   if (e == hipSuccess) e = device_malloc(ctx, (void**)&a, nvox * 4);
   if (e == hipSuccess) e = device_malloc(ctx, (void**)&b, nvox * 4);
+  if (e == hipSuccess && f.mat) e = device_malloc(ctx, (void**)&d.mat, (size_t)f.bytes);
+  if (e == hipSuccess && f.mat)
+    e = hipMemcpyAsync(d.mat, f.mat, (size_t)f.bytes, hipMemcpyDeviceToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemsetAsync(d.data, 0, (size_t)f.bytes, ctx->stream);
   if (e == hipSuccess) e = ctx->launch_begin();
   if (e == hipSuccess) e = launch_edt(f, a, b, d.data, ctx->stream);
@@ -227,6 +230,7 @@ RE_API re_status re_sdf_distance_volume(re_ctx* ctx, int32_t vol_id, int32_t* di
   if (b) (void)hipFree(b);
   if (e != hipSuccess) {
     if (d.data) (void)hipFree(d.data);
+    if (d.mat) (void)hipFree(d.mat);
     return hip_err(ctx, e, "re_sdf_distance_volume");
   }
   int32_t id = ctx->next_id++;
