@@ -154,12 +154,16 @@ RE_API re_status re_batch_create(re_ctx* ctx, const re_batch_scene* scenes, int3
   // rays 2.25 / 2.42 (128: 2.24), 12 M rays 4.59 / 4.43 (128: 4.41).
   BatchPlan units;
   {
-    int64_t total = 0;
-    for (const BatchItem& it : plan.items) total += it.count;
+    int64_t total = 0, plain_total = 0;
+    for (const BatchItem& it : plan.items) {
+      total += it.count;
+      if (it.kind == kItemPlain) plain_total += it.count;
+    }
     int32_t cut = coop_lanes(total);
     while (cut < cfg.item_rays && total >= 2 * (int64_t)cut * 8 * 6144) cut *= 2;
     const re_status st = plan_batch(scenes, n_scenes, tiles, n_tiles, n_rays,
-                                    cfg.item_rays < cut ? cfg.item_rays : cut, units);
+                                    cfg.item_rays < cut ? cfg.item_rays : cut, units,
+                                    plain_item_rays(plain_total, cfg.item_rays));
     if (st) {
       free_batch(b);
       const std::string msg = std::string("re_batch_create: ") + g_last_error;

@@ -12,8 +12,9 @@
 namespace re {
 
 re_status plan_batch(const re_batch_scene* scenes, int32_t n_scenes, const re_batch_tile* tiles, int32_t n_tiles,
-                     int64_t n_rays, int32_t item_rays, BatchPlan& out) {
+                     int64_t n_rays, int32_t item_rays, BatchPlan& out, int32_t plain_rays) {
   out = BatchPlan{};
+  if (plain_rays <= 0) plain_rays = item_rays;
   if (n_scenes < 0 || n_tiles < 0 || n_scenes + n_tiles <= 0 || n_rays <= 0 || (n_scenes > 0 && !scenes) ||
       (n_tiles > 0 && !tiles) || item_rays < 1 || item_rays > (1 << 16))
     return fail(RE_ERR_INVALID, "batch plan: bad arguments");
@@ -28,8 +29,8 @@ re_status plan_batch(const re_batch_scene* scenes, int32_t n_scenes, const re_ba
   auto count_of = [&](int32_t s) { return s < n_scenes ? scenes[s].ray_count : tiles[s - n_scenes].ray_count; };
   int64_t total = 0;
   for (int32_t s = 0; s < n_slots; ++s) {
-    const bool surrogate = s >= n_scenes && tiles[s - n_scenes].mode == 2;
-    if (!surrogate) total += (count_of(s) + item_rays - 1) / item_rays;
+    const int32_t mode = s < n_scenes ? 0 : tiles[s - n_scenes].mode, per = mode == 1 ? plain_rays : item_rays;
+    if (mode != 2) total += (count_of(s) + per - 1) / per;
   }
   if (total > kMaxBatchItems) return fail(RE_ERR_INVALID, "batch plan: more than 2^30 work items (raise item_rays)");
   std::vector<int32_t> order(n_slots);
@@ -57,8 +58,9 @@ re_status plan_batch(const re_batch_scene* scenes, int32_t n_scenes, const re_ba
       }
       kind = tl.mode == 0 ? kItemExact : kItemPlain;
     }
-    for (int64_t off = 0; off < count; off += item_rays) {
-      const int32_t c = (int32_t)std::min<int64_t>(item_rays, count - off);
+    const int32_t per = kind == kItemPlain ? plain_rays : item_rays;
+    for (int64_t off = 0; off < count; off += per) {
+      const int32_t c = (int32_t)std::min<int64_t>(per, count - off);
       out.items.push_back(BatchItem{kind, target, begin + off, c, s});
       ++out.remaining[s];
     }

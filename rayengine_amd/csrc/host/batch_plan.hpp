@@ -34,11 +34,24 @@ struct BatchPlan {
 
 // Targets (slots: scenes 0..n_scenes-1, then tiles) in ascending ray count,
 // ties in slot order; each target's range cut into items of item_rays rays
-// (the last one shorter).  Surrogate tiles (mode 2) get no items: they run as
-// their own launches, and their slot counts one completion.  RE_ERR_INVALID
-// for a range outside [0, n_rays), a bad mode or item_rays outside
-// [1, 65536]; more than kMaxBatchItems items is RE_ERR_INVALID too.
+// (the last one shorter), sphere-traced tiles' (mode 1) into items of
+// plain_rays where that is given.  Surrogate tiles (mode 2) get no items: they
+// run as their own launches, and their slot counts one completion.
+// RE_ERR_INVALID for a range outside [0, n_rays), a bad mode or item_rays
+// outside [1, 65536]; more than kMaxBatchItems items is RE_ERR_INVALID too.
 re_status plan_batch(const re_batch_scene* scenes, int32_t n_scenes, const re_batch_tile* tiles, int32_t n_tiles,
-                     int64_t n_rays, int32_t item_rays, BatchPlan& out);
+                     int64_t n_rays, int32_t item_rays, BatchPlan& out, int32_t plain_rays = 0);
+
+// Rays per item of the sphere-traced tiles, at most item_rays: their marches
+// are short, so that what a launch of them takes is soon the counter's
+// contention: 64 rays, twice as many while there would be more than 1,024
+// items.  us per run for items of 64 / 128 / 256 rays: 2,000 rays 40 / 46 / 55;
+// 40,000 51 / 52 / 63; 90,000 69 / 58 / 73; 180,000 102 / 77 / 76; 360,000 170 /
+// 108 / 93; 1.2 M 328 / 221 / 162.
+inline int32_t plain_item_rays(int64_t plain_total, int32_t item_rays) {
+  int32_t per = 64;
+  while (per < item_rays && plain_total > (int64_t)per * 1024) per *= 2;
+  return per < item_rays ? per : item_rays;
+}
 
 }  // namespace re
