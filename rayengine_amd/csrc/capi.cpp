@@ -282,16 +282,23 @@ RE_API re_status re_scene_export(re_ctx* ctx, int32_t scene_id, void* nodes, voi
   HIP_TRY(ctx, hipSetDevice(ctx->device), "hipSetDevice");
   if (nodes && s.n_nodes)
     HIP_TRY(ctx, hipMemcpyAsync(nodes, s.nodes, s.n_nodes * sizeof(NodeEntry), hipMemcpyDeviceToHost, ctx->stream), "export nodes");
-  // Leaf records in the flat field order (the device holds them as DevLeaf).
-  std::vector<DevLeaf> dl(leaves ? (size_t)s.n_leaves : 0);
-  if (!dl.empty())
-    HIP_TRY(ctx, hipMemcpyAsync(dl.data(), s.leaves, dl.size() * sizeof(DevLeaf), hipMemcpyDeviceToHost, ctx->stream), "export leaves");
+  // Leaf records in the flat field order (the device holds them as DevLeaf),
+  // through the staging buffer, 16 MB at a time
+  if (leaves && s.n_leaves) {
+    const int64_t per = std::min<int64_t>(s.n_leaves, (16 << 20) / (int64_t)sizeof(LeafRec));
+    const re_status st = ensure_stage(ctx, (size_t)per * sizeof(LeafRec));
+    if (st) return st;
+    for (int64_t at = 0; at < s.n_leaves; at += per) {
+      const int64_t n = std::min(per, s.n_leaves - at);
+      HIP_TRY(ctx, launch_flat_leaves(s.leaves + at, (LeafRec*)ctx->stage, n, ctx->stream), "export leaves");
+      HIP_TRY(ctx, hipMemcpyAsync((char*)leaves + at * sizeof(LeafRec), ctx->stage, n * sizeof(LeafRec), hipMemcpyDeviceToHost, ctx->stream), "export leaves");
+    }
+  }
   if (tris && s.n_trirecs)
     HIP_TRY(ctx, hipMemcpyAsync(tris, s.tris, s.n_trirecs * sizeof(TriRec), hipMemcpyDeviceToHost, ctx->stream), "export tris");
   if (objs)
     HIP_TRY(ctx, hipMemcpyAsync(objs, s.objs, s.n_obj * sizeof(ObjXform), hipMemcpyDeviceToHost, ctx->stream), "export objs");
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream), "export sync");
-  for (size_t i = 0; i < dl.size(); ++i) static_cast<LeafRec*>(leaves)[i] = flat_leaf(dl[i]);
   return RE_OK;
   });
 }

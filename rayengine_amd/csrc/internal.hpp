@@ -53,6 +53,8 @@ struct ScenePlace {
 int64_t scene_place_blocks(const ScenePlace& p);
 // Places all objects; place: n_obj records in device memory.
 hipError_t launch_scene_place(const DevScene& s, const ScenePlace* place, int32_t n_obj, int64_t blocks, hipStream_t st);
+// n leaf records in the flat field order.
+hipError_t launch_flat_leaves(const DevLeaf* leaves, LeafRec* out, int64_t n, hipStream_t st);
 
 struct AttrLaunch {
   const DevScene* scene;

@@ -57,6 +57,13 @@ __global__ void __launch_bounds__(kPlaceBlock) scene_place_kernel(NodeEntry* __r
   if (i < P.n_tris && P.prim_offset != 0) tris[i].prim += P.prim_offset;
 }
 
+// Leaf records back in the flat field order, for an export.
+__global__ void __launch_bounds__(kPlaceBlock) flat_leaves_kernel(const DevLeaf* __restrict__ leaves,
+                                                                  LeafRec* __restrict__ out, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * kPlaceBlock + threadIdx.x;
+  if (i < n) out[i] = flat_leaf(leaves[i]);
+}
+
 }  // namespace
 
 int64_t scene_place_blocks(const ScenePlace& p) {
@@ -71,6 +78,13 @@ hipError_t launch_scene_place(const DevScene& s, const ScenePlace* place, int32_
   if (blocks <= 0) return hipSuccess;
   hipLaunchKernelGGL(scene_place_kernel, dim3((unsigned)blocks), dim3(kPlaceBlock), 0, st, s.nodes, s.leaves, s.tris,
                      place, n_obj);
+  return hipGetLastError();
+}
+
+hipError_t launch_flat_leaves(const DevLeaf* leaves, LeafRec* out, int64_t n, hipStream_t st) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(flat_leaves_kernel, dim3((unsigned)((n + kPlaceBlock - 1) / kPlaceBlock)), dim3(kPlaceBlock), 0,
+                     st, leaves, out, n);
   return hipGetLastError();
 }
 
