@@ -270,20 +270,19 @@ __device__ __forceinline__ float box_distance(float px, float py, float pz, cons
 // distance with h^2 k / 4 taken off its distance), SPHERE_SUBTRACT and
 // CUBE_SUBTRACT: the pair of the larger distance against the negated brush
 // distance (sdf_fmaxf), CUBE_ADD: the componentwise minimum (fminf on
-// float2) -- sdf_functions.cuh:270-289.  One work-group per brick, as in the
-// noise fill; the kernel streams the volume once (8 bytes in and out per
-// voxel).
+// float2) -- sdf_functions.cuh:270-289.  A work-group takes eight consecutive
+// 4^3 blocks, a wave per block, so that the kernel streams the volume once in
+// the order of memory (8 bytes in and out per voxel).
 __global__ void __launch_bounds__(256) volume_edit_kernel(EditLaunch L) {
-  const int64_t brick = blockIdx.x;
-  const int gx = (int)(brick % L.bdim[0]), gy = (int)((brick / L.bdim[0]) % L.bdim[1]);
-  const int gz = (int)(brick / ((int64_t)L.bdim[0] * L.bdim[1]));
-  for (int m = threadIdx.x; m < kBrickVox; m += blockDim.x) {
-    int qx, qy, qz, lx, ly, lz;
-    brick_block((uint32_t)m >> 6, qx, qy, qz);
-    block_voxel((uint32_t)m & 63u, lx, ly, lz);
-    const int x = gx * kBrick + qx * kBlock + lx, y = gy * kBrick + qy * kBlock + ly, z = gz * kBrick + qz * kBlock + lz;
+  const uint32_t nx = 2u * (uint32_t)L.bdim[0], ny = 2u * (uint32_t)L.bdim[1];
+  int lx, ly, lz;
+  block_voxel((uint32_t)threadIdx.x & 63u, lx, ly, lz);
+  for (uint32_t k = threadIdx.x >> 6; k < 8u; k += blockDim.x >> 6) {
+    // (at most 2^30 blocks: dimensions go up to 4096)
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 8u + k));
+    const int x = (int)(b % nx) * kBlock + lx, y = (int)(b / nx % ny) * kBlock + ly, z = (int)(b / nx / ny) * kBlock + lz;
     if (x >= L.dim[0] || y >= L.dim[1] || z >= L.dim[2]) continue;
-    const int64_t i = vox_index(L.bdim, x, y, z);
+    const int64_t i = (int64_t)b * kBlockVox + (threadIdx.x & 63);
     float px = (float)x * L.spacing[0] - L.center[0];
     const float py = (float)y * L.spacing[1] - L.center[1];
     float pz = (float)z * L.spacing[2] - L.center[2];
