@@ -217,8 +217,9 @@ typedef struct re_trace_params {
                                  lanes have finished their rays, they take the
                                  next rays at the next leaf round (rays taken
                                  from the end of the array); faster than 4 on
-                                 large launches of incoherent rays in large
-                                 trees, others are launched as 4.
+                                 large launches of incoherent rays in a large
+                                 tree (scenes of one object); others are
+                                 launched as 4.
                               Variants 4 and 5 give a wave fewer rays when the
                               launch would not fill the device.
                               Results are identical for every variant. */

@@ -399,7 +399,7 @@ re_status trace_common(re_ctx* ctx, int32_t scene_id, const float* ray_o, const 
     if (g <= 0) g = p.variant == 5 ? trace_coop_refill_grid(blk) : trace_persistent_grid(blk);
     L.grid_blocks = g;
   }
-  const bool queue = p.variant == 1 || trace_refills(p.variant, n, it->second.n_trirecs);
+  const bool queue = p.variant == 1 || trace_refills(p.variant, n, it->second);
   const bool dev = (flags & RE_DEVICE_PTRS) != 0;
   const size_t ray_bytes = (size_t)n * 12;
   char* base = nullptr;

@@ -176,16 +176,19 @@ inline int spread_rays(int64_t n, int32_t n_obj) {
 // Whether variant 5 refills its waves, or is the plain cooperative kernel (the
 // same walks, one set of rays a wave).  Refill keeps lanes busy where walks are
 // long and uneven, and pays for it with a counter per 64 rays, a setup of 32
-// rays at a time and waves whose halves are apart.  It is ahead once a launch
-// has two rounds of resident waves (256 CUs x 24) and the scene 10^5 triangle
-// records.  us, refill / plain, diffuse bounces: 2,919,928 records, 207,360
-// rays 231 / 205, 507,206 358 / 342, 829,440 437 / 457, 1,866,240 722 / 846;
-// 157,048 records, 829,440 rays 369 / 345, 3,317,760 943 / 1035; 68,589
-// records, 207,360 rays 158 / 126, 829,440 305 / 258, 3,317,760 773 / 748;
-// 17,832 records, 1,866,240 rays 343 / 269.
+// rays at a time and waves whose halves are apart.  With one object it is ahead
+// from two rounds of resident waves (256 CUs x 24) and 10^5 triangle records
+// on, or shortly after: us, refill / plain, diffuse bounces: 3,029,743 records,
+// 339,950 rays 285 / 245, 870,239 457 / 475, 1,958,113 805 / 927, 3,481,247
+// 1,182 / 1,541; 520,794 records, 681,695 rays 428 / 416, 1,534,595 681 / 765;
+// 156,138 records, 841,060 rays 425 / 409, 1,495,642 622 / 643; 68,343 records,
+// 860,254 rays 374 / 330.  (Rays of a camera, 3,686,400 on 3,029,743 records
+// 908 / 607, are variant 4's.)  With several objects the plain kernel's waves
+// take them together: 2,000,000 incoherent rays on 3 objects of 100,000
+// triangles 7,400 / 5,900, on 30 of 10,000 44,000 / 34,600.
 constexpr int64_t kRefillRays = 2 * 6144 * 64, kRefillRecs = 100000;
-inline bool trace_refills(int variant, int64_t n, int64_t n_trirecs) {
-  return variant == 5 && n > kRefillRays && n_trirecs > kRefillRecs;
+inline bool trace_refills(int variant, int64_t n, const DevScene& s) {
+  return variant == 5 && s.n_obj == 1 && n > kRefillRays && s.n_trirecs > kRefillRecs;
 }
 
 hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s);

@@ -373,18 +373,17 @@ constexpr int kRefillLanes = 32;  // refill threshold: half a wave
 // until its t_entry passes the hit, so its last leaf is the one whose cell
 // holds the hit point (when the walk ends there, not at the visit cap or a
 // missing rope), the leaf a ray leaving that point starts in.
-// One object and no hints fit 72 registers with 6 spilled: 7 waves per SIMD,
-// 1.87 M bounce rays on 2^20 triangles 720 us at 6 and 690 at 7.  (The plain
-// cooperative kernel spills 16 and is slower: 563,563 rays 190 and 215.)
-template <bool COUNT, bool ONE_SIDED, bool ONE_OBJ, int HINT = 0>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ONE_OBJ && HINT == 0 ? 7 : 6)))
+// Scenes of one object only (trace_refills).  Without hints it fits 72
+// registers with 6 spilled: 7 waves per SIMD, 1.87 M bounce rays on 2^20
+// triangles 720 us at 6 and 690 at 7.
+template <bool COUNT, bool ONE_SIDED, int HINT = 0>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HINT == 0 ? 7 : 6)))
 trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ queue,
                          const int32_t* __restrict__ start_leaf, int32_t* __restrict__ hit_leaf, int64_t n_leaves) {
   extern __shared__ CoopWave waves[];
   CoopWave& W = waves[threadIdx.x >> 6];
   const int lane = (int)(threadIdx.x & 63);
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const int32_t k_end = ONE_OBJ ? 1 : n_obj;
   int64_t pool_next = 0, pool_end = 0;  // wave-uniform
   bool drained = false;                 // wave-uniform
   // The rays are split into kQueueSlots equal parts, each with its own
@@ -399,22 +398,22 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
   f3 ro{0, 0, 0}, rd{0, 0, 0}, fr{0, 0, 0};
   float t_entry = 0.0f, t_exit = 0.0f, hit_t = kInf, best_t = kInf;
   uint32_t hit_rec = 0;  // record of the walk's hit, valid when found
-  int32_t k_obj = -1, cur = 0, visits = 0, best_prim = -1, best_obj = -1;
+  int32_t cur = 0, visits = 0, best_prim = -1, best_obj = -1;
   int32_t hint = -1, walk_leaf = -1, best_leaf = -1;  // HINT only
   bool live = false, open = false, found = false, have_window = false;
   uint4 w = make_uint4(0u, 0u, 0u, 0u);
   WalkMemo memo;
   RayCounts rc;
   unsigned c_hit = 0;
-  // the walk of object k from the ray (o, d): its first visit, or none
-  auto start_walk = [&](const ObjXform& ob, int32_t k) {
-    f3 o, d;  // read again for each object: no registers held during a walk
+  // the ray's walk: its first visit, or none
+  auto start_walk = [&](const ObjXform& ob) {
+    f3 o, d;
     load_ray(ray_o, ray_d, ray, o, d);
     xform_ray(ob, o, d, secondary != 0, ro, rd);
     fr = f3{recip(rd.x), recip(rd.y), recip(rd.z)};
     if (!ray_box_inv(ob.root_min, ob.root_max, ro, fr, t_entry, t_exit)) return;
     cur = ob.root;
-    if (HINT != 0) cur = hinted_start(leaves, n_leaves, hint, k, add(ro, smul(t_entry, rd)), cur);
+    if (HINT != 0) cur = hinted_start(leaves, n_leaves, hint, 0, add(ro, smul(t_entry, rd)), cur);
     found = false;
     hit_t = kInf;
     visits = 0;
@@ -422,13 +421,6 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
     memo = WalkMemo{};
     live = t_entry < t_exit && visits < cap;
     open = live;
-  };
-  // the next object whose root box the ray enters (trace_ray's object loop)
-  auto start_next = [&]() {
-    while (!live && k_obj + 1 < k_end) {
-      ++k_obj;
-      start_walk(objs[k_obj], k_obj);
-    }
   };
   auto finish = [&]() {
     prim_out[ray] = best_prim;
@@ -440,17 +432,16 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
   };
 #pragma unroll 1
   for (;;) {
-    // close a finished walk: the next object, or the ray's result
+    // close a finished walk
     if (ray >= 0 && !live) {
       if (open && found && hit_t < best_t) {
         best_t = hit_t;
         best_prim = tris[hit_rec].prim;
-        best_obj = ONE_OBJ ? 0 : k_obj;
+        best_obj = 0;
         if (HINT == 2) best_leaf = walk_leaf;
       }
       open = false;
-      if (!ONE_OBJ) start_next();
-      if (!live) finish();
+      finish();
     }
     // refill (wave-uniform), once half the lanes or more have no ray: they
     // take the next rays of the wave's chunk; the chunk start is taken with
@@ -492,13 +483,8 @@ trace_coop_refill_kernel(RE_CLOSEST_PARAMS, unsigned long long* __restrict__ que
           if (HINT != 0) hint = start_leaf ? start_leaf[ray] : -1;
           live = false;
           open = false;
-          if (ONE_OBJ) {
-            start_walk(objs[0], 0);
-          } else {
-            k_obj = -1;
-            start_next();
-          }
-          if (!live) finish();  // enters no object: a miss
+          start_walk(objs[0]);
+          if (!live) finish();  // does not enter the object: a miss
         }
         const int64_t taken = (int64_t)__popcll(need) < avail ? (int64_t)__popcll(need) : avail;
         pool_next += taken;
@@ -807,7 +793,7 @@ int64_t trace_coop_refill_grid(int block) {
   int dev = 0, cus = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trace_coop_refill_kernel<false, true, true>, block,
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, trace_coop_refill_kernel<false, true>, block,
                                                     (size_t)(block / 64) * sizeof(CoopWave)) != hipSuccess)
     return 0;
   return (int64_t)cus * (per_cu > 0 ? per_cu : 1);
@@ -836,7 +822,7 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
   // the one-ray-per-thread kernels (finer dispatch granularity at the tail;
   // 64 and 128 measured alike and ahead of 256 on the cluster workload).
   const int block = trace_launch_block(L.block, L.variant);
-  const bool refill = trace_refills(L.variant, L.n, L.scene->n_trirecs);
+  const bool refill = trace_refills(L.variant, L.n, *L.scene);
   const bool coop = L.variant == 4 || (L.variant == 5 && !refill);
   if (refill) {
     // Persistent cooperative waves: enough blocks to fill every CU at the
@@ -847,24 +833,21 @@ hipError_t launch_trace_closest(const TraceLaunch& L, hipStream_t s) {
     const DevScene& S5 = *L.scene;
     const int32_t cap5 = (L.cap > 0 && L.cap < kMaxLeafVisits) ? L.cap : kMaxLeafVisits;
     const int hint = L.hit_leaf ? 2 : (L.start_leaf ? 1 : 0);
-#define RE_LAUNCH_REFILL_H(C, O, ONE, H)                                                                       \
-  hipLaunchKernelGGL((trace_coop_refill_kernel<C, O, ONE, H>), dim3((unsigned)grid), dim3(block),              \
+#define RE_LAUNCH_REFILL_H(C, O, H)                                                                            \
+  hipLaunchKernelGGL((trace_coop_refill_kernel<C, O, H>), dim3((unsigned)grid), dim3(block),                   \
                      (block / 64) * sizeof(CoopWave), s, S5.nodes, S5.leaves, S5.tris, S5.objs, S5.n_obj,        \
                      L.ray_o, L.ray_d, L.n, cap5, L.secondary, L.prim, L.t, L.obj, L.counts, L.queue,            \
                      L.start_leaf, L.hit_leaf, S5.n_leaves)
-#define RE_LAUNCH_REFILL(C, O, ONE)                                         \
+#define RE_LAUNCH_REFILL(C, O)                                              \
   do {                                                                      \
-    if (hint == 2) RE_LAUNCH_REFILL_H(C, O, ONE, 2);                        \
-    else if (hint == 1) RE_LAUNCH_REFILL_H(C, O, ONE, 1);                   \
-    else RE_LAUNCH_REFILL_H(C, O, ONE, 0);                                  \
+    if (hint == 2) RE_LAUNCH_REFILL_H(C, O, 2);                             \
+    else if (hint == 1) RE_LAUNCH_REFILL_H(C, O, 1);                        \
+    else RE_LAUNCH_REFILL_H(C, O, 0);                                       \
   } while (0)
-    const bool one = S5.n_obj == 1;
     if (L.counts) {
-      if (L.one_sided) { if (one) RE_LAUNCH_REFILL(true, true, true); else RE_LAUNCH_REFILL(true, true, false); }
-      else { if (one) RE_LAUNCH_REFILL(true, false, true); else RE_LAUNCH_REFILL(true, false, false); }
+      if (L.one_sided) RE_LAUNCH_REFILL(true, true); else RE_LAUNCH_REFILL(true, false);
     } else {
-      if (L.one_sided) { if (one) RE_LAUNCH_REFILL(false, true, true); else RE_LAUNCH_REFILL(false, true, false); }
-      else { if (one) RE_LAUNCH_REFILL(false, false, true); else RE_LAUNCH_REFILL(false, false, false); }
+      if (L.one_sided) RE_LAUNCH_REFILL(false, true); else RE_LAUNCH_REFILL(false, false);
     }
 #undef RE_LAUNCH_REFILL
 #undef RE_LAUNCH_REFILL_H

@@ -1,6 +1,6 @@
 """Child process of test_gpu_refill_forms.py (RE_LIBRARY=debug is set by the
-parent): the refill kernel of the bounds-checked library on one object and
-three, plain, counted and hinted, against the one-ray-per-lane kernel, with no
+parent): the bounds-checked library's refill kernel, and with three objects its
+plain cooperative one, as they are, counted and hinted, against the one-ray-per-lane kernel, with no
 bounds-check bit set."""
 import sys
 from pathlib import Path

@@ -1,5 +1,6 @@
-"""Launches that variant 5 refills its waves in: more than 786,432 rays on more
-than 100,000 triangle records (fewer are launched as variant 4)."""
+"""Launches that variant 5 refills its waves in: more than 786,432 rays on one
+object of more than 100,000 triangle records (others are launched as variant
+4, so with three objects)."""
 import numpy as np
 
 import rayengine_amd as re

@@ -1,8 +1,9 @@
 """The refill kernel in every form a launch can ask for: visit caps, two-sided
 and secondary rays, block sizes, counters, walk-start hints (the hit leaves of
 the same rays, random ids in and out of range) with and without hit leaves,
-one object and three, the fixed scratch area, and the bounds-checked library;
-the one-ray-per-lane kernel's hits, bit for bit."""
+the fixed scratch area, and the bounds-checked library; the one-ray-per-lane
+kernel's hits, bit for bit.  The same for three objects, whose launches of
+variant 5 are the plain cooperative kernel's."""
 import ctypes as C
 import os
 import subprocess
