@@ -157,6 +157,7 @@ static int emu_uniform(int v) { return v; }
 hipError_t hipGetLastError() { return hipSuccess; }
 template <typename... A>
 static unsigned emu_unused(A...) { std::abort(); }
+static float __shfl(float, int) { std::abort(); }
 static float __uint_as_float(unsigned u) { float f; std::memcpy(&f, &u, 4); return f; }
 static unsigned __float_as_uint(float f) { unsigned u; std::memcpy(&u, &f, 4); return u; }
 #define __builtin_amdgcn_mbcnt_lo emu_unused
