@@ -780,7 +780,9 @@ constexpr int kDeferTile = 16;
 // wave taking rays until the block's are gone.  With a block per 512 rays a
 // block stayed until its longest march was done and whole blocks of the image
 // cost many times others: 921,600 rays on 192^3 1,042 us, now 964 (their 7.7 M
-// network points alone take 610 at the inference kernel's rate).
+// network points alone take 610 at the inference kernel's rate).  Times here
+// and below are the kernel's alone, with one network trained for the sweep;
+// another network evaluates another number of points.
 constexpr int64_t kHybridBlocks = 512;
 // Rays a wave holds: 64, or fewer while 12,288 runs (three per wave) are not
 // reached, as a wave lasts as long as its longest march and the network's
